@@ -182,6 +182,10 @@ struct sg_amr {
     int hydro_ready = 0;
     int4 *d_hx = nullptr, *d_fg = nullptr, *d_rf = nullptr;
     std::vector<int> hx_off, fg_off;
+    // the same exchanges resolved per ghost region (k_hx_fill), 27 entries per block: [0] a level's own
+    // exchange, [1] its same-level part on all arrays; hx_one: levels where the resolved form holds
+    int2 *d_hxe[2] = {};
+    std::vector<int> hx_one[2];
     std::vector<std::vector<int>> rf_rounds;   // per coarse level: offsets of its rounds, + end
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1687,6 +1691,7 @@ void release(sg_amr *s)
     for (int *q : ip) if (q) (void)hipFree(q);
     if (s->d_crop) (void)hipFree(s->d_crop);
     for (int4 *q : {s->d_hx, s->d_fg, s->d_rf}) if (q) (void)hipFree(q);
+    for (int2 *q : s->d_hxe) if (q) (void)hipFree(q);
     if (s->rhs0c) (void)hipFree(s->rhs0c);
     for (float *q : {s->u0c, s->res0c, s->gs0}) if (q) (void)hipFree(q);
     for (long *q : {s->d_at_ptr, s->d_bt_ptr}) if (q) (void)hipFree(q);
@@ -2710,9 +2715,64 @@ int upload4(sg_amr &s, int4 **dptr, const std::vector<int4> &v)
     return SG_OK;
 }
 
+// What face f of block b holds for the exchange: 0 nothing, 1 a same-level neighbour, 2 the coarse grid
+// of the parent's face (interpolation; nothing with same_only); *src: that grid.
+int hx_face(const sg_amr &s, int b, int f, int same_only, int *src)
+{
+    const int l = s.level[b], m = s.nbr[6 * b + f];
+    if (m >= 0 && s.level[m] == l) {
+        *src = m;
+        return 1;
+    }
+    if (l == 0 || same_only) return 0;
+    const int g = s.nbr[6 * s.parent[b] + f];
+    *src = g;
+    return g >= 0 && s.level[g] == l - 1 ? 2 : 0;
+}
+
+// The source of ghost region `side` (-1, 0, 1 per axis) of block b after the x, y, z passes, as
+// k_hx_fill reads it.  Returns 0 where the chain ends at a ghost cell that a pass of the same launch
+// writes (an inner corner of the refined region in the same-level part): the staged passes then
+// see an older value there.
+int hx_resolve(const sg_amr &s, int b, const int side[3], int same_only, int2 *out)
+{
+    int q = b, src = -1, moved = 0;
+    for (int d = 2; d >= 0; --d) {
+        if (side[d] == 0) continue;
+        const int lr = side[d] > 0, kind = hx_face(s, q, 2 * d + lr, same_only, &src);
+        if (kind == 2) {
+            *out = make_int2(src, moved | 8 | (d << 4) | (lr << 6) | (s.octant[q] << 7));
+            return 1;
+        }
+        if (kind == 1) {
+            q = src;
+            moved |= 1 << d;
+        }
+    }
+    if (!moved) {
+        *out = make_int2(-1, 0);
+        return 1;
+    }
+    for (int d = 0; d < 3; ++d)
+        if (side[d] != 0 && !((moved >> d) & 1) && hx_face(s, q, 2 * d + (side[d] > 0), same_only, &src)) return 0;
+    *out = make_int2(q, moved);
+    return 1;
+}
+
 int build_hydro_tables(sg_amr &s)
 {
     if (s.hydro_ready) return SG_OK;
+    for (int so = 0; so < 2; ++so) {
+        std::vector<int2> ent((size_t)27 * s.nblk, make_int2(-1, 0));
+        s.hx_one[so].assign(s.nlev, 1);
+        for (int b = 0; b < s.nblk; ++b)
+            for (int r = 0; r < 27; ++r) {
+                const int side[3] = {r % 3 - 1, (r / 3) % 3 - 1, r / 9 - 1};
+                if (!hx_resolve(s, b, side, so, &ent[(size_t)27 * b + r])) s.hx_one[so][s.level[b]] = 0;
+            }
+        SG_HIP(hipMalloc((void **)&s.d_hxe[so], ent.size() * sizeof(int2)));
+        SG_HIP(hipMemcpy(s.d_hxe[so], ent.data(), ent.size() * sizeof(int2), hipMemcpyHostToDevice));
+    }
     const int nl = s.nlev;
     std::vector<int4> hx, fg, rf;
     s.hx_off.assign(3 * nl + 1, 0);
@@ -2919,9 +2979,29 @@ int sg_amr_hydro_boundary_dev(sg_amr *ctx, double *pool, int level, int mode)
         SG_CHECK_LAUNCH();
         return SG_OK;
     };
-    if (level >= 1)
-        for (int d = 0; d < 3; ++d) SG_TRY(pass(level - 1, d, 3, 1));
-    for (int d = 0; d < 3; ++d) SG_TRY(pass(level, d, 1, 0));
+    // one launch per level where every ghost region's source is known beforehand, else the three
+    // staged passes (an inner corner of the refined region in the same-level part)
+    auto exchange = [&](int l, int ntab, int same_only) -> int {
+        const long wide = (long)(s.lev_start[l + 1] - s.lev_start[l]) * ntab;
+        if (!s.hx_one[same_only][l] || wide > 0x7fffffffL) {
+            for (int d = 0; d < 3; ++d) SG_TRY(pass(l, d, ntab, same_only));
+            return SG_OK;
+        }
+        const int b0 = s.lev_start[l], nb = s.lev_start[l + 1] - b0;
+        const unsigned groups = (unsigned)wide;
+        const int2 *ent = s.d_hxe[same_only] + (size_t)27 * b0;
+        const int *su = s.d_slot_u, *s1 = s.d_slot_u1, *s2 = s.d_slot_u2;
+        if (s.bml.ng == 2)
+            hipLaunchKernelGGL(k_hx_fill<2>, dim3(groups), dim3(256), 0, s.stream, pool, ent, b0, nb, su,
+                               s1, s2, mode, s.bml);
+        else
+            hipLaunchKernelGGL(k_hx_fill<0>, dim3(groups), dim3(256), 0, s.stream, pool, ent, b0, nb, su,
+                               s1, s2, mode, s.bml);
+        SG_CHECK_LAUNCH();
+        return SG_OK;
+    };
+    if (level >= 1) SG_TRY(exchange(level - 1, 3, 1));
+    SG_TRY(exchange(level, 1, 0));
     SG_HIP(hipStreamSynchronize(s.stream));
     return SG_OK;
 }

@@ -22,6 +22,42 @@ def _hier(which):
             "random-periodic": lambda: ah.random_hierarchy(4, 3, 0.35, seed=7, bc=ah.PERIODIC)}[which]()
 
 
+# Where the one-launch exchange has to follow the passes' order: refined regions with an inner corner
+# (its same-level part takes the staged passes), at the domain boundary (ghosts no pass writes), one
+# block wide (both neighbours of a block are the same), two wide and periodic (a block is its own
+# neighbour's neighbour), and the whole domain refined.
+EXCHANGE_HIERS = {
+    "inner-corner": lambda: ah.build((4, 4, 4), [{(1, 1, 1), (2, 1, 1), (1, 2, 1), (1, 1, 2), (2, 1, 2)}], bc=ah.SPHERE),
+    "at-boundary": lambda: ah.build((3, 4, 2), [{(0, 0, 0), (0, 1, 0), (1, 0, 0)}], bc=ah.SPHERE),
+    "one-wide": lambda: ah.build((1, 2, 3), [{(0, 0, 0), (0, 1, 0), (0, 0, 1), (0, 1, 1), (0, 0, 2), (0, 1, 2)}],
+                                 bc=ah.PERIODIC),
+    "random-sphere": lambda: ah.random_hierarchy(4, 3, 0.45, seed=11, bc=ah.SPHERE),
+}
+
+
+@pytest.mark.parametrize("ng", [2, 4])
+@pytest.mark.parametrize("which", sorted(EXCHANGE_HIERS))
+def test_hydro_boundary_region_sources(which, ng, gpu):
+    """Copies and interpolations only: bit for bit the oracle's staged passes."""
+    import torch
+    h = EXCHANGE_HIERS[which]()
+    lay = dict(LAY["hd"], ng=ng, stride=9 * (8 + 2 * ng) ** 3)
+    pool, su, s1, s2 = problems.blockmem_pool(h, lay, seed=65)
+    s = AmrSolver(h)
+    try:
+        s.set_blockmem(lay, pool.shape[0], su, s1, s2)
+        for level in range(h.nlev):
+            for mode in (1, 2):
+                exp = pool.copy()
+                oracle.bm_grid_boundary(exp, oracle.blockmem(**lay), h, su, s1, s2, level, mode)
+                dp = torch.from_numpy(pool).to(gpu)
+                s.hydro_boundary(dp, level, mode)
+                got = dp.cpu().numpy()
+                assert np.array_equal(got, exp), f"level {level} mode {mode}: " + _diff(got, exp)
+    finally:
+        s.close()
+
+
 def _diff(got, exp):
     bad = np.argwhere(got != exp)
     return f"{len(bad)} pool values differ, first {bad[:5].tolist()}"
