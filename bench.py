@@ -305,23 +305,28 @@ def bench_uniform(a, dev):
     ft = torch.tensor(f, device=dev)
     solver = UniformSolver(n, h, precisions=SG_PREC_FP64 | SG_PREC_MIXED)
 
-    def solve(prec, steps, warm):
+    def solve(prec, steps, warm, fused=True):
         psi = torch.zeros_like(ft)
         st = None
         for _ in range(warm):
             psi.zero_()
-            st = solver.cycle(psi, ft, tol=a.tol, maxit=60, precision=prec)
+            st = solver.cycle(psi, ft, tol=a.tol, maxit=60, precision=prec, fused=fused)
         torch.cuda.synchronize()
         t0 = time.perf_counter()
         for _ in range(steps):
             psi.zero_()
-            st = solver.cycle(psi, ft, tol=a.tol, maxit=60, precision=prec)
+            st = solver.cycle(psi, ft, tol=a.tol, maxit=60, precision=prec, fused=fused)
         torch.cuda.synchronize()
         ms = (time.perf_counter() - t0) * 1e3 / max(steps, 1)
         return ms, st, psi
 
+    # plain FP64: one kernel per reference loop nest, launched eagerly; then with the fused kernels
+    # (the solver's default, same bits)
     log("[bench] plain FP64 GPU solve")
-    ms64, st64, psi64 = solve(SG_PREC_FP64, max(1, a.uniform_steps // 2), 1)
+    ms64, st64, psi64 = solve(SG_PREC_FP64, max(1, a.uniform_steps // 2), 1, fused=False)
+    ms64_fz, _, psi64_fz = solve(SG_PREC_FP64, max(1, a.uniform_steps // 2), 1)
+    fz_same = bool(torch.equal(psi64, psi64_fz))
+    del psi64_fz
     log(f"[bench] fp64: {ms64:.3f} ms/solve, {st64['iterations']} it, rel {st64['rel_linf']:.3e}")
     log("[bench] mixed-precision GPU solve")
     msmx, stmx, psimx = solve(SG_PREC_MIXED, a.uniform_steps, 2)
@@ -418,6 +423,7 @@ def bench_uniform(a, dev):
         "workload": f"periodic {n}^3 clumpy-density Poisson solve to rel. residual {a.tol:g}",
         "n": n, "clumps": 8, "sigma_cells": 4, "seed": 0,
         "mixed_gpu_ms": round(msmx, 4), "fp64_gpu_ms": round(ms64, 4),
+        "fp64_gpu_ms_fused": round(ms64_fz, 4), "fp64_fused_bitwise_equal": fz_same,
         "speedup_mixed_vs_fp64": round(ms64 / msmx, 3),
         "iterations": {"mixed": stmx["iterations"], "fp64": st64["iterations"]},
         "rel_residual": {"mixed_linf": stmx["rel_linf"], "mixed_l2": stmx["rel_l2"], "fp64_linf": st64["rel_linf"]},

@@ -11,12 +11,14 @@
 // those device lists, eagerly or as a captured graph.  A problem that has converged is switched off
 // through a device activity flag and drops out of every later launch.
 //
-//  * FP64 (plain): one kernel per reference loop nest, as the single-grid plain solver, with
-//    general index arithmetic.  Each problem's values are bitwise those of the CPU restatement.
-//  * Mixed: FP32 inner mg_lin with the fused LDS-tiled sweeps, tiled tricubic prolongation and the
-//    single-workgroup coarse kernel (one workgroup per problem), tile shapes per level chosen by
-//    timing the batched launches; FP64 outer residual and update (ping-pong phi buffers).  A
-//    power-of-two problem gets bitwise the single-grid mixed solver's values.
+// Both precisions run mg_lin with the fused LDS-tiled sweeps, the tiled tricubic prolongation and the
+// single-workgroup coarse kernel (one workgroup per problem), and the FP64 outer residual and update
+// between two phi buffers:
+//  * FP64 (plain): the reference's cycle down to 1^3 (3^3); sweep shapes by rule.  Each problem's values
+//    are bitwise those of the CPU restatement.
+//  * Mixed: FP32 inner mg_lin, exact coarse-grid solve by default; sweep shapes per level chosen by
+//    timing the batched launches.  A power-of-two problem gets bitwise the single-grid mixed solver's
+//    values.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -55,11 +57,12 @@ struct sg_batch {
     std::vector<void *> allocs;
     std::vector<PL<double>> h_pl64;
     std::vector<PL<float>> h_pl32;
-    std::vector<CoarseDesc> h_desc;
+    std::vector<CoarseDesc<float>> h_desc;      // coarse kernel, FP32 and FP64
+    std::vector<CoarseDesc<double>> h_desc64;
     PL<double> *d_pl64 = nullptr;
     PL<float> *d_pl32 = nullptr;
-    CoarseDesc *d_desc = nullptr;
-    double *d_q3 = nullptr, *d_lam3 = nullptr;  // exact 3^3 solve: basis, eigenvalues per problem
+    CoarseDesc<float> *d_desc = nullptr;
+    CoarseDesc<double> *d_desc64 = nullptr;
     Outer *h_outer = nullptr, *d_outer = nullptr;
     int *h_active = nullptr, *d_active = nullptr;
     double *d_pmax = nullptr, *d_psum = nullptr;
@@ -70,14 +73,14 @@ struct sg_batch {
     float tune_ms[kBLev][32] = {};
     bool tuned = false;
     Plan plan[2];  // [0] FP64, [1] mixed
-    hipGraphExec_t graph[2] = {nullptr, nullptr};
-    int graph_plan_gen[2] = {-1, -1};
+    hipGraphExec_t graph[4] = {nullptr, nullptr, nullptr, nullptr};   // 2 mixed + phi-buffer parity
+    int graph_plan_gen[4] = {-1, -1, -1, -1};
     int plan_gen = 0;
     // executor state
     Plan *cur = nullptr;
     bool recording = false;
     size_t cursor = 0;
-    int ecode = CU;  // mixed: code of the FP32 buffer holding level 0's correction
+    int ecode = CU;  // code of the buffer holding level 0's correction
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -143,38 +146,6 @@ template <typename T> int pl_n(sg_batch *c, int p, int l)
 
 // ---- launches of the generic kernels --------------------------------------------------------
 
-template <typename T> int op_relax(sg_batch *c, const Pairs &pl, int cu, int crhs, int ipass)
-{
-    const Item *d;
-    int cnt, tot;
-    SG_TRY(take(c, pl, [&](int p, int l) {
-        const int n = pl_n<T>(c, p, l);
-        return n == 1 ? 1 : nblk_cells(cells(n) / 2);
-    }, &d, &cnt, &tot));
-    if (!cnt) return SG_OK;
-    hipLaunchKernelGGL(kb_relax<T>, dim3(tot), dim3(kThreads), 0, c->stream, bl<T>(c, d, cnt), cu, crhs, ipass);
-    SG_CHECK_LAUNCH();
-    return SG_OK;
-}
-
-// one mg_relax call (both colours) of each listed level
-template <typename T> int op_relax2(sg_batch *c, const Pairs &pl, int cu, int crhs)
-{
-    SG_TRY(op_relax<T>(c, pl, cu, crhs, 1));
-    return op_relax<T>(c, pl, cu, crhs, 2);
-}
-
-template <typename T> int op_resid(sg_batch *c, const Pairs &pl, int cres, int cu, int crhs)
-{
-    const Item *d;
-    int cnt, tot;
-    SG_TRY(take(c, pl, [&](int p, int l) { return nblk_cells(cells(pl_n<T>(c, p, l))); }, &d, &cnt, &tot));
-    if (!cnt) return SG_OK;
-    hipLaunchKernelGGL(kb_resid<T>, dim3(tot), dim3(kThreads), 0, c->stream, bl<T>(c, d, cnt), cres, cu, crhs);
-    SG_CHECK_LAUNCH();
-    return SG_OK;
-}
-
 // pairs name the coarse level
 template <typename T> int op_restrict(sg_batch *c, const Pairs &pl, int cdst, int csrc)
 {
@@ -188,251 +159,158 @@ template <typename T> int op_restrict(sg_batch *c, const Pairs &pl, int cdst, in
     return SG_OK;
 }
 
-template <typename T> int op_fill0(sg_batch *c, const Pairs &pl, int code)
-{
-    const Item *d;
-    int cnt, tot;
-    SG_TRY(take(c, pl, [&](int p, int l) { return nblk_cells(cells(pl_n<T>(c, p, l))); }, &d, &cnt, &tot));
-    if (!cnt) return SG_OK;
-    hipLaunchKernelGGL(kb_fill0<T>, dim3(tot), dim3(kThreads), 0, c->stream, bl<T>(c, d, cnt), code);
-    SG_CHECK_LAUNCH();
-    return SG_OK;
-}
+// ---- fused mg_lin over the batch (mg.F90:106-218) ---------------------------------------------------------
 
-// mg_interp (mg.F90:608-633) of each listed fine level from the next coarser one: tricubic for
-// the FMG step when the coarse grid plus ghosts is at least 4 wide, trilinear otherwise.  The
-// tricubic levels that an LDS tile shape (x extent 32, 16 or 8, widest first; 8 x 8 in y, z)
-// divides take the tiled form, the others the per-cell form (same values).
-template <typename T> int op_interp(sg_batch *c, const Pairs &pl, int cdst, int csrc, bool cubic, bool add)
-{
-    Pairs pc, pln, pt[3];
-    for (auto &q : pl) {
-        SG_REQUIRE(q.second + 1 < c->nlev[q.first], "batch schedule: interpolation from a missing level");
-        const int nc = pl_n<T>(c, q.first, q.second + 1), n = pl_n<T>(c, q.first, q.second);
-        if (!(cubic && nc + 2 >= 4 && !add)) {
-            (cubic && nc + 2 >= 4 ? pc : pln).push_back(q);
-            continue;
-        }
-        int g = -1;
-        for (int e = 0; e < 3 && g < 0; ++e)
-            if (n >= kCubicFXs[e] && n % kCubicFXs[e] == 0 && n % 8 == 0) g = e;
-        (g < 0 ? pc : pt[g]).push_back(q);
-    }
-    for (int e = 0; e < 3; ++e) {
-        const int fx = kCubicFXs[e];
-        const Item *d;
-        int cnt, tot;
-        SG_TRY(take(c, pt[e], [&](int p, int l) {
-            const int n = pl_n<T>(c, p, l);
-            return (n / fx) * (n / 8) * (n / 8);
-        }, &d, &cnt, &tot));
-        if (!cnt) continue;
-        const BL<T> L = bl<T>(c, d, cnt);
-        const dim3 grid(8 * ((tot + 7) / 8)), block(256);
-        if (fx == 32)
-            hipLaunchKernelGGL((kb_interp_cubic_tile_codes<32, 8, 8, 256, T>), grid, block, 0, c->stream, L, tot, cdst, csrc);
-        else if (fx == 16)
-            hipLaunchKernelGGL((kb_interp_cubic_tile_codes<16, 8, 8, 256, T>), grid, block, 0, c->stream, L, tot, cdst, csrc);
-        else
-            hipLaunchKernelGGL((kb_interp_cubic_tile_codes<8, 8, 8, 256, T>), grid, block, 0, c->stream, L, tot, cdst, csrc);
-        SG_CHECK_LAUNCH();
-    }
-    for (int pass = 0; pass < 2; ++pass) {
-        const Pairs &pp = pass == 0 ? pc : pln;
-        const Item *d;
-        int cnt, tot;
-        SG_TRY(take(c, pp, [&](int p, int l) { return nblk_cells(cells(pl_n<T>(c, p, l))); }, &d, &cnt, &tot));
-        if (!cnt) continue;
-        const BL<T> L = bl<T>(c, d, cnt);
-        if (pass == 0)
-            hipLaunchKernelGGL((kb_interp<T, true, false>), dim3(tot), dim3(kThreads), 0, c->stream, L, cdst, csrc);
-        else if (add)
-            hipLaunchKernelGGL((kb_interp<T, false, true>), dim3(tot), dim3(kThreads), 0, c->stream, L, cdst, csrc);
-        else
-            hipLaunchKernelGGL((kb_interp<T, false, false>), dim3(tot), dim3(kThreads), 0, c->stream, L, cdst, csrc);
-        SG_CHECK_LAUNCH();
-    }
-    return SG_OK;
-}
-
-// mg_slvsml (mg.F90:540-546) on each problem's coarsest level: two sweeps at 1^3 (only the second
-// colour has a cell), the exact solve at 3^3.
-int op_slvsml64(sg_batch *c, const Pairs &pl)
-{
-    Pairs p1, p3;
-    for (auto &q : pl) (pl_n<double>(c, q.first, q.second) == 3 ? p3 : p1).push_back(q);
-    for (int it = 0; it < 2; ++it) SG_TRY(op_relax<double>(c, p1, CU, CRHS, 2));
-    const Item *d;
-    int cnt, tot;
-    SG_TRY(take(c, p3, [](int, int) { return 1; }, &d, &cnt, &tot));
-    if (cnt) {
-        hipLaunchKernelGGL(kb_exact3<double>, dim3(tot), dim3(64), 0, c->stream, bl<double>(c, d, cnt), CU, CRHS,
-                           (const double *)c->d_q3, (const double *)c->d_lam3);
-        SG_CHECK_LAUNCH();
-    }
-    return SG_OK;
-}
-
-// ---- FP64 plain mg_lin over the batch (mg.F90:106-218) ----------------------------------------
-
-int plain_mg_lin(sg_batch *c, int ncycle, int npre, int npost)
-{
-    const int Lmax = c->maxlev - 1;
-    auto at = [&](int l, int minlev) {  // problems with more than minlev levels, at level l
-        return members(c, [&](int p) { return c->nlev[p] > minlev ? l : -1; });
-    };
-    for (int l = 1; l <= Lmax; ++l) SG_TRY(op_restrict<double>(c, at(l, l), CRHS, CRHS));
-    const Pairs bottom = members(c, [&](int p) { return c->nlev[p] - 1; });
-    SG_TRY(op_fill0<double>(c, bottom, CU));
-    SG_TRY(op_slvsml64(c, bottom));
-    for (int ml = Lmax - 1; ml >= 0; --ml) {
-        const Pairs M = at(ml, ml + 1);
-        const Pairs Mb = members(c, [&](int p) { return c->nlev[p] > ml + 1 ? c->nlev[p] - 1 : -1; });
-        SG_TRY(op_interp<double>(c, M, CU, CU, true, false));
-        for (int jc = 0; jc < ncycle; ++jc) {
-            for (int v = ml; v <= Lmax - 1; ++v) {
-                const Pairs Mv = at(v, v + 1), Mv1 = at(v + 1, v + 1);
-                for (int q = 0; q < npre; ++q) SG_TRY(op_relax2<double>(c, Mv, CU, CRHS));
-                SG_TRY(op_resid<double>(c, Mv, CRES, CU, CRHS));
-                SG_TRY(op_restrict<double>(c, Mv1, CRHS, CRES));
-                SG_TRY(op_fill0<double>(c, Mv1, CU));
-            }
-            SG_TRY(op_slvsml64(c, Mb));
-            for (int v = Lmax - 1; v >= ml; --v) {
-                const Pairs Mv = at(v, v + 1);
-                SG_TRY(op_interp<double>(c, Mv, CU, CU, false, true));
-                for (int q = 0; q < npost; ++q) SG_TRY(op_relax2<double>(c, Mv, CU, CRHS));
-            }
-        }
-    }
-    return SG_OK;
-}
-
-// ---- fused FP32 mg_lin over the batch ---------------------------------------------------------
-
-template <class TL, int NS, bool FS>
-void sweep_variant(sg_batch *c, const BL<float> &L, int tot, int cin, int cout, int cuc, bool zero, bool prolong,
+template <class TL, int NS, bool FS, typename T>
+void sweep_variant(sg_batch *c, const BL<T> &L, int tot, int cin, int cout, int cuc, bool zero, bool prolong,
                    bool resid)
 {
     const dim3 grid(8 * ((tot + 7) / 8)), block(TL::NT);
     if (resid && zero)
-        hipLaunchKernelGGL((kb_sweep<TL, NS, true, false, true, FS>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+        hipLaunchKernelGGL((kb_sweep<TL, NS, true, false, true, FS, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
     else if (resid)
-        hipLaunchKernelGGL((kb_sweep<TL, NS, false, false, true, FS>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+        hipLaunchKernelGGL((kb_sweep<TL, NS, false, false, true, FS, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
     else if (prolong)
-        hipLaunchKernelGGL((kb_sweep<TL, NS, false, true, false, FS>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+        hipLaunchKernelGGL((kb_sweep<TL, NS, false, true, false, FS, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
     else if (zero)
-        hipLaunchKernelGGL((kb_sweep<TL, NS, true, false, false, FS>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+        hipLaunchKernelGGL((kb_sweep<TL, NS, true, false, false, FS, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
     else
-        hipLaunchKernelGGL((kb_sweep<TL, NS, false, false, false, FS>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+        hipLaunchKernelGGL((kb_sweep<TL, NS, false, false, false, FS, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
 }
 
-template <class TL>
-void sweep_ns(sg_batch *c, int ns, bool fs, const BL<float> &L, int tot, int cin, int cout, int cuc, bool zero,
+template <class TL, typename T>
+void sweep_ns(sg_batch *c, int ns, bool fs, const BL<T> &L, int tot, int cin, int cout, int cuc, bool zero,
               bool prolong, bool resid)
 {
     if (ns == 2 && fs) {
-        if constexpr (sweep_fits_lds<TL, 2, true>()) sweep_variant<TL, 2, true>(c, L, tot, cin, cout, cuc, zero, prolong, resid);
+        if constexpr (sweep_built<TL, 2, true, T>())
+            sweep_variant<TL, 2, true, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid);
     } else if (ns == 2) {
-        if constexpr (sweep_fits_lds<TL, 2, false>()) sweep_variant<TL, 2, false>(c, L, tot, cin, cout, cuc, zero, prolong, resid);
+        if constexpr (sweep_built<TL, 2, false, T>())
+            sweep_variant<TL, 2, false, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid);
     } else if (fs) {
-        if constexpr (sweep_fits_lds<TL, 1, true>()) sweep_variant<TL, 1, true>(c, L, tot, cin, cout, cuc, zero, prolong, resid);
+        if constexpr (sweep_built<TL, 1, true, T>())
+            sweep_variant<TL, 1, true, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid);
     } else {
-        sweep_variant<TL, 1, false>(c, L, tot, cin, cout, cuc, zero, prolong, resid);
+        if constexpr (sweep_built<TL, 1, false, T>())
+            sweep_variant<TL, 1, false, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid);
     }
 }
 
-template <class SS>
-void stream_variant(sg_batch *c, const BL<float> &L, int tot, int cin, int cout, int cuc, bool zero, bool prolong,
+template <class SS, typename T>
+void stream_variant(sg_batch *c, const BL<T> &L, int tot, int cin, int cout, int cuc, bool zero, bool prolong,
                     bool resid)
 {
-    const dim3 grid(8 * ((tot + 7) / 8)), block(SS::NT);
-    if (resid && zero)
-        hipLaunchKernelGGL((kb_stream<SS, true, false, true>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
-    else if (resid)
-        hipLaunchKernelGGL((kb_stream<SS, false, false, true>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
-    else if (prolong)
-        hipLaunchKernelGGL((kb_stream<SS, false, true, false>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
-    else if (zero)
-        hipLaunchKernelGGL((kb_stream<SS, true, false, false>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
-    else
-        hipLaunchKernelGGL((kb_stream<SS, false, false, false>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+    if constexpr (stream_built<SS, T>()) {
+        const dim3 grid(8 * ((tot + 7) / 8)), block(SS::NT);
+        if (resid && zero)
+            hipLaunchKernelGGL((kb_stream<SS, true, false, true, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+        else if (resid)
+            hipLaunchKernelGGL((kb_stream<SS, false, false, true, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+        else if (prolong)
+            hipLaunchKernelGGL((kb_stream<SS, false, true, false, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+        else if (zero)
+            hipLaunchKernelGGL((kb_stream<SS, true, false, false, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+        else
+            hipLaunchKernelGGL((kb_stream<SS, false, false, false, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+    }
 }
 
 // ns fused sweeps of level l of the listed problems with tile shape cfg: buffer cin -> cout;
 // zero: start from u = 0; prolong: add the trilinear correction from level l + 1's buffer cuc;
 // resid: restrict the residual into level l + 1's RHS.
+template <typename T>
 int op_sweep_cfg(sg_batch *c, const Pairs &pl, int cfg, int ns, bool fs, int cin, int cout, int cuc, bool zero,
                  bool prolong, bool resid)
 {
-    SG_REQUIRE(cfg >= 0 && cfg < kNumCfg && cfg_ok(cfg, ns, fs), "bad sweep configuration %d/%d/%d", cfg, ns, (int)fs);
+    SG_REQUIRE(cfg >= 0 && cfg < kNumCfg && cfg_ok<T>(cfg, ns, fs), "bad sweep configuration %d/%d/%d", cfg, ns, (int)fs);
     const int *td = cfg < kNumTiles ? kTileDims[cfg] : kStreamDims[cfg - kNumTiles];
     for (auto &q : pl) {
         SG_REQUIRE(q.second < c->lc[q.first], "batch schedule: fused sweep on a coarse-kernel level");
-        SG_REQUIRE(cfg_fits(cfg, c->h_pl32[q.first * kBLev + q.second].n), "sweep shape %d does not fit n = %d", cfg,
-                   c->h_pl32[q.first * kBLev + q.second].n);
-        SG_REQUIRE(c->h_pl32[q.first * kBLev + q.second].n > 2 * (2 * ns + 1), "tile halo wider than the grid");
+        SG_REQUIRE(cfg_fits(cfg, pl_n<T>(c, q.first, q.second)), "sweep shape %d does not fit n = %d", cfg,
+                   pl_n<T>(c, q.first, q.second));
+        SG_REQUIRE(pl_n<T>(c, q.first, q.second) > 2 * (2 * ns + 1), "tile halo wider than the grid");
     }
     const Item *d;
     int cnt, tot;
     SG_TRY(take(c, pl, [&](int p, int l) {
-        const int n = c->h_pl32[p * kBLev + l].n;
+        const int n = pl_n<T>(c, p, l);
         return (n / td[0]) * (n / td[1]) * (n / td[2]);
     }, &d, &cnt, &tot));
     if (!cnt) return SG_OK;
-    const BL<float> L = bl<float>(c, d, cnt);
+    const BL<T> L = bl<T>(c, d, cnt);
     switch (cfg) {
-    case kNumTiles + 0: stream_variant<Stream0>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 1: stream_variant<Stream1>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 2: stream_variant<Stream2>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 3: stream_variant<Stream3>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 4: stream_variant<Stream4>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 5: stream_variant<Stream5>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 6: stream_variant<Stream6>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 7: stream_variant<Stream7>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 8: stream_variant<Stream8>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case 0: sweep_ns<Tile0>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case 1: sweep_ns<Tile1>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case 2: sweep_ns<Tile2>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case 3: sweep_ns<Tile3>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    default: sweep_ns<Tile4>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 0: stream_variant<Stream0, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 1: stream_variant<Stream1, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 2: stream_variant<Stream2, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 3: stream_variant<Stream3, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 4: stream_variant<Stream4, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 5: stream_variant<Stream5, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 6: stream_variant<Stream6, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 7: stream_variant<Stream7, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 8: stream_variant<Stream8, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case 0: sweep_ns<Tile0, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case 1: sweep_ns<Tile1, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case 2: sweep_ns<Tile2, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case 3: sweep_ns<Tile3, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    default: sweep_ns<Tile4, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     }
     SG_CHECK_LAUNCH();
     return SG_OK;
 }
 
-int op_interp_cubic_tile(sg_batch *c, const Pairs &pl, int fx, int cuc)
+template <typename T> int op_interp_cubic_tile(sg_batch *c, const Pairs &pl, int fx, int cuc)
 {
     for (auto &q : pl) {
-        const int n = c->h_pl32[q.first * kBLev + q.second].n;
+        const int n = pl_n<T>(c, q.first, q.second);
         SG_REQUIRE(q.second < c->lc[q.first] && n >= fx && n % fx == 0 && n % 8 == 0,
                    "batch schedule: tricubic tile %d does not fit n = %d", fx, n);
     }
     const Item *d;
     int cnt, tot;
     SG_TRY(take(c, pl, [&](int p, int l) {
-        const int n = c->h_pl32[p * kBLev + l].n;
+        const int n = pl_n<T>(c, p, l);
         return (n / fx) * (n / 8) * (n / 8);
     }, &d, &cnt, &tot));
     if (!cnt) return SG_OK;
-    const BL<float> L = bl<float>(c, d, cnt);
+    const BL<T> L = bl<T>(c, d, cnt);
     const dim3 grid(8 * ((tot + 7) / 8)), block(256);
-    if (fx == 32) hipLaunchKernelGGL((kb_interp_cubic_tile<32, 8, 8, 256>), grid, block, 0, c->stream, L, tot, cuc);
-    else if (fx == 16) hipLaunchKernelGGL((kb_interp_cubic_tile<16, 8, 8, 256>), grid, block, 0, c->stream, L, tot, cuc);
-    else hipLaunchKernelGGL((kb_interp_cubic_tile<8, 8, 8, 256>), grid, block, 0, c->stream, L, tot, cuc);
+    if (fx == 32) hipLaunchKernelGGL((kb_interp_cubic_tile<32, 8, 8, 256, T>), grid, block, 0, c->stream, L, tot, cuc);
+    else if (fx == 16) hipLaunchKernelGGL((kb_interp_cubic_tile<16, 8, 8, 256, T>), grid, block, 0, c->stream, L, tot, cuc);
+    else hipLaunchKernelGGL((kb_interp_cubic_tile<8, 8, 8, 256, T>), grid, block, 0, c->stream, L, tot, cuc);
     SG_CHECK_LAUNCH();
     return SG_OK;
 }
 
-int op_coarse(sg_batch *c, const Pairs &pl, int mode, int ncycle, int npre, int npost, bool exact)
+// Coarse-grid solve of each pair's first level of <= 16^3 cells: the reference's cycles from there down;
+// exact (FP32): the exact solve, for the problems with finer levels.
+template <typename T> int op_coarse(sg_batch *c, const Pairs &pl, int mode, int ncycle, int npre, int npost, bool exact)
 {
+    Pairs cyc;
     for (auto &q : pl) SG_REQUIRE(q.second == c->lc[q.first], "batch schedule: coarse kernel off its level");
+    if constexpr (std::is_same<T, float>::value) {
+        Pairs ex;
+        for (auto &q : pl) (exact && c->h_desc[q.first].exact ? ex : cyc).push_back(q);
+        const Item *d;
+        int cnt, tot;
+        SG_TRY(take(c, ex, [](int, int) { return 1; }, &d, &cnt, &tot));
+        if (cnt) {
+            hipLaunchKernelGGL(kb_coarse_exact, dim3(tot), dim3(kCoarseThreads), 0, c->stream, bl<float>(c, d, cnt),
+                               (const CoarseDesc<float> *)c->d_desc);
+            SG_CHECK_LAUNCH();
+        }
+    } else {
+        cyc = pl;
+    }
+    const CoarseDesc<T> *desc;
+    if constexpr (std::is_same<T, float>::value) desc = c->d_desc;
+    else desc = c->d_desc64;
     const Item *d;
     int cnt, tot;
-    SG_TRY(take(c, pl, [](int, int) { return 1; }, &d, &cnt, &tot));
+    SG_TRY(take(c, cyc, [](int, int) { return 1; }, &d, &cnt, &tot));
     if (!cnt) return SG_OK;
-    hipLaunchKernelGGL(kb_coarse, dim3(tot), dim3(kCoarseThreads), 0, c->stream, bl<float>(c, d, cnt),
-                       (const CoarseDesc *)c->d_desc, mode, ncycle, npre, npost, exact ? 1 : 0);
+    hipLaunchKernelGGL(kb_coarse<T>, dim3(tot), dim3(kCoarseThreads), 0, c->stream, bl<T>(c, d, cnt), desc, mode, ncycle,
+                       npre, npost);
     SG_CHECK_LAUNCH();
     return SG_OK;
 }
@@ -442,15 +320,15 @@ int op_coarse(sg_batch *c, const Pairs &pl, int mode, int ncycle, int npre, int 
 int op_exact_planes(sg_batch *c, const Pairs &pl)
 {
     for (auto &q : pl) {
-        const int n = c->h_pl32[q.first * kBLev + q.second].n;
+        const int n = pl_n<float>(c, q.first, q.second);
         SG_REQUIRE(q.second == c->lb[q.first] && q.second != c->lc[q.first] && c->h_desc[q.first].qp &&
                        n <= kPlaneMaxN && n % 4 == 0,
                    "batch schedule: plane-parallel exact solve off its level");
     }
     const Item *d;
     int cnt, tot;
-    auto planes = [&](int p, int l) { return c->h_pl32[p * kBLev + l].n; };
-    const CoarseDesc *D = (const CoarseDesc *)c->d_desc;
+    auto planes = [&](int p, int l) { return pl_n<float>(c, p, l); };
+    const CoarseDesc<float> *D = c->d_desc;
     for (int step = 0; step < 3; ++step) {
         SG_TRY(take(c, pl, planes, &d, &cnt, &tot));
         if (!cnt) continue;
@@ -464,11 +342,49 @@ int op_exact_planes(sg_batch *c, const Pairs &pl)
     return SG_OK;
 }
 
-// mg_lin in FP32 with the fused kernels (the single-grid fused mg_lin, stepped over all problems
+// sweeps per launch on level v (of every problem there, so that all keep u in the same buffer)
+template <typename T> int level_ns(sg_batch *c, int v)
+{
+    if constexpr (std::is_same<T, float>::value) return c->tile_ns[v];
+    long m = 0;
+    for (int p = 0; p < c->np; ++p)
+        if (c->lc[p] > v) m += cells(c->n[p] >> v);
+    return fp64_two_sweeps(m) ? 2 : 1;
+}
+
+// ns sweeps of level v of the listed problems.  FP32: one launch with the autotuned shape.  FP64: the
+// problems whose width is a multiple of 32 apart from the others, so that one 24^3 or 48^3 problem does
+// not hold the large ones to an 8^3 or 16 x 8 x 8 tile (12 problems of 24 ... 128: three 128^3 levels
+// took 58 us per sweep in a shape fitting all of 32 x 16 columns).
+template <typename T>
+int op_sweep(sg_batch *c, const Pairs &pl, int v, int ns, int cin, int cout, int cuc, bool zero, bool prolong, bool resid)
+{
+    if constexpr (std::is_same<T, float>::value) {
+        return op_sweep_cfg<T>(c, pl, c->tile_cfg[v], ns, c->tile_fs[v] != 0, cin, cout, cuc, zero, prolong, resid);
+    } else {
+        const bool two = level_ns<T>(c, v) == 2;
+        for (int cls = 0; cls < 2; ++cls) {
+            Pairs w;
+            int unit = 64;
+            long m = 0;
+            for (auto &q : pl) {
+                const int n = c->n[q.first] >> q.second;
+                if ((n % 32 != 0) != (cls == 1)) continue;
+                while (n % unit) unit /= 2;
+                m += cells(n);
+                w.push_back(q);
+            }
+            SG_TRY(op_sweep_cfg<T>(c, w, fp64_sweep_shape(unit, m, two), ns, false, cin, cout, cuc, zero, prolong, resid));
+        }
+        return SG_OK;
+    }
+}
+
+// mg_lin with the fused kernels (the single-grid fused mg_lin, stepped over all problems
 // with the same fine level index at once).  c->ecode receives the buffer code that holds level 0's
 // correction for problems with at least one fine level.  exact: the cycle of a problem with finer
-// levels ends at its level lb, solved exactly (as the single-grid solver's SG_COARSE_EXACT).
-int fast_mg_lin(sg_batch *c, int ncycle, int npre, int npost, bool exact)
+// levels ends at its level lb, solved exactly (FP32; as the single-grid solver's SG_COARSE_EXACT).
+template <typename T> int fast_mg_lin(sg_batch *c, int ncycle, int npre, int npost, bool exact)
 {
     const std::vector<int> &bot = exact ? c->lb : c->lc;  // level of each problem's coarse-grid solve
     const int maxlc = exact ? c->maxlb : c->maxlc;
@@ -478,29 +394,28 @@ int fast_mg_lin(sg_batch *c, int ncycle, int npre, int npost, bool exact)
     // coarse-grid solve of the problems selected by pred: k_coarse, or the plane-parallel kernels
     auto bottom = [&](auto pred, int mode) -> int {
         auto planes = [&](int p) { return exact && c->lb[p] != c->lc[p]; };
-        SG_TRY(op_coarse(c, members(c, [&](int p) { return pred(p) && !planes(p) ? c->lc[p] : -1; }), mode, ncycle,
+        SG_TRY(op_coarse<T>(c, members(c, [&](int p) { return pred(p) && !planes(p) ? c->lc[p] : -1; }), mode, ncycle,
                          npre, npost, exact));
         if (exact) SG_TRY(op_exact_planes(c, members(c, [&](int p) { return pred(p) && planes(p) ? c->lb[p] : -1; })));
         return SG_OK;
     };
     for (int l = 1; l <= maxlc; ++l)
-        SG_TRY(op_restrict<float>(c, members(c, [&](int p) { return bot[p] >= l ? l : -1; }), CRHS, CRHS));
+        SG_TRY(op_restrict<T>(c, members(c, [&](int p) { return bot[p] >= l ? l : -1; }), CRHS, CRHS));
     SG_TRY(bottom([&](int p) { return bot[p] == 0; }, 0));
     int cur[kBLev] = {};
     auto code = [](int b) { return b ? CU1 : CU; };
     for (int ml = maxlc - 1; ml >= 0; --ml) {
         SG_TRY(bottom([&](int p) { return bot[p] == ml + 1; }, 0));
         const Pairs M = fine_at(ml, ml);
-        SG_TRY(op_interp_cubic_tile(c, M, c->cubic_fx[ml], code(cur[ml + 1])));
+        SG_TRY(op_interp_cubic_tile<T>(c, M, c->cubic_fx[ml], code(cur[ml + 1])));
         cur[ml] = 0;
         for (int jc = 0; jc < ncycle; ++jc) {
             for (int v = ml; v <= maxlc - 1; ++v) {
                 const Pairs Mv = fine_at(v, v);
                 for (int r = npre, first = 1; r > 0; first = 0) {
-                    const int k = std::min(r, c->tile_ns[v]);
+                    const int k = std::min(r, level_ns<T>(c, v));
                     const bool last = r == k;
-                    SG_TRY(op_sweep_cfg(c, Mv, c->tile_cfg[v], k, c->tile_fs[v] != 0, code(cur[v]), code(1 - cur[v]),
-                                        CU, first && v > ml, false, last));
+                    SG_TRY(op_sweep<T>(c, Mv, v, k, code(cur[v]), code(1 - cur[v]), CU, first && v > ml, false, last));
                     cur[v] ^= 1;
                     r -= k;
                 }
@@ -509,9 +424,8 @@ int fast_mg_lin(sg_batch *c, int ncycle, int npre, int npost, bool exact)
             for (int v = maxlc - 1; v >= ml; --v) {
                 const Pairs Mv = fine_at(v, v);
                 for (int r = npost, first = 1; r > 0; first = 0) {
-                    const int k = std::min(r, c->tile_ns[v]);
-                    SG_TRY(op_sweep_cfg(c, Mv, c->tile_cfg[v], k, c->tile_fs[v] != 0, code(cur[v]), code(1 - cur[v]),
-                                        code(cur[v + 1]), false, first, false));
+                    const int k = std::min(r, level_ns<T>(c, v));
+                    SG_TRY(op_sweep<T>(c, Mv, v, k, code(cur[v]), code(1 - cur[v]), code(cur[v + 1]), false, first, false));
                     cur[v] ^= 1;
                     r -= k;
                 }
@@ -588,11 +502,11 @@ int run_init(sg_batch *c, bool mixed)
 int run_iteration(sg_batch *c, bool mixed, const sg_params *p, int parity)
 {
     if (mixed) {
-        SG_TRY(fast_mg_lin(c, p->ncycle, p->npre, p->npost, p->coarse == SG_COARSE_EXACT));
+        SG_TRY(fast_mg_lin<float>(c, p->ncycle, p->npre, p->npost, p->coarse == SG_COARSE_EXACT));
         return op_outer_resid<float>(c, parity, true, c->ecode);
     }
-    SG_TRY(plain_mg_lin(c, p->ncycle, p->npre, p->npost));
-    return op_outer_resid<double>(c, parity, true, CU);
+    SG_TRY(fast_mg_lin<double>(c, p->ncycle, p->npre, p->npost, false));
+    return op_outer_resid<double>(c, parity, true, c->ecode);
 }
 
 // Record the launch sequence of (precision, cycle shape) once and upload its item lists.
@@ -627,13 +541,14 @@ int replay_iteration(sg_batch *c, bool mixed, const sg_params *p, int parity)
 {
     Plan &P = c->plan[mixed ? 1 : 0];
     c->cur = &P;
-    if (!(mixed && p->use_graph)) {
+    if (!p->use_graph) {
         c->cursor = P.iter_begin;
         return run_iteration(c, mixed, p, parity);
     }
-    if (!c->graph[parity] || c->graph_plan_gen[parity] != c->plan_gen) {
-        if (c->graph[parity]) (void)hipGraphExecDestroy(c->graph[parity]);
-        c->graph[parity] = nullptr;
+    const int gi = (mixed ? 2 : 0) + parity;
+    if (!c->graph[gi] || c->graph_plan_gen[gi] != c->plan_gen) {
+        if (c->graph[gi]) (void)hipGraphExecDestroy(c->graph[gi]);
+        c->graph[gi] = nullptr;
         hipGraph_t g = nullptr;
         c->cursor = P.iter_begin;
         SG_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
@@ -644,12 +559,12 @@ int replay_iteration(sg_batch *c, bool mixed, const sg_params *p, int parity)
             return rc;
         }
         SG_HIP(e);
-        const hipError_t e2 = hipGraphInstantiate(&c->graph[parity], g, nullptr, nullptr, 0);
+        const hipError_t e2 = hipGraphInstantiate(&c->graph[gi], g, nullptr, nullptr, 0);
         (void)hipGraphDestroy(g);
         SG_HIP(e2);
-        c->graph_plan_gen[parity] = c->plan_gen;
+        c->graph_plan_gen[gi] = c->plan_gen;
     }
-    SG_HIP(hipGraphLaunch(c->graph[parity], c->stream));
+    SG_HIP(hipGraphLaunch(c->graph[gi], c->stream));
     return SG_OK;
 }
 
@@ -666,24 +581,13 @@ int autotune(sg_batch *c)
     int rc = SG_OK;
     for (int v = 0; v < c->maxlc && rc == SG_OK; ++v) {
         const Pairs Mv = members(c, [&](int p) { return c->lc[p] > v ? v : -1; });
-        // tricubic tile: the widest x extent that divides every member's level
-        c->cubic_fx[v] = 0;
-        for (int fx : kCubicFXs) {
-            bool ok = true;
-            for (auto &q : Mv) {
-                const int n = c->h_pl32[q.first * kBLev + v].n;
-                ok = ok && n >= fx && n % fx == 0 && n % 8 == 0;
-            }
-            if (ok) { c->cubic_fx[v] = fx; break; }
-        }
-        if (c->cubic_fx[v] == 0) { set_error("no tricubic tile fits level %d", v); rc = SG_ERR_ARG; break; }
         c->tile_cfg[v] = -1;
         float best = 1e30f;
         for (int cand = 0; cand < kNumCand && rc == SG_OK; ++cand) {
             int cfg, ns;
             bool fs;
             cand_decode(cand, cfg, ns, fs);
-            bool fits = cfg_ok(cfg, ns, fs);
+            bool fits = cfg_ok<float>(cfg, ns, fs);
             for (auto &q : Mv) fits = fits && cfg_fits(cfg, c->h_pl32[q.first * kBLev + v].n);
             c->tune_ms[v][cand] = -1.f;
             if (!fits) continue;
@@ -693,7 +597,7 @@ int autotune(sg_batch *c)
             int flip = 0;
             auto visit = [&]() -> int {
                 auto one = [&](int k, bool prolong, bool resid) {
-                    const int r = op_sweep_cfg(c, Mv, cfg, k, fs, flip ? CU1 : CU, flip ? CU : CU1, CU, false, prolong,
+                    const int r = op_sweep_cfg<float>(c, Mv, cfg, k, fs, flip ? CU1 : CU, flip ? CU : CU1, CU, false, prolong,
                                                resid);
                     flip ^= 1;
                     return r;
@@ -891,9 +795,8 @@ int create(sg_batch **out, int np, const int *ns, const double *hs, int precisio
     c->lb.resize(np);
     c->h_pl64.assign((size_t)np * kBLev, PL<double>{});
     c->h_pl32.assign((size_t)np * kBLev, PL<float>{});
-    c->h_desc.assign(np, CoarseDesc{});
-    std::vector<double> lam3(3 * np, 0.0), q3(9, 0.0), lamtmp(3);
-    hartley_basis(3, 1.0, q3.data(), lamtmp.data());
+    c->h_desc.assign(np, CoarseDesc<float>{});
+    c->h_desc64.assign(np, CoarseDesc<double>{});
     auto fail = [&](int rc) { destroy(c); return rc; };
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
@@ -933,7 +836,6 @@ int create(sg_batch **out, int np, const int *ns, const double *hs, int precisio
             a.n = b.n = m;
             a.lc = b.lc = lc;
             a.dn = b.dn = make_div((unsigned)m);
-            a.dnh = b.dnh = make_div((unsigned)std::max(m / 2, 1));
             a.h2 = hl * hl;
             a.h2i = 1.0 / (hl * hl);
             b.h2 = (float)(hl * hl);
@@ -941,43 +843,30 @@ int create(sg_batch **out, int np, const int *ns, const double *hs, int precisio
             const size_t len = (size_t)cells(m);
             int rc = SG_OK;
             if (precisions & SG_PREC_FP64) {
-                double *u, *rhs, *res;
-                if ((rc = dev_alloc(c, &u, len)) || (rc = dev_alloc(c, &rhs, len)) || (rc = dev_alloc(c, &res, len)))
+                double *u, *u1, *rhs;
+                if ((rc = dev_alloc(c, &u, len)) || (rc = dev_alloc(c, &u1, len)) || (rc = dev_alloc(c, &rhs, len)))
                     return fail(rc);
-                a.a[CU] = u; a.a[CRHS] = rhs; a.a[CRES] = res; a.a[CU1] = nullptr;
+                a.a[CU] = u; a.a[CU1] = u1; a.a[CRHS] = rhs;
             }
             if (precisions & SG_PREC_MIXED) {
                 float *u, *u1, *rhs;
                 if ((rc = dev_alloc(c, &u, len)) || (rc = dev_alloc(c, &u1, len)) || (rc = dev_alloc(c, &rhs, len)))
                     return fail(rc);
-                b.a[CU] = u; b.a[CU1] = u1; b.a[CRHS] = rhs; b.a[CRES] = nullptr;
-            }
-            if (m == 3) {
-                double Qd[9], ld[3];
-                hartley_basis(3, hl, Qd, ld);
-                for (int e = 0; e < 3; ++e) lam3[3 * q + e] = ld[e];
+                b.a[CU] = u; b.a[CU1] = u1; b.a[CRHS] = rhs;
             }
         }
         // coarse kernel levels: lc .. nlev-1
-        CoarseDesc &D = c->h_desc[q];
-        D.nlev = nl - lc;
-        int off = 0;
-        for (int k = 0; k < D.nlev; ++k) {
-            const int l = lc + k, m = ns[q] >> l;
-            const double hl = hs[q] * (double)(1 << l);
-            D.n[k] = m;
-            D.h2[k] = (float)(hl * hl);
-            D.h2i[k] = (float)(1.0 / (hl * hl));
-            D.off[k] = off;
-            D.dn[k] = make_div((unsigned)m);
-            D.dnh[k] = make_div((unsigned)std::max(m / 2, 1));
-            off += m * m * m;
-            if (m == 3) {
-                double Qd[9], ld[3];
-                hartley_basis(3, hl, Qd, ld);
-                for (int e = 0; e < 9; ++e) D.q3[e] = (float)Qd[e];
-                for (int e = 0; e < 3; ++e) D.lam3[e] = (float)ld[e];
-            }
+        CoarseDesc<float> &D = c->h_desc[q];
+        CoarseDesc<double> &D64 = c->h_desc64[q];
+        const double hc = hs[q] * (double)(1 << lc);
+        D.n = D64.n = ns[q] >> lc;
+        D.coef = coarse_coef<float>(hc);
+        D64.coef = coarse_coef<double>(hc);
+        if ((ns[q] >> (nl - 1)) == 3) {
+            double Qd[9], ld[3];
+            hartley_basis(3, hs[q] * (double)(1 << (nl - 1)), Qd, ld);
+            for (int e = 0; e < 9; ++e) { D64.coef.q3[e] = Qd[e]; D.coef.q3[e] = (float)Qd[e]; }
+            for (int e = 0; e < 3; ++e) { D64.coef.lam3[e] = ld[e]; D.coef.lam3[e] = (float)ld[e]; }
         }
         // exact solve of held level 0 when the problem has finer levels (SG_COARSE_EXACT)
         D.exact = lc > 0 ? 1 : 0;
@@ -1010,15 +899,19 @@ int create(sg_batch **out, int np, const int *ns, const double *hs, int precisio
             D.qp = qp;
             D.invp = invp;
         }
-        if (off > kCoarseCellsB || D.nlev > 8) {
-            set_error("problem %d: coarse levels exceed the coarse kernel's capacity", q);
-            return fail(SG_ERR_ARG);
-        }
     }
+    // tricubic tile per level: the widest x extent that divides every member's level
+    for (int v = 0; v < c->maxlc; ++v)
+        for (int fx : kCubicFXs) {
+            bool ok = true;
+            for (int q = 0; q < np; ++q)
+                if (c->lc[q] > v) ok = ok && (ns[q] >> v) % fx == 0 && (ns[q] >> v) % 8 == 0;
+            if (ok) { c->cubic_fx[v] = fx; break; }
+        }
     int rc = SG_OK;
     if ((rc = dev_alloc(c, &c->d_pl64, c->h_pl64.size())) || (rc = dev_alloc(c, &c->d_pl32, c->h_pl32.size())) ||
-        (rc = dev_alloc(c, &c->d_desc, c->h_desc.size())) || (rc = dev_alloc(c, &c->d_q3, 9)) ||
-        (rc = dev_alloc(c, &c->d_lam3, lam3.size())) || (rc = dev_alloc(c, &c->d_outer, 1)) ||
+        (rc = dev_alloc(c, &c->d_desc, c->h_desc.size())) || (rc = dev_alloc(c, &c->d_desc64, c->h_desc64.size())) ||
+        (rc = dev_alloc(c, &c->d_outer, 1)) ||
         (rc = dev_alloc(c, &c->d_active, np)) || (rc = dev_alloc(c, &c->d_pmax, part)) ||
         (rc = dev_alloc(c, &c->d_psum, part)) || (rc = dev_alloc(c, &c->d_norm, 2 * np)) ||
         (rc = dev_alloc(c, &c->d_snorm, 2 * np)))
@@ -1040,9 +933,9 @@ int create(sg_batch **out, int np, const int *ns, const double *hs, int precisio
     }
     if (hipMemcpy(c->d_pl64, c->h_pl64.data(), sizeof(PL<double>) * c->h_pl64.size(), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_pl32, c->h_pl32.data(), sizeof(PL<float>) * c->h_pl32.size(), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->d_desc, c->h_desc.data(), sizeof(CoarseDesc) * c->h_desc.size(), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->d_q3, q3.data(), sizeof(double) * 9, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(c->d_lam3, lam3.data(), sizeof(double) * lam3.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(c->d_desc, c->h_desc.data(), sizeof(c->h_desc[0]) * c->h_desc.size(), hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(c->d_desc64, c->h_desc64.data(), sizeof(c->h_desc64[0]) * c->h_desc64.size(), hipMemcpyHostToDevice) !=
+            hipSuccess ||
         hipMemcpy(c->d_outer, c->h_outer, sizeof(Outer), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(c->d_active, c->h_active, sizeof(int) * np, hipMemcpyHostToDevice) != hipSuccess) {
         set_error("table upload failed");

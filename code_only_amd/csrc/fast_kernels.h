@@ -1,4 +1,4 @@
-// Fused FP32 kernels of the mixed-precision inner solve (gfx950).
+// Fused kernels of the inner solve (gfx950), in FP32 (mixed precision) and FP64 (plain).
 //
 //  * k_sweep_tile: one full red-black sweep (mg_poisson.F90:55-74, both colours) of a TX*TY*TZ
 //    tile held in LDS with an H-cell halo, optionally
@@ -14,10 +14,10 @@
 //    timing (all shapes give identical values).
 //  * k_interp_cubic_tile: the FMG tricubic prolongation (interpolation.F90:98-217) as the
 //    reference's three separable passes, on an LDS-staged coarse tile.
-//  * k_coarse: every level of <= 16^3 cells in one workgroup's LDS: the FMG part of mg_lin
-//    (mg.F90:142-215) from the coarsest level up to the first fine level, or one V-cycle from that
-//    level down and back (the bottom of each fine-level V-cycle); or, in both places, the exact
-//    solve of the first level of <= 16^3 cells by Hartley transforms (coarse_exact).
+//  * k_coarse: every level of <= 16^3 cells in one workgroup's LDS (coarse_levels.h): the FMG part of
+//    mg_lin (mg.F90:142-215) from the coarsest level up to the first fine level, or one V-cycle from
+//    that level down and back (the bottom of each fine-level V-cycle); k_coarse_exact: in both places,
+//    the exact solve of the first level of <= 16^3 cells by Hartley transforms (coarse_exact).
 //
 // Every cell value is produced by the same helpers (relax_value, resid_value, restrict_value,
 // trilinear_value, cubic_stencil) as the one-kernel-per-loop path, in the same order, so the fused
@@ -25,64 +25,12 @@
 #pragma once
 #include <cmath>
 
+#include "coarse_levels.h"
 #include "uniform_kernels.h"
 
 namespace sg {
 
-constexpr int kCoarseMaxN = 16;
-constexpr int kCoarseThreads = 1024;
-
 __device__ __forceinline__ int wrapn(int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); }
-
-// Trilinear prolongation value at fine cell (i, j, k) of a periodic coarse grid of nc cells;
-// C(a, b, d) returns coarse cell (a, b, d).
-template <typename T, typename Acc>
-__device__ __forceinline__ T trilinear_point(const Acc &C, int i, int j, int k, int nc)
-{
-    const int ic = i >> 1, jc = j >> 1, kc = k >> 1;
-    const int ic1 = wrap_g(ic + 2 * (i & 1) - 1, nc);
-    const int jc1 = wrap_g(jc + 2 * (j & 1) - 1, nc);
-    const int kc1 = wrap_g(kc + 2 * (k & 1) - 1, nc);
-    return trilinear_value<T>(C(ic, jc, kc), C(ic1, jc, kc), C(ic, jc1, kc), C(ic, jc, kc1), C(ic, jc1, kc1),
-                              C(ic1, jc, kc1), C(ic1, jc1, kc), C(ic1, jc1, kc1));
-}
-
-// 4-point cubic combination in the reference's order: (a0 v0 + a1 v1) + a2 v2 + a3 v3.
-template <typename T> __device__ __forceinline__ T cubic4(const T w[4], T v0, T v1, T v2, T v3)
-{
-    T s = w[0] * v0 + w[1] * v1;
-    s = s + w[2] * v2;
-    s = s + w[3] * v3;
-    return s;
-}
-
-// Tricubic value at fine cell (i, j, k) (interpolation.F90:98-217), nc >= 2.
-template <typename T, typename Acc>
-__device__ __forceinline__ T tricubic_point(const Acc &C, int i, int j, int k, int nc)
-{
-    int ix[4], iy[4], iz[4];
-    double ax[4], ay[4], az[4];
-    cubic_stencil(i, -1, nc, ix, ax);
-    cubic_stencil(j, -1, nc, iy, ay);
-    cubic_stencil(k, -1, nc, iz, az);
-    T wx[4], wy[4], wz[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        wx[q] = (T)ax[q]; wy[q] = (T)ay[q]; wz[q] = (T)az[q];
-        ix[q] = wrap_g(ix[q], nc); iy[q] = wrap_g(iy[q], nc); iz[q] = wrap_g(iz[q], nc);
-    }
-    T bz[4];
-#pragma unroll
-    for (int kq = 0; kq < 4; ++kq) {
-        T by[4];
-#pragma unroll
-        for (int jq = 0; jq < 4; ++jq)
-            by[jq] = cubic4<T>(wx, C(ix[0], iy[jq], iz[kq]), C(ix[1], iy[jq], iz[kq]), C(ix[2], iy[jq], iz[kq]),
-                               C(ix[3], iy[jq], iz[kq]));
-        bz[kq] = cubic4<T>(wy, by[0], by[1], by[2], by[3]);
-    }
-    return cubic4<T>(wz, bz[0], bz[1], bz[2], bz[3]);
-}
 
 // Tile index with XCD-aware placement: consecutive workgroups are dealt round-robin to the 8
 // XCDs, so workgroup b is given tile (b % 8) * per + b / 8 -- each XCD works through a contiguous
@@ -119,23 +67,23 @@ inline bool tile_fits(int cfg, int n)
 // One colour of the sweep over the LDS region shrunk by margin M: cells with
 // (gx + gy + gz) % 2 == colour, where colour 1 is the reference's first pass (ipass = 1).  The
 // source values are fetched for all of a thread's cells before any update.
-template <class TL, int LX, int LY, int LZ, int M, int H, bool FS>
-__device__ __forceinline__ void tile_colour(float *su, const float *sf, const float *__restrict__ f, int n, int x0,
-                                            int y0, int z0, int colour, float h2, double &amax)
+template <class TL, int LX, int LY, int LZ, int M, int H, bool FS, typename T>
+__device__ __forceinline__ void tile_colour(T *su, const T *sf, const T *__restrict__ f, int n, int x0,
+                                            int y0, int z0, int colour, T h2, double &amax)
 {
     constexpr int RX = (LX - 2 * M) / 2, RY = LY - 2 * M, RZ = LZ - 2 * M;
     constexpr int CNT = RX * RY * RZ;
     constexpr int IT = (CNT + TL::NT - 1) / TL::NT;
     static_assert((LX - 2 * M) % 2 == 0, "region x extent must be even");
     static_assert(IT <= 32, "too many cells per thread");
-    float fv[IT];
+    T fv[IT];
     int cv[IT];
     unsigned core = 0u;
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
         const int q = threadIdx.x + it * TL::NT;
         cv[it] = -1;
-        fv[it] = 0.0f;
+        fv[it] = T(0);
         if (CNT % TL::NT == 0 || q < CNT) {
             const int xh = q % RX;
             const int y = M + (q / RX) % RY;
@@ -156,9 +104,9 @@ __device__ __forceinline__ void tile_colour(float *su, const float *sf, const fl
     for (int it = 0; it < IT; ++it) {
         const int c = cv[it];
         if (c >= 0) {
-            float s;
-            su[c] = relax_value<float>(su[c], su[c + 1], su[c - 1], su[c + LX], su[c - LX], su[c + LX * LY],
-                                       su[c - LX * LY], fv[it], h2, &s);
+            T s;
+            su[c] = relax_value<T>(su[c], su[c + 1], su[c - 1], su[c + LX], su[c - LX], su[c + LX * LY],
+                                   su[c - LX * LY], fv[it], h2, &s);
             if (core & (1u << it)) amax = fmax(amax, fabs((double)s));
         }
     }
@@ -166,64 +114,50 @@ __device__ __forceinline__ void tile_colour(float *su, const float *sf, const fl
 
 // Sweeps S .. NS-1 of a multi-sweep tile: sweep s updates the first colour on margin 2s+1 and the
 // second on margin 2s+2.  Only the last sweep feeds the max|resh2| (one mg_relax call's Resmaxg).
-template <class TL, int LX, int LY, int LZ, int H, int S, int NS, bool FS> struct TileSweeps {
-    static __device__ __forceinline__ void run(float *su, const float *sf, const float *__restrict__ f, int n, int x0,
-                                               int y0, int z0, float h2, double &amax)
+template <class TL, int LX, int LY, int LZ, int H, int S, int NS, bool FS, typename T> struct TileSweeps {
+    static __device__ __forceinline__ void run(T *su, const T *sf, const T *__restrict__ f, int n, int x0,
+                                               int y0, int z0, T h2, double &amax)
     {
         double dummy = 0.0;
         double &acc = (S == NS - 1) ? amax : dummy;
-        tile_colour<TL, LX, LY, LZ, 2 * S + 1, H, FS>(su, sf, f, n, x0, y0, z0, 1, h2, acc);
+        tile_colour<TL, LX, LY, LZ, 2 * S + 1, H, FS, T>(su, sf, f, n, x0, y0, z0, 1, h2, acc);
         __syncthreads();
-        tile_colour<TL, LX, LY, LZ, 2 * S + 2, H, FS>(su, sf, f, n, x0, y0, z0, 0, h2, acc);
+        tile_colour<TL, LX, LY, LZ, 2 * S + 2, H, FS, T>(su, sf, f, n, x0, y0, z0, 0, h2, acc);
         __syncthreads();
-        TileSweeps<TL, LX, LY, LZ, H, S + 1, NS, FS>::run(su, sf, f, n, x0, y0, z0, h2, amax);
+        TileSweeps<TL, LX, LY, LZ, H, S + 1, NS, FS, T>::run(su, sf, f, n, x0, y0, z0, h2, amax);
     }
 };
-template <class TL, int LX, int LY, int LZ, int H, int NS, bool FS> struct TileSweeps<TL, LX, LY, LZ, H, NS, NS, FS> {
-    static __device__ __forceinline__ void run(float *, const float *, const float *__restrict__, int, int, int, int,
-                                               float, double &)
+template <class TL, int LX, int LY, int LZ, int H, int NS, bool FS, typename T>
+struct TileSweeps<TL, LX, LY, LZ, H, NS, NS, FS, T> {
+    static __device__ __forceinline__ void run(T *, const T *, const T *__restrict__, int, int, int, int, T, double &)
     {
     }
 };
 
 // LDS bytes of the largest variant of a (tile, sweeps, staging) choice: the residual variant has
 // the widest halo, the prolongation variant adds the staged coarse tile.
-template <class TL, int NS, bool FS> constexpr int sweep_lds_bytes()
+template <class TL, int NS, bool FS, typename T = float> constexpr int sweep_lds_bytes()
 {
     constexpr int H1 = 2 * NS + 1, H2 = 2 * NS;
     constexpr int r1 = (TL::TX + 2 * H1) * (TL::TY + 2 * H1) * (TL::TZ + 2 * H1) * (FS ? 2 : 1);
     constexpr int r2 = (TL::TX + 2 * H2) * (TL::TY + 2 * H2) * (TL::TZ + 2 * H2) * (FS ? 2 : 1) +
                        ((TL::TX + 2 * H2) / 2 + 2) * ((TL::TY + 2 * H2) / 2 + 2) * ((TL::TZ + 2 * H2) / 2 + 2);
-    return 4 * (r1 > r2 ? r1 : r2) + 1024;
+    return (int)sizeof(T) * (r1 > r2 ? r1 : r2) + 1024;
 }
-template <class TL, int NS, bool FS> constexpr bool sweep_fits_lds() { return sweep_lds_bytes<TL, NS, FS>() <= 163840; }
-
-template <class TL> inline bool fits_lds(int ns, bool fs)
+template <class TL, int NS, bool FS, typename T = float> constexpr bool sweep_fits_lds()
 {
-    if (ns == 2) return fs ? sweep_fits_lds<TL, 2, true>() : sweep_fits_lds<TL, 2, false>();
-    return fs ? sweep_fits_lds<TL, 1, true>() : sweep_fits_lds<TL, 1, false>();
+    return sweep_lds_bytes<TL, NS, FS, T>() <= 163840;
 }
 
-// whether (tile shape, sweeps per launch, staging) is instantiated (fits the 160 KB of LDS)
-inline bool cand_ok(int cfg, int ns, bool fs)
-{
-    switch (cfg) {
-    case 0: return fits_lds<Tile0>(ns, fs);
-    case 1: return fits_lds<Tile1>(ns, fs);
-    case 2: return fits_lds<Tile2>(ns, fs);
-    case 3: return fits_lds<Tile3>(ns, fs);
-    default: return fits_lds<Tile4>(ns, fs);
-    }
-}
 
 // NS full sweeps (temporal blocking: halo 2 per sweep, +1 for the residual).  FS stages the source
 // on the same LDS region as u, loaded together with u, so the colour passes touch LDS only.
 // Body of the fused sweep for tile t of an n^3 level (n even, divisible by the tile extents);
 // called by every thread of a workgroup with the same t.
-template <class TL, int NS, bool ZERO, bool PROLONG, bool RESID, bool FS>
-__device__ __forceinline__ void sweep_tile(const float *__restrict__ uin, float *__restrict__ uout,
-                                           const float *__restrict__ f, int n, float h2, float h2i,
-                                           const float *__restrict__ uc, float *__restrict__ rc, double *resmax, int t)
+template <class TL, int NS, bool ZERO, bool PROLONG, bool RESID, bool FS, typename T = float>
+__device__ __forceinline__ void sweep_tile(const T *__restrict__ uin, T *__restrict__ uout,
+                                           const T *__restrict__ f, int n, T h2, T h2i,
+                                           const T *__restrict__ uc, T *__restrict__ rc, double *resmax, int t)
 {
     constexpr int H = 2 * NS + (RESID ? 1 : 0);
     constexpr int TX = TL::TX, TY = TL::TY, TZ = TL::TZ, NT = TL::NT;
@@ -231,9 +165,9 @@ __device__ __forceinline__ void sweep_tile(const float *__restrict__ uin, float 
     constexpr int CX = LX / 2 + 2, CY = LY / 2 + 2, CZ = LZ / 2 + 2;  // staged coarse region
     static_assert(!RESID || H >= 3, "residual needs a 3-cell halo");
     static_assert(H % 2 == 0 || !PROLONG, "prolongation staging assumes an even tile origin");
-    __shared__ float su[LX * LY * LZ];
-    __shared__ float sf[FS ? LX * LY * LZ : 1];
-    __shared__ float sc[PROLONG ? CX * CY * CZ : 1];
+    __shared__ T su[LX * LY * LZ];
+    __shared__ T sf[FS ? LX * LY * LZ : 1];
+    __shared__ T sc[PROLONG ? CX * CY * CZ : 1];
     const int ntx = n / TX, nty = n / TY;
     const int tx = t % ntx, ty = (t / ntx) % nty, tz = t / (ntx * nty);
     const int x0 = tx * TX - H, y0 = ty * TY - H, z0 = tz * TZ - H;
@@ -244,9 +178,9 @@ __device__ __forceinline__ void sweep_tile(const float *__restrict__ uin, float 
         // cells x0/2 - 1 .. x0/2 + LX/2 (x0 even) that the trilinear correction reads
         constexpr int CNT = LX * LY * LZ, IT = (CNT + NT - 1) / NT;
         constexpr int CNTC = CX * CY * CZ, ITC = PROLONG ? (CNTC + NT - 1) / NT : 1;
-        float v[IT];
-        float fvl[FS ? IT : 1];
-        float cvl[ITC];
+        T v[IT];
+        T fvl[FS ? IT : 1];
+        T cvl[ITC];
         if (!ZERO || FS) {
 #pragma unroll
             for (int it = 0; it < IT; ++it) {
@@ -279,7 +213,7 @@ __device__ __forceinline__ void sweep_tile(const float *__restrict__ uin, float 
         for (int it = 0; it < IT; ++it) {
             const int q = threadIdx.x + it * NT;
             if (CNT % NT == 0 || q < CNT) {
-                su[q] = ZERO ? 0.0f : v[it];
+                su[q] = ZERO ? T(0) : v[it];
                 if (FS) sf[q] = fvl[FS ? it : 0];
             }
         }
@@ -297,7 +231,7 @@ __device__ __forceinline__ void sweep_tile(const float *__restrict__ uin, float 
                 const int ic = (x >> 1) + 1, jc = (y >> 1) + 1, kc = (z >> 1) + 1;
                 const int ic1 = ic + 2 * (x & 1) - 1, jc1 = jc + 2 * (y & 1) - 1, kc1 = kc + 2 * (z & 1) - 1;
                 auto C = [&](int a, int b, int d) { return sc[(d * CY + b) * CX + a]; };
-                su[q] = su[q] + trilinear_value<float>(C(ic, jc, kc), C(ic1, jc, kc), C(ic, jc1, kc), C(ic, jc, kc1),
+                su[q] = su[q] + trilinear_value<T>(C(ic, jc, kc), C(ic1, jc, kc), C(ic, jc1, kc), C(ic, jc, kc1),
                                                        C(ic, jc1, kc1), C(ic1, jc, kc1), C(ic1, jc1, kc),
                                                        C(ic1, jc1, kc1));
             }
@@ -305,7 +239,7 @@ __device__ __forceinline__ void sweep_tile(const float *__restrict__ uin, float 
         __syncthreads();
     }
     double amax = 0.0;
-    TileSweeps<TL, LX, LY, LZ, H, 0, NS, FS>::run(su, sf, f, n, x0, y0, z0, h2, amax);
+    TileSweeps<TL, LX, LY, LZ, H, 0, NS, FS, T>::run(su, sf, f, n, x0, y0, z0, h2, amax);
     {
         constexpr int CNT = TX * TY * TZ, IT = (CNT + NT - 1) / NT;
 #pragma unroll
@@ -322,7 +256,7 @@ __device__ __forceinline__ void sweep_tile(const float *__restrict__ uin, float 
         // residual of the 8 fine cells of each coarse cell of the tile, restricted
         constexpr int QX = TX / 2, QY = TY / 2, QZ = TZ / 2;
         constexpr int CNT = QX * QY * QZ, IT = (CNT + NT - 1) / NT;
-        float fv[IT][8];
+        T fv[IT][8];
 #pragma unroll
         for (int it = 0; it < IT; ++it) {
             const int q = threadIdx.x + it * NT;
@@ -345,33 +279,33 @@ __device__ __forceinline__ void sweep_tile(const float *__restrict__ uin, float 
             const int q = threadIdx.x + it * NT;
             if (CNT % NT == 0 || q < CNT) {
                 const int cx = q % QX, cy = (q / QX) % QY, cz = q / (QX * QY);
-                float r[8];
+                T r[8];
 #pragma unroll
                 for (int o = 0; o < 8; ++o) {
                     const int a = o & 1, b = (o >> 1) & 1, d = (o >> 2) & 1;
                     const int c = ((H + 2 * cz + d) * LY + (H + 2 * cy + b)) * LX + (H + 2 * cx + a);
-                    r[o] = resid_value<float>(su[c], su[c + 1], su[c - 1], su[c + LX], su[c - LX], su[c + LX * LY],
+                    r[o] = resid_value<T>(su[c], su[c + 1], su[c - 1], su[c + LX], su[c - LX], su[c + LX * LY],
                                               su[c - LX * LY], fv[it][o], h2i);
                 }
                 // restriction.F90:140-143 order: 000 100 010 001 110 101 011 111
                 const int gci = tx * QX + cx, gcj = ty * QY + cy, gck = tz * QZ + cz;
                 rc[(gck * nc + gcj) * nc + gci] =
-                    restrict_value<float>(r[0], r[1], r[2], r[4], r[3], r[5], r[6], r[7]);
+                    restrict_value<T>(r[0], r[1], r[2], r[4], r[3], r[5], r[6], r[7]);
             }
         }
     }
     if (resmax) block_atomic_max(resmax, amax);
 }
 
-template <class TL, int NS, bool ZERO, bool PROLONG, bool RESID, bool FS>
+template <class TL, int NS, bool ZERO, bool PROLONG, bool RESID, bool FS, typename T = float>
 __global__ void __launch_bounds__(TL::NT)
-k_sweep_tile(const float *__restrict__ uin, float *__restrict__ uout, const float *__restrict__ f, int n, float h2,
-             float h2i, const float *__restrict__ uc, float *__restrict__ rc, double *resmax)
+k_sweep_tile(const T *__restrict__ uin, T *__restrict__ uout, const T *__restrict__ f, int n, T h2,
+             T h2i, const T *__restrict__ uc, T *__restrict__ rc, double *resmax)
 {
     const int ntiles = (n / TL::TX) * (n / TL::TY) * (n / TL::TZ);
     const int t = xcd_tile(ntiles);
     if (t >= ntiles) return;  // uniform per workgroup, before any barrier
-    sweep_tile<TL, NS, ZERO, PROLONG, RESID, FS>(uin, uout, f, n, h2, h2i, uc, rc, resmax, t);
+    sweep_tile<TL, NS, ZERO, PROLONG, RESID, FS, T>(uin, uout, f, n, h2, h2i, uc, rc, resmax, t);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -399,7 +333,7 @@ template <int SX_, int SY_, int ZC_, int NT_> struct StreamShape {
     static constexpr int SX = SX_, SY = SY_, ZC = ZC_, NT = NT_;
 };
 
-template <class SS, bool PROLONG, bool RESID> struct StreamGeom {
+template <class SS, bool PROLONG, bool RESID, typename T = float> struct StreamGeom {
     static constexpr int H = RESID ? 3 : 2;
     static constexpr int PX = SS::SX + 2 * H, PY = SS::SY + 2 * H, PP = PX * PY;
     static constexpr int R = RESID ? 6 : 5;                    // ring slots
@@ -410,13 +344,13 @@ template <class SS, bool PROLONG, bool RESID> struct StreamGeom {
     static constexpr int IS = (SS::SX * SS::SY + SS::NT - 1) / SS::NT;  // core cells per thread
     static constexpr int RX1 = (PX - 2) / 2, RY1 = PY - 2, C1 = RX1 * RY1, I1 = (C1 + SS::NT - 1) / SS::NT;
     static constexpr int RX2 = (PX - 4) / 2, RY2 = PY - 4, C2 = RX2 * RY2, I2 = (C2 + SS::NT - 1) / SS::NT;
-    static constexpr int lds_bytes = 4 * (2 * R * PP + (PROLONG ? CR * CP : 0) + (RESID ? SS::SX * SS::SY : 0));
+    static constexpr int lds_bytes = (int)sizeof(T) * (2 * R * PP + (PROLONG ? CR * CP : 0) + (RESID ? SS::SX * SS::SY : 0));
     static_assert(IL <= 32 && I1 <= 32 && I2 <= 32 && IS <= 32, "per-thread bit masks hold 32 cells");
 };
 
-template <class SS, bool PROLONG, bool RESID> constexpr bool stream_fits_lds()
+template <class SS, bool PROLONG, bool RESID, typename T = float> constexpr bool stream_fits_lds()
 {
-    return StreamGeom<SS, PROLONG, RESID>::lds_bytes + 1024 <= 163840;
+    return StreamGeom<SS, PROLONG, RESID, T>::lds_bytes + 1024 <= 163840;
 }
 
 __device__ __forceinline__ int pmod(int a, int m) { const int r = a % m; return r < 0 ? r + m : r; }
@@ -446,27 +380,27 @@ __device__ __forceinline__ void pass_cells(PassCells<N> &P, int tid)
     }
 }
 
-template <class SS, bool ZERO, bool PROLONG, bool RESID>
-__device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, float *__restrict__ uout,
-                                             const float *__restrict__ f, int n, float h2, float h2i,
-                                             const float *__restrict__ uc, float *__restrict__ rc, double *resmax, int t)
+template <class SS, bool ZERO, bool PROLONG, bool RESID, typename T = float>
+__device__ __forceinline__ void sweep_stream(const T *__restrict__ uin, T *__restrict__ uout,
+                                             const T *__restrict__ f, int n, T h2, T h2i,
+                                             const T *__restrict__ uc, T *__restrict__ rc, double *resmax, int t)
 {
-    using G = StreamGeom<SS, PROLONG, RESID>;
+    using G = StreamGeom<SS, PROLONG, RESID, T>;
     constexpr int SX = SS::SX, SY = SS::SY, ZC = SS::ZC, NT = SS::NT;
-    constexpr int H = G::H, PX = G::PX, PY = G::PY, PP = G::PP, R = G::R, CX = G::CX, CP = G::CP, CR = G::CR;
+    constexpr int H = G::H, PX = G::PX, PP = G::PP, R = G::R, CX = G::CX, CP = G::CP, CR = G::CR;
     static_assert(SX % 2 == 0 && SY % 2 == 0 && ZC % 2 == 0, "stream shape");
     static_assert(!PROLONG || H % 2 == 0, "the coarse-value window starts on an even fine plane");
-    __shared__ float su[R * PP];
-    __shared__ float sf[R * PP];
-    __shared__ float scz[PROLONG ? CR * CP : 1];
-    __shared__ float srp[RESID ? SX * SY : 1];
+    __shared__ T su[R * PP];
+    __shared__ T sf[R * PP];
+    __shared__ T scz[PROLONG ? CR * CP : 1];
+    __shared__ T srp[RESID ? SX * SY : 1];
     const int ntx = n / SX, nty = n / SY;
     const int tx = t % ntx, ty = (t / ntx) % nty, tz = t / (ntx * nty);
     const int x0 = tx * SX, y0 = ty * SY, z0 = tz * ZC;
     const int nc = n >> 1;
     const int tid = threadIdx.x;
     const bool want = resmax != nullptr;
-    float amax = 0.f;
+    T amax = T(0);
 
     // ---- per-thread geometry, fixed for the whole march ----
     int goff[G::IL];         // global (y, x) offset of ring cell tid + it NT
@@ -507,13 +441,13 @@ __device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, floa
         sl[it] = (y + H) * PX + x + H;
     }
 
-    float ru[G::IL], rf[G::IL], rcz[PROLONG ? G::ICL : 1];
+    T ru[G::IL], rf[G::IL], rcz[PROLONG ? G::ICL : 1];
     auto fetch = [&](int k) {
         const int base = wrapn(k, n) * n * n;
 #pragma unroll
         for (int it = 0; it < G::IL; ++it) {
             if (PP % NT == 0 || tid + it * NT < PP) {
-                ru[it] = ZERO ? 0.0f : uin[base + goff[it]];
+                ru[it] = ZERO ? T(0) : uin[base + goff[it]];
                 rf[it] = f[base + goff[it]];
             }
         }
@@ -525,7 +459,7 @@ __device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, floa
             if (CP % NT == 0 || tid + it * NT < CP) rcz[PROLONG ? it : 0] = uc[base + cgoff[PROLONG ? it : 0]];
     };
     auto put_coarse = [&](int c) {
-        float *dst = scz + (c & (CR - 1)) * CP;
+        T *dst = scz + (c & (CR - 1)) * CP;
 #pragma unroll
         for (int it = 0; it < G::ICL; ++it)
             if (CP % NT == 0 || tid + it * NT < CP) dst[tid + it * NT] = rcz[PROLONG ? it : 0];
@@ -534,9 +468,9 @@ __device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, floa
     // planes a put reads, held in registers: win[0] plane m, win[1] plane m + 1 for the fine
     // planes 2m + 1 and 2m + 2, so each coarse plane is read from LDS once per thread, not 4 times
     constexpr int WI = PROLONG ? G::IL : 1;
-    float win[2][WI][4];
+    T win[2][WI][4];
     auto win_load = [&](int w, int c) {
-        const float *src = scz + (c & (CR - 1)) * CP;
+        const T *src = scz + (c & (CR - 1)) * CP;
 #pragma unroll
         for (int it = 0; it < WI; ++it)
             if (PP % NT == 0 || tid + it * NT < PP)
@@ -546,7 +480,7 @@ __device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, floa
     // the fetched plane k into ring slot `slot` (adding the trilinear correction with PROLONG:
     // coarse planes kc = floor(k / 2) and kc1 = kc - 1 (k even) or kc + 1 (k odd))
     auto put = [&](int k, int slot) {
-        float *du = su + slot * PP, *df = sf + slot * PP;
+        T *du = su + slot * PP, *df = sf + slot * PP;
         const bool odd = (k & 1) != 0;
         if (PROLONG && odd) {
 #pragma unroll
@@ -559,16 +493,16 @@ __device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, floa
         for (int it = 0; it < G::IL; ++it) {
             const int q = tid + it * NT;
             if (PP % NT == 0 || q < PP) {
-                float v = ru[it];
+                T v = ru[it];
                 if (PROLONG) {
                     const int w = PROLONG ? it : 0;
-                    float a[4], b[4];  // plane kc, plane kc1
+                    T a[4], b[4];  // plane kc, plane kc1
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         a[e] = odd ? win[0][w][e] : win[1][w][e];
                         b[e] = odd ? win[1][w][e] : win[0][w][e];
                     }
-                    v = v + trilinear_value<float>(a[0], a[1], a[2], b[0], b[2], b[1], a[3], b[3]);
+                    v = v + trilinear_value<T>(a[0], a[1], a[2], b[0], b[2], b[1], a[3], b[3]);
                 }
                 du[q] = v;
                 df[q] = rf[it];
@@ -576,7 +510,7 @@ __device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, floa
         }
     };
     // one colour pass over the cells P on plane k: u (slot of k), um / up (k - 1 / k + 1), fk
-    auto colour = [&](auto &P, int k, float *u, const float *um, const float *up, const float *fk, bool out) {
+    auto colour = [&](auto &P, int k, T *u, const T *um, const T *up, const T *fk, bool out) {
         constexpr int N = sizeof(P.cb) / sizeof(int);
         const unsigned kb = (unsigned)(k & 1);
 #pragma unroll
@@ -584,16 +518,16 @@ __device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, floa
             if (((P.valid >> i) & 1u) == 0u) continue;
             const unsigned d = ((P.yb >> i) & 1u) ^ kb;
             const int c = P.cb[i] + (int)d;
-            float s;
-            u[c] = relax_value<float>(u[c], u[c + 1], u[c - 1], u[c + PX], u[c - PX], up[c], um[c], fk[c], h2, &s);
-            if (want && out && ((((d ? P.core1 : P.core0) >> i) & 1u) != 0u)) amax = fmaxf(amax, fabsf(s));
+            T s;
+            u[c] = relax_value<T>(u[c], u[c + 1], u[c - 1], u[c + PX], u[c - PX], up[c], um[c], fk[c], h2, &s);
+            if (want && out && ((((d ? P.core1 : P.core0) >> i) & 1u) != 0u)) amax = fmax(amax, fabs(s));
         }
     };
     auto resid_at = [&](int slot, int slotm, int slotp, int x, int y) {
-        const float *u = su + slot * PP, *um = su + slotm * PP, *up = su + slotp * PP;
-        const float *fk = sf + slot * PP;
+        const T *u = su + slot * PP, *um = su + slotm * PP, *up = su + slotp * PP;
+        const T *fk = sf + slot * PP;
         const int c = (y + H) * PX + x + H;
-        return resid_value<float>(u[c], u[c + 1], u[c - 1], u[c + PX], u[c - PX], up[c], um[c], fk[c], h2i);
+        return resid_value<T>(u[c], u[c + 1], u[c - 1], u[c + PX], u[c - PX], up[c], um[c], fk[c], h2i);
     };
 
     const int zlo = z0 - H, zhi = z0 + ZC + H - 1;  // planes held at some point
@@ -654,7 +588,7 @@ __device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, floa
             __syncthreads();
             // 3. store plane pa - 1; residual of plane pa - 2
             if (pa - 1 >= z0 && pa - 1 < z0 + ZC) {
-                const float *u = su + S(-1) * PP;
+                const T *u = su + S(-1) * PP;
                 const int gz = wrapn(pa - 1, n) * n * n;
 #pragma unroll
                 for (int it = 0; it < G::IS; ++it)
@@ -674,17 +608,17 @@ __device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, floa
                         for (int q = tid; q < SX * SY / 2; q += NT) {
                             const int b = q & 1, cx = (q >> 1) % (SX / 2), cy = (q >> 1) / (SX / 2);
                             const int y = 2 * cy + b;
-                            const float e0 = srp[y * SX + 2 * cx], e1 = srp[y * SX + 2 * cx + 1];
-                            const float o0 = resid_at(S(-2), S(-3), S(-1), 2 * cx, y);
-                            const float o1 = resid_at(S(-2), S(-3), S(-1), 2 * cx + 1, y);
-                            const float pe0 = __shfl_xor(e0, 1), pe1 = __shfl_xor(e1, 1);
-                            const float po0 = __shfl_xor(o0, 1), po1 = __shfl_xor(o1, 1);
+                            const T e0 = srp[y * SX + 2 * cx], e1 = srp[y * SX + 2 * cx + 1];
+                            const T o0 = resid_at(S(-2), S(-3), S(-1), 2 * cx, y);
+                            const T o1 = resid_at(S(-2), S(-3), S(-1), 2 * cx + 1, y);
+                            const T pe0 = __shfl_xor(e0, 1), pe1 = __shfl_xor(e1, 1);
+                            const T po0 = __shfl_xor(o0, 1), po1 = __shfl_xor(o1, 1);
                             if (b == 0) {
                                 // r[a + 2 b + 4 dz]: own row is b = 0, the partner's b = 1
-                                const float r[8] = {e0, e1, pe0, pe1, o0, o1, po0, po1};
+                                const T r[8] = {e0, e1, pe0, pe1, o0, o1, po0, po1};
                                 const int gcx = x0 / 2 + cx, gcy = y0 / 2 + cy, gcz = wrapn(kq, n) / 2;
                                 rc[(gcz * nc + gcy) * nc + gcx] =
-                                    restrict_value<float>(r[0], r[1], r[2], r[4], r[3], r[5], r[6], r[7]);
+                                    restrict_value<T>(r[0], r[1], r[2], r[4], r[3], r[5], r[6], r[7]);
                             }
                         }
                     }
@@ -695,15 +629,15 @@ __device__ __forceinline__ void sweep_stream(const float *__restrict__ uin, floa
     if (want) block_atomic_max(resmax, (double)amax);
 }
 
-template <class SS, bool ZERO, bool PROLONG, bool RESID>
+template <class SS, bool ZERO, bool PROLONG, bool RESID, typename T = float>
 __global__ void __launch_bounds__(SS::NT)
-k_sweep_stream(const float *__restrict__ uin, float *__restrict__ uout, const float *__restrict__ f, int n, float h2,
-               float h2i, const float *__restrict__ uc, float *__restrict__ rc, double *resmax)
+k_sweep_stream(const T *__restrict__ uin, T *__restrict__ uout, const T *__restrict__ f, int n, T h2,
+               T h2i, const T *__restrict__ uc, T *__restrict__ rc, double *resmax)
 {
     const int ntiles = (n / SS::SX) * (n / SS::SY) * (n / SS::ZC);
     const int t = xcd_tile(ntiles);
     if (t >= ntiles) return;
-    sweep_stream<SS, ZERO, PROLONG, RESID>(uin, uout, f, n, h2, h2i, uc, rc, resmax, t);
+    sweep_stream<SS, ZERO, PROLONG, RESID, T>(uin, uout, f, n, h2, h2i, uc, rc, resmax, t);
 }
 
 // Streaming shapes the autotuners choose from beside the tiles (one sweep per launch, source always
@@ -736,12 +670,86 @@ inline bool cfg_fits(int cfg, int n)
     return n >= d[0] && n >= d[1] && n >= d[2] && n % d[0] == 0 && n % d[1] == 0 && n % d[2] == 0;
 }
 
+
+// Whether a sweep kernel is instantiated for T: FP32 (autotuned), every shape that fits the LDS; FP64,
+// the shapes of fp64_sweep_shape.
+template <class TL, int NS, bool FS, typename T> constexpr bool sweep_built()
+{
+    if (sizeof(T) == sizeof(float)) return sweep_fits_lds<TL, NS, FS, T>();
+    return !FS && ((TL::NT == 1024 && NS == 1) || (TL::TX == 16 && TL::NT == 1024) || (TL::TX == 16 && NS == 1) || TL::TX == 8);
+}
+template <class SS, typename T> constexpr bool stream_built()
+{
+    if (sizeof(T) == sizeof(float)) return stream_fits_lds<SS, true, false, T>() && stream_fits_lds<SS, false, true, T>();
+    return SS::ZC == 32 && SS::NT == 512 && (SS::SX == 64 ? SS::SY == 16 : SS::SX == 32);
+}
+template <class TL, int NS, bool FS, typename T> constexpr bool sweep_built_fits()
+{
+    return !sweep_built<TL, NS, FS, T>() || sweep_fits_lds<TL, NS, FS, T>();
+}
+static_assert(sweep_built_fits<Tile0, 1, false, double>() && sweep_built_fits<Tile1, 2, false, double>() &&
+                  sweep_built_fits<Tile2, 1, false, double>() && sweep_built_fits<Tile4, 2, false, double>() &&
+                  stream_fits_lds<Stream0, true, false, double>() && stream_fits_lds<Stream0, false, true, double>() &&
+                  stream_fits_lds<Stream7, true, false, double>() && stream_fits_lds<Stream7, false, true, double>(),
+              "FP64 sweep shapes exceed the LDS");
+
+// The FP64 sweep shape of a launch over levels whose widths are all multiples of `unit` (64, 32, 16 or
+// 8) with `cells` cells in all: the largest shape that still makes 256 workgroups, one per CU, since a
+// workgroup's halo costs less the larger its tile; below that the levels are bound by latency, and two
+// sweeps per launch halve the launches (two_sweeps: the caller's choice for all launches of the level,
+// fp64_two_sweeps).  One V(2,2) visit of one grid, us: 512^3 stream 64 x 16 z32 3358, 32 x 32 z32
+// 3605, tile 32 x 16 x 16 4383; 256^3 426, 448, 522; 128^3 tile 32 x 16 x 16 64, stream 78, tile
+// 16 x 8 x 8 76; 64^3 tile 16 x 8 x 8 with two sweeps 20.3, with one 21.0, tile 8^3 22.1; 32^3 tile 8^3
+// with two sweeps 14.6, with one 16.4, tile 16 x 8 x 8 18.1.
+constexpr long kSweepCUs = 256;
+inline bool fp64_two_sweeps(long cells) { return cells < kSweepCUs * 32 * 16 * 16; }
+inline int fp64_sweep_shape(int unit, long cells, bool two_sweeps)
+{
+    if (!two_sweeps) {
+        if (unit >= 64 && cells >= kSweepCUs * 64 * 16 * 32) return kNumTiles + 0;
+        if (unit >= 32 && cells >= kSweepCUs * 32 * 32 * 32) return kNumTiles + 7;
+        if (unit >= 32) return 0;
+        return unit >= 16 ? 2 : 4;
+    }
+    return unit >= 16 && cells >= kSweepCUs * 16 * 8 * 8 ? 1 : 4;
+}
+
+template <class TL, typename T> inline bool built(int ns, bool fs)
+{
+    if (ns == 2) return fs ? sweep_built<TL, 2, true, T>() : sweep_built<TL, 2, false, T>();
+    return fs ? sweep_built<TL, 1, true, T>() : sweep_built<TL, 1, false, T>();
+}
+
+// whether (tile shape, sweeps per launch, staging) is instantiated
+template <typename T> inline bool cand_ok(int cfg, int ns, bool fs)
+{
+    switch (cfg) {
+    case 0: return built<Tile0, T>(ns, fs);
+    case 1: return built<Tile1, T>(ns, fs);
+    case 2: return built<Tile2, T>(ns, fs);
+    case 3: return built<Tile3, T>(ns, fs);
+    default: return built<Tile4, T>(ns, fs);
+    }
+}
+
 // whether configuration cfg with (ns, fs) exists: streams take one sweep per launch and always
 // stage the source (reported as fs = 0)
-inline bool cfg_ok(int cfg, int ns, bool fs)
+template <typename T> inline bool cfg_ok(int cfg, int ns, bool fs)
 {
-    if (cfg < kNumTiles) return cand_ok(cfg, ns, fs);
-    return cfg < kNumCfg && ns == 1 && !fs;
+    if (cfg < kNumTiles) return cand_ok<T>(cfg, ns, fs);
+    if (ns != 1 || fs) return false;
+    switch (cfg - kNumTiles) {
+    case 0: return stream_built<Stream0, T>();
+    case 1: return stream_built<Stream1, T>();
+    case 2: return stream_built<Stream2, T>();
+    case 3: return stream_built<Stream3, T>();
+    case 4: return stream_built<Stream4, T>();
+    case 5: return stream_built<Stream5, T>();
+    case 6: return stream_built<Stream6, T>();
+    case 7: return stream_built<Stream7, T>();
+    case 8: return stream_built<Stream8, T>();
+    default: return false;
+    }
 }
 
 // autotuner candidate index -> (cfg, ns, fs)
@@ -847,18 +855,22 @@ __global__ void __launch_bounds__(NT) k_interp_cubic_tile(T *__restrict__ uf, co
 }
 
 // ------------------------------------------------------------------------------------------------
-// Single-workgroup solver for the levels of <= 16^3 cells, all resident in LDS.
+// Single-workgroup solvers of the first level of <= 16^3 cells: the reference's cycles from there down
+// (coarse_levels.h), or its exact solve.
 // ------------------------------------------------------------------------------------------------
-struct CoarseLevels {
-    int nlev;               // levels held: 0 .. nlev-1 (local numbering), n_0 <= 16
-    int n[8], lg[8];        // cells per side and its log2
-    float h2[8], h2i[8];
-    int off[8];             // offset of level l inside each LDS array
-    int exact;              // 1: held level 0 solved exactly instead (coarse_exact)
-    float Q[kCoarseMaxN * kCoarseMaxN], lam[kCoarseMaxN];  // its Hartley basis and eigenvalues
-};
+template <typename T, int N>
+__global__ void __launch_bounds__(kCoarseThreads)
+k_coarse(const T *__restrict__ rhs_in, T *__restrict__ u_out, CoarseCoef<T> P, int mode, int ncycle, int npre, int npost,
+         double *resmax)
+{
+    __shared__ CoarseLds<T> S;
+    coarse_solve<T, N>(S, P, rhs_in, u_out, mode, ncycle, npre, npost, resmax);
+}
 
-constexpr int kCoarseCells = 16 * 16 * 16 + 8 * 8 * 8 + 4 * 4 * 4 + 2 * 2 * 2 + 1;
+struct CoarseExact {
+    int n;                                                 // cells per side, <= 16
+    float Q[kCoarseMaxN * kCoarseMaxN], lam[kCoarseMaxN];  // Hartley basis and eigenvalues
+};
 
 // Hartley basis of the periodic 3-point second difference on n cells, Q[m n + k] =
 // (cos a + sin a) / sqrt(n) with a = 2 pi ((m k) mod n) / n, and its eigenvalues
@@ -962,139 +974,11 @@ __device__ inline void coarse_exact(float *g, float *s, const float *Qg, const f
     }
 }
 
-__device__ __forceinline__ void c_relax(float *U, const float *R, int n, int lg, float h2, double *resmax)
-{
-    double amax = 0.0;
-    const int lgh = lg > 0 ? lg - 1 : 0;  // log2 of cells per colour row (n >= 2), 1 for n == 1
-    const int m = n - 1;
-    for (int ipass = 1; ipass <= 2; ++ipass) {
-        for (int t = threadIdx.x; t < (n * n * n + 1) / 2; t += kCoarseThreads) {
-            const int ih = t & ((1 << lgh) - 1), j = (t >> lgh) & m, k = t >> (lgh + lg);
-            const int i = (n == 1) ? 0 : 2 * ih + ((j + k + ipass) & 1);
-            if (n == 1 && ipass == 1) continue;   // single cell has colour "even" (ipass 2)
-            const int c = (k * n + j) * n + i, row = (k * n + j) * n;
-            float s;
-            U[c] = relax_value<float>(U[c], U[row + ((i + 1) & m)], U[row + ((i - 1) & m)],
-                                      U[(k * n + ((j + 1) & m)) * n + i], U[(k * n + ((j - 1) & m)) * n + i],
-                                      U[(((k + 1) & m) * n + j) * n + i], U[(((k - 1) & m) * n + j) * n + i], R[c],
-                                      h2, &s);
-            amax = fmax(amax, fabs((double)s));
-        }
-        __syncthreads();
-    }
-    if (resmax) block_atomic_max(resmax, amax);
-}
-
-// residual of level (n, U, R) restricted into Rc: each coarse cell evaluates its 8 fine residuals
-// (mg_poisson.F90:17-27 then restriction.F90:132-147, same values as the two separate passes).
-__device__ __forceinline__ void c_resid_restrict(const float *U, const float *R, int n, int lg, float h2i, float *Rc)
-{
-    const int nc = n >> 1, lgc = lg - 1, m = n - 1;
-    for (int q = threadIdx.x; q < nc * nc * nc; q += kCoarseThreads) {
-        const int cx = q & (nc - 1), cy = (q >> lgc) & (nc - 1), cz = q >> (2 * lgc);
-        float r[8];
-#pragma unroll
-        for (int o = 0; o < 8; ++o) {
-            const int i = 2 * cx + (o & 1), j = 2 * cy + ((o >> 1) & 1), k = 2 * cz + ((o >> 2) & 1);
-            const int c = (k * n + j) * n + i, row = (k * n + j) * n;
-            r[o] = resid_value<float>(U[c], U[row + ((i + 1) & m)], U[row + ((i - 1) & m)],
-                                      U[(k * n + ((j + 1) & m)) * n + i], U[(k * n + ((j - 1) & m)) * n + i],
-                                      U[(((k + 1) & m) * n + j) * n + i], U[(((k - 1) & m) * n + j) * n + i], R[c],
-                                      h2i);
-        }
-        Rc[q] = restrict_value<float>(r[0], r[1], r[2], r[4], r[3], r[5], r[6], r[7]);
-    }
-    __syncthreads();
-}
-
-__device__ __forceinline__ void c_restrict(float *Rc, const float *Rf, int nc, int lgc)
-{
-    const int nf = 2 * nc;
-    for (int q = threadIdx.x; q < nc * nc * nc; q += kCoarseThreads) {
-        const int i = 2 * (q & (nc - 1)), j = 2 * ((q >> lgc) & (nc - 1)), k = 2 * (q >> (2 * lgc));
-        auto F = [&](int a, int b, int d) { return Rf[((k + d) * nf + (j + b)) * nf + (i + a)]; };
-        Rc[q] = restrict_value<float>(F(0, 0, 0), F(1, 0, 0), F(0, 1, 0), F(0, 0, 1), F(1, 1, 0), F(1, 0, 1),
-                                      F(0, 1, 1), F(1, 1, 1));
-    }
-    __syncthreads();
-}
-
-__device__ __forceinline__ void c_fill0(float *U, int n)
-{
-    for (int c = threadIdx.x; c < n * n * n; c += kCoarseThreads) U[c] = 0.0f;
-    __syncthreads();
-}
-
-// mg_interp (mg.F90:608-633): cubic (FMG) unless the coarse grid plus ghosts is narrower than 4.
-__device__ __forceinline__ void c_interp(float *Uf, const float *Uc, int nf, int lgf, bool cubic, bool add)
-{
-    const int nc = nf >> 1;
-    auto C = [&](int a, int b, int d) { return Uc[(d * nc + b) * nc + a]; };
-    for (int c = threadIdx.x; c < nf * nf * nf; c += kCoarseThreads) {
-        const int i = c & (nf - 1), j = (c >> lgf) & (nf - 1), k = c >> (2 * lgf);
-        float v;
-        if (cubic && nc + 2 >= 4) v = tricubic_point<float>(C, i, j, k, nc);
-        else v = trilinear_point<float>(C, i, j, k, nc);
-        Uf[c] = add ? Uf[c] + v : v;
-    }
-    __syncthreads();
-}
-
-// mode 0: FMG over all held levels from RHO of local level 0 (mg.F90:142-215 restricted to them);
-// mode 1: one V-cycle from local level 0 with zero initial guess (mg.F90:179-210).
-// resmax receives max|resh2| of the final smoothing call when non-null (only meaningful when the
-// held level 0 is the finest level of the problem).  With L.exact both modes solve held level 0
-// exactly (coarse_exact).
 static __global__ void __launch_bounds__(kCoarseThreads)
-k_coarse(const float *__restrict__ rhs_in, float *__restrict__ u_out, CoarseLevels L, int mode, int ncycle,
-         int npre, int npost, double *resmax)
+k_coarse_exact(const float *__restrict__ rhs_in, float *__restrict__ u_out, CoarseExact E)
 {
-    __shared__ float sU[kCoarseCells], sR[kCoarseCells];
-    static_assert(kCoarseMaxN * kCoarseMaxN * (kCoarseMaxN + 1) <= kCoarseCells &&
-                      kCoarseMaxN * kCoarseMaxN + kCoarseMaxN <= kCoarseCells,
-                  "exact coarse solve exceeds the coarse kernel's LDS");
-    const int lmax = L.nlev - 1;
-    const int n0 = L.n[0];
-    if (L.exact) {
-        coarse_exact(sU, sR, L.Q, L.lam, rhs_in, u_out, n0);
-        return;
-    }
-    for (int c = threadIdx.x; c < n0 * n0 * n0; c += kCoarseThreads) sR[c] = rhs_in[c];
-    __syncthreads();
-    auto U = [&](int l) { return sU + L.off[l]; };
-    auto R = [&](int l) { return sR + L.off[l]; };
-    auto vcycle = [&](int ml, bool last_cycle) {
-        for (int v = ml; v <= lmax - 1; ++v) {
-            for (int p = 0; p < npre; ++p) c_relax(U(v), R(v), L.n[v], L.lg[v], L.h2[v], nullptr);
-            c_resid_restrict(U(v), R(v), L.n[v], L.lg[v], L.h2i[v], R(v + 1));
-            c_fill0(U(v + 1), L.n[v + 1]);
-        }
-        for (int it = 0; it < 2; ++it) c_relax(U(lmax), R(lmax), L.n[lmax], L.lg[lmax], L.h2[lmax], nullptr);
-        for (int v = lmax - 1; v >= ml; --v) {
-            c_interp(U(v), U(v + 1), L.n[v], L.lg[v], false, true);
-            for (int p = 0; p < npost; ++p) {
-                const bool last = last_cycle && v == 0 && p == npost - 1;
-                c_relax(U(v), R(v), L.n[v], L.lg[v], L.h2[v], last ? resmax : nullptr);
-            }
-        }
-    };
-    if (mode == 0) {
-        for (int l = 1; l <= lmax; ++l) c_restrict(R(l), R(l - 1), L.n[l], L.lg[l]);
-        c_fill0(U(lmax), L.n[lmax]);
-        for (int it = 0; it < 2; ++it) c_relax(U(lmax), R(lmax), L.n[lmax], L.lg[lmax], L.h2[lmax], nullptr);
-        for (int ml = lmax - 1; ml >= 0; --ml) {
-            c_interp(U(ml), U(ml + 1), L.n[ml], L.lg[ml], true, false);
-            for (int jc = 0; jc < ncycle; ++jc) vcycle(ml, ml == 0 && jc == ncycle - 1);
-        }
-    } else {
-        c_fill0(U(0), n0);
-        if (lmax == 0) {
-            for (int it = 0; it < 2; ++it) c_relax(U(0), R(0), n0, L.lg[0], L.h2[0], nullptr);
-        } else {
-            vcycle(0, false);
-        }
-    }
-    for (int c = threadIdx.x; c < n0 * n0 * n0; c += kCoarseThreads) u_out[c] = sU[c];
+    __shared__ float g[kCoarseMaxN * kCoarseMaxN * (kCoarseMaxN + 1)], q[kCoarseMaxN * kCoarseMaxN + kCoarseMaxN];
+    coarse_exact(g, q, E.Q, E.lam, rhs_in, u_out, E.n);
 }
 
 } // namespace sg

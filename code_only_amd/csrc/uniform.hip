@@ -3,12 +3,13 @@
 // declared in sg.h.
 //
 // Two inner solvers share the same kernels:
-//  * SG_PREC_FP64 ("plain"): every level array FP64, one launch per reference loop nest,
-//    launched eagerly.  Bitwise equal to the CPU FP64 restatement (same operand order, no FMA
-//    contraction).
+//  * SG_PREC_FP64 ("plain"): every level array FP64, the reference's cycle down to 1^3.  Bitwise equal
+//    to the CPU FP64 restatement (same operand order, no FMA contraction).
 //  * SG_PREC_MIXED: the inner mg_lin runs on FP32 level arrays; the outer residual
-//    r = f - L phi and the update phi += e stay FP64.  One outer iteration (inner solve, update,
-//    next outer residual and its norms) is captured once into a hipGraph and replayed.
+//    r = f - L phi and the update phi += e stay FP64.
+// Either runs the fused kernels with its inner solve captured once into a hipGraph and replayed (FP64,
+// 64^3: 1 732 launches of 1.4-2 us each, host-bound at 6.2 ms per solve, became 111 and 0.9 ms; 16^3:
+// 3.1 to 0.43 ms), or with fused = 0 one kernel per reference loop nest.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -47,6 +48,8 @@ template <typename T> struct Levels {
     T *U[kMaxLev] = {};
     T *RES[kMaxLev] = {};
     T *RHO[kMaxLev] = {};  // RHO[l] also serves as RHS[l]: see mg_lin below
+    T *U1[kMaxLev] = {};   // second U buffer: the fused sweeps ping-pong
+    void *mem = nullptr;   // the allocation that holds them all
 };
 
 static inline unsigned nblocks(long work) { return (unsigned)((work + kBlock - 1) / kBlock); }
@@ -69,13 +72,12 @@ struct sg_uniform {
     double hl[kMaxLev] = {};
     Levels<double> d;
     Levels<float> f;
-    float *U1[kMaxLev] = {};   // second FP32 U buffer per level: the fused sweeps ping-pong
-    int tile_cfg[kMaxLev] = {}; // autotuned sweep tile shape per fine level
+    int tile_cfg[kMaxLev] = {}; // FP32: autotuned sweep tile shape per fine level
     int tile_ns[kMaxLev] = {};  // autotuned sweeps per launch per fine level
     int tile_fs[kMaxLev] = {};  // autotuned: source staged in LDS
     float tune_ms[kMaxLev][32] = {};
-    CoarseLevels coarse;       // levels held by k_coarse, with the exact-solve basis of the first
-    int lc = 0;                // first level of <= 16^3 cells
+    int lc = 0;                // first level of <= 16^3 cells: held by k_coarse with all below it
+    CoarseExact cexact{};      // its exact solve (lc > 0)
     int lb = 0;                // bottom level of the exact-coarse cycle (lc, or a level of <= 64^3)
     float *d_qx = nullptr, *d_invx = nullptr;  // Hartley basis of level lb, 1 / Lambda (planes)
     double *psi_dev = nullptr, *src_dev = nullptr;   // staging for the host-pointer entry point
@@ -89,14 +91,13 @@ struct sg_uniform {
     double *hnorm_dev = nullptr;  // its device-side address (hipHostGetDevicePointer)
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr, evn = nullptr;
-    // graphs of one mixed-precision outer iteration (one per phi buffer parity), keyed on the
-    // arguments they were captured with
+    // graphs of the inner solve RHO[0] -> correction ([0] mixed, [1] FP64), keyed on the cycle shape
+    // they were captured with: they touch the context's own arrays only, so a call with other phi and
+    // source arrays replays the same graph (the outer step with the caller's arrays is launched after it)
     struct Graph {
         hipGraphExec_t exec = nullptr;
-        const double *pin = nullptr;
-        double *pout = nullptr;
-        const double *src = nullptr;
         int ncycle = -1, npre = -1, npost = -1, fused = -1, stop = -1, coarse = -1;
+        const void *u0 = nullptr;   // the buffer that holds the correction
     } graph[2];
 };
 
@@ -225,18 +226,18 @@ template <typename T> static int launch_interp(hipStream_t s, T *uf, const T *uc
 // end at level lb (the first level below level 0 with <= 64^3 cells, or with <= 16^3), solved
 // exactly (exact_bottom) where the reference sweeps its coarsest level (mg_slvsml,
 // mg.F90:540-546) -- the fused path's coarse-grid solve, so both paths keep the same values.
-static int exact_bottom(sg_uniform *c, int mode, int ncycle, int npre, int npost);
+static int exact_bottom(sg_uniform *c);
 
 template <typename T> static int mg_lin(sg_uniform *c, int ncycle, int npre, int npost, double *resmax,
                                         bool exact = false)
 {
     Levels<T> &A = levels<T>(c);
     hipStream_t s = c->stream;
-    exact = exact && std::is_same<T, float>::value && c->coarse.exact;
+    exact = exact && std::is_same<T, float>::value && c->lc > 0;
     const int lmax = exact ? c->lb : c->nlev - 1;
     auto bottom = [&]() -> int {
         if constexpr (std::is_same<T, float>::value) {
-            if (exact) return exact_bottom(c, 0, ncycle, npre, npost);
+            if (exact) return exact_bottom(c);
         }
         for (int it = 0; it < 2; ++it)
             SG_TRY(launch_relax<T>(s, A.U[lmax], A.RHO[lmax], c->nl[lmax], c->hl[lmax], nullptr));
@@ -268,85 +269,89 @@ template <typename T> static int mg_lin(sg_uniform *c, int ncycle, int npre, int
     return SG_OK;
 }
 
-template <class TL, int NS, bool FS>
-static void sweep_variant(hipStream_t s, const float *uin, float *uout, const float *f, int n, float h2, float h2i,
-                          bool zero, bool prolong, bool resid, const float *uc, float *rc, double *resmax)
+template <class TL, int NS, bool FS, typename T>
+static void sweep_variant(hipStream_t s, const T *uin, T *uout, const T *f, int n, T h2, T h2i,
+                          bool zero, bool prolong, bool resid, const T *uc, T *rc, double *resmax)
 {
     const int ntiles = (n / TL::TX) * (n / TL::TY) * (n / TL::TZ);
     const dim3 grid(8 * ((ntiles + 7) / 8)), block(TL::NT);
     if (resid && zero)
-        hipLaunchKernelGGL((k_sweep_tile<TL, NS, true, false, true, FS>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+        hipLaunchKernelGGL((k_sweep_tile<TL, NS, true, false, true, FS, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
     else if (resid)
-        hipLaunchKernelGGL((k_sweep_tile<TL, NS, false, false, true, FS>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+        hipLaunchKernelGGL((k_sweep_tile<TL, NS, false, false, true, FS, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
     else if (prolong)
-        hipLaunchKernelGGL((k_sweep_tile<TL, NS, false, true, false, FS>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+        hipLaunchKernelGGL((k_sweep_tile<TL, NS, false, true, false, FS, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
     else if (zero)
-        hipLaunchKernelGGL((k_sweep_tile<TL, NS, true, false, false, FS>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+        hipLaunchKernelGGL((k_sweep_tile<TL, NS, true, false, false, FS, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
     else
-        hipLaunchKernelGGL((k_sweep_tile<TL, NS, false, false, false, FS>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+        hipLaunchKernelGGL((k_sweep_tile<TL, NS, false, false, false, FS, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
 }
 
-template <class TL>
-static void sweep_ns(hipStream_t s, int ns, bool fs, const float *uin, float *uout, const float *f, int n, float h2,
-                     float h2i, bool zero, bool prolong, bool resid, const float *uc, float *rc, double *resmax)
+template <class TL, typename T>
+static void sweep_ns(hipStream_t s, int ns, bool fs, const T *uin, T *uout, const T *f, int n, T h2,
+                     T h2i, bool zero, bool prolong, bool resid, const T *uc, T *rc, double *resmax)
 {
     if (ns == 2 && fs) {
-        if constexpr (sweep_fits_lds<TL, 2, true>())
-            sweep_variant<TL, 2, true>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax);
+        if constexpr (sweep_built<TL, 2, true, T>())
+            sweep_variant<TL, 2, true, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax);
     } else if (ns == 2) {
-        if constexpr (sweep_fits_lds<TL, 2, false>())
-            sweep_variant<TL, 2, false>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax);
+        if constexpr (sweep_built<TL, 2, false, T>())
+            sweep_variant<TL, 2, false, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax);
     } else if (fs) {
-        if constexpr (sweep_fits_lds<TL, 1, true>())
-            sweep_variant<TL, 1, true>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax);
+        if constexpr (sweep_built<TL, 1, true, T>())
+            sweep_variant<TL, 1, true, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax);
     } else {
-        sweep_variant<TL, 1, false>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax);
+        if constexpr (sweep_built<TL, 1, false, T>())
+            sweep_variant<TL, 1, false, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax);
     }
 }
 
 // ns (1 or 2) fused red-black sweeps of a fine level (n >= 32) with tile shape cfg, the source
 // staged in LDS when fs: uin -> uout.
-template <class SS>
-static void stream_variant(hipStream_t s, const float *uin, float *uout, const float *f, int n, float h2, float h2i,
-                           bool zero, bool prolong, bool resid, const float *uc, float *rc, double *resmax)
+template <class SS, typename T>
+static void stream_variant(hipStream_t s, const T *uin, T *uout, const T *f, int n, T h2, T h2i,
+                           bool zero, bool prolong, bool resid, const T *uc, T *rc, double *resmax)
 {
-    const int ntiles = (n / SS::SX) * (n / SS::SY) * (n / SS::ZC);
-    const dim3 grid(8 * ((ntiles + 7) / 8)), block(SS::NT);
-    if (resid && zero)
-        hipLaunchKernelGGL((k_sweep_stream<SS, true, false, true>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
-    else if (resid)
-        hipLaunchKernelGGL((k_sweep_stream<SS, false, false, true>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
-    else if (prolong)
-        hipLaunchKernelGGL((k_sweep_stream<SS, false, true, false>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
-    else if (zero)
-        hipLaunchKernelGGL((k_sweep_stream<SS, true, false, false>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
-    else
-        hipLaunchKernelGGL((k_sweep_stream<SS, false, false, false>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+    if constexpr (stream_built<SS, T>()) {
+        const int ntiles = (n / SS::SX) * (n / SS::SY) * (n / SS::ZC);
+        const dim3 grid(8 * ((ntiles + 7) / 8)), block(SS::NT);
+        if (resid && zero)
+            hipLaunchKernelGGL((k_sweep_stream<SS, true, false, true, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+        else if (resid)
+            hipLaunchKernelGGL((k_sweep_stream<SS, false, false, true, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+        else if (prolong)
+            hipLaunchKernelGGL((k_sweep_stream<SS, false, true, false, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+        else if (zero)
+            hipLaunchKernelGGL((k_sweep_stream<SS, true, false, false, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+        else
+            hipLaunchKernelGGL((k_sweep_stream<SS, false, false, false, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+    }
 }
 
-static int launch_sweep_cfg(hipStream_t s, int cfg, int ns, bool fs, const float *uin, float *uout, const float *f,
-                            int n, double h, bool zero, bool prolong, bool resid, const float *uc, float *rc,
+template <typename T>
+static int launch_sweep_cfg(hipStream_t s, int cfg, int ns, bool fs, const T *uin, T *uout, const T *f,
+                            int n, double h, bool zero, bool prolong, bool resid, const T *uc, T *rc,
                             double *resmax)
 {
     SG_REQUIRE(cfg >= 0 && cfg < kNumCfg && cfg_fits(cfg, n), "sweep shape %d does not fit n = %d", cfg, n);
     SG_REQUIRE(ns >= 1 && ns <= kMaxSweepsPerLaunch, "bad sweeps per launch %d", ns);
-    SG_REQUIRE(cfg_ok(cfg, ns, fs), "sweep shape %d with %d sweeps (staged %d) does not exist", cfg, ns, (int)fs);
-    const float h2 = (float)(h * h), h2i = (float)(1.0 / (h * h));
+    SG_REQUIRE(cfg_ok<T>(cfg, ns, fs), "sweep shape %d with %d sweeps (staged %d) does not exist", cfg, ns, (int)fs);
+    const T h2 = (T)(h * h), h2i = (T)(1.0 / (h * h));
     switch (cfg) {
-    case kNumTiles + 0: stream_variant<Stream0>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 1: stream_variant<Stream1>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 2: stream_variant<Stream2>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 3: stream_variant<Stream3>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 4: stream_variant<Stream4>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 5: stream_variant<Stream5>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 6: stream_variant<Stream6>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 7: stream_variant<Stream7>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 8: stream_variant<Stream8>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case 0: sweep_ns<Tile0>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case 1: sweep_ns<Tile1>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case 2: sweep_ns<Tile2>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case 3: sweep_ns<Tile3>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    default: sweep_ns<Tile4>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 0: stream_variant<Stream0, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 1: stream_variant<Stream1, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 2: stream_variant<Stream2, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 3: stream_variant<Stream3, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 4: stream_variant<Stream4, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 5: stream_variant<Stream5, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 6: stream_variant<Stream6, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 7: stream_variant<Stream7, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 8: stream_variant<Stream8, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case 0: sweep_ns<Tile0, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case 1: sweep_ns<Tile1, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case 2: sweep_ns<Tile2, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case 3: sweep_ns<Tile3, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    default: sweep_ns<Tile4, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     }
     SG_CHECK_LAUNCH();
     return SG_OK;
@@ -359,12 +364,26 @@ static int level_of(const sg_uniform *c, int n)
     return -1;
 }
 
-// One launch of ns sweeps on level l with its autotuned tile shape.
-static int launch_sweep(sg_uniform *c, int l, int ns, const float *uin, float *uout, bool zero, bool prolong,
-                        bool resid, const float *uc, float *rc, double *resmax)
+// sweeps per launch on level l; one launch of ns sweeps there with its shape (FP32: autotuned)
+template <typename T> static int level_ns(sg_uniform *c, int l)
 {
-    return launch_sweep_cfg(c->stream, c->tile_cfg[l], ns, c->tile_fs[l] != 0, uin, uout, c->f.RHO[l], c->nl[l],
-                            c->hl[l], zero, prolong, resid, uc, rc, resmax);
+    if constexpr (std::is_same<T, float>::value) return c->tile_ns[l];
+    else return fp64_two_sweeps(n3(c->nl[l])) ? 2 : 1;
+}
+
+template <typename T>
+static int launch_sweep(sg_uniform *c, int l, int ns, const T *uin, T *uout, bool zero, bool prolong, bool resid,
+                        const T *uc, T *rc, double *resmax)
+{
+    const int n = c->nl[l];
+    int cfg = c->tile_cfg[l];
+    bool fs = c->tile_fs[l] != 0;
+    if constexpr (std::is_same<T, double>::value) {
+        cfg = fp64_sweep_shape(n >= 64 ? 64 : n, n3(n), fp64_two_sweeps(n3(n)));
+        fs = false;
+    }
+    return launch_sweep_cfg<T>(c->stream, cfg, ns, fs, uin, uout, levels<T>(c).RHO[l], n, c->hl[l], zero, prolong,
+                               resid, uc, rc, resmax);
 }
 
 // Autotuner: for every fine level, time each fitting (tile shape, sweeps per launch) on the
@@ -388,12 +407,12 @@ static int autotune_tiles(sg_uniform *c)
             bool fs;
             cand_decode(cand, cfg, ns, fs);
             c->tune_ms[l][cand] = -1.f;
-            if (!cfg_fits(cfg, n) || !cfg_ok(cfg, ns, fs)) continue;
+            if (!cfg_fits(cfg, n) || !cfg_ok<float>(cfg, ns, fs)) continue;
             const int reps = n >= 256 ? 3 : 6;  // timed visits, after one untimed
             int flip = 0;
             auto launch = [&](int k, bool prolong, bool resid) {
-                const int r = launch_sweep_cfg(c->stream, cfg, k, fs, flip ? c->U1[l] : c->f.U[l],
-                                               flip ? c->f.U[l] : c->U1[l], c->f.RHO[l], n, c->hl[l], false, prolong,
+                const int r = launch_sweep_cfg<float>(c->stream, cfg, k, fs, flip ? c->f.U1[l] : c->f.U[l],
+                                               flip ? c->f.U[l] : c->f.U1[l], c->f.RHO[l], n, c->hl[l], false, prolong,
                                                resid, prolong ? c->f.U[l + 1] : nullptr,
                                                resid ? c->f.RHO[l + 1] : nullptr, nullptr);
                 flip ^= 1;
@@ -432,41 +451,23 @@ static int autotune_tiles(sg_uniform *c)
     return rc;
 }
 
-// The levels of <= 16^3 cells held by k_coarse (from the first such level, lc) and the Hartley
-// basis of level lc for its exact solve, which applies only when lc > 0 (a grid of <= 16^3 cells
-// keeps the V-cycle: its smoothing also yields Resmaxg).
+// The first level of <= 16^3 cells, lc, and the Hartley basis of its exact solve, which applies only
+// when lc > 0 (a grid of <= 16^3 cells keeps the V-cycle: its smoothing also yields Resmaxg).
 static int coarse_levels(sg_uniform *c)
 {
-    const int lmax = c->nlev - 1;
     int lc = 0;
     while (c->nl[lc] > kCoarseMaxN) ++lc;
-    CoarseLevels &L = c->coarse;
-    L = CoarseLevels{};
-    L.nlev = lmax - lc + 1;
-    SG_REQUIRE(L.nlev <= 8, "too many coarse levels");
-    int off = 0;
-    for (int q = 0; q < L.nlev; ++q) {
-        const int l = lc + q;
-        L.n[q] = c->nl[l];
-        L.lg[q] = 0;
-        while ((1 << L.lg[q]) < c->nl[l]) ++L.lg[q];
-        L.h2[q] = (float)(c->hl[l] * c->hl[l]);
-        L.h2i[q] = (float)(1.0 / (c->hl[l] * c->hl[l]));
-        L.off[q] = off;
-        off += c->nl[l] * c->nl[l] * c->nl[l];
-    }
-    SG_REQUIRE(off <= kCoarseCells, "coarse levels exceed LDS capacity");
-    L.exact = lc > 0;
-    if (L.exact) {
+    if (lc > 0) {
         const int m = c->nl[lc];
         double Q[kCoarseMaxN * kCoarseMaxN], lam[kCoarseMaxN];
         hartley_basis(m, c->hl[lc], Q, lam);
-        for (int e = 0; e < m * m; ++e) L.Q[e] = (float)Q[e];
-        for (int e = 0; e < m; ++e) L.lam[e] = (float)lam[e];
+        c->cexact.n = m;
+        for (int e = 0; e < m * m; ++e) c->cexact.Q[e] = (float)Q[e];
+        for (int e = 0; e < m; ++e) c->cexact.lam[e] = (float)lam[e];
     }
     c->lc = lc;
     // the exact-coarse cycle ends at the first level below level 0 with <= 64^3 cells; with more
-    // than 16^3 cells it is solved by the plane-parallel kernels, else by k_coarse
+    // than 16^3 cells it is solved by the plane-parallel kernels, else by k_coarse_exact
     int lb = lc;
     if (lc > 0) {
         int l = 1;
@@ -489,88 +490,107 @@ static int coarse_levels(sg_uniform *c)
     return SG_OK;
 }
 
-// k_coarse on the held levels; exact: solve level lc exactly (needs c->coarse.exact).
-static int launch_coarse_k(sg_uniform *c, bool exact, const float *rhs, float *u, int mode, int ncycle, int npre,
-                           int npost, double *resmax)
+template <typename T, int N>
+static void coarse_n(sg_uniform *c, const T *rhs, T *u, int mode, int ncycle, int npre, int npost, double *resmax)
 {
-    SG_REQUIRE(!exact || c->coarse.exact, "exact coarse solve needs a level below the finest");
-    CoarseLevels L = c->coarse;
-    L.exact = exact ? 1 : 0;
-    hipLaunchKernelGGL(k_coarse, dim3(1), dim3(kCoarseThreads), 0, c->stream, rhs, u, L, mode, ncycle, npre, npost,
-                       resmax);
+    hipLaunchKernelGGL((k_coarse<T, N>), dim3(1), dim3(kCoarseThreads), 0, c->stream, rhs, u,
+                       coarse_coef<T>(c->hl[c->lc]), mode, ncycle, npre, npost, resmax);
+}
+
+// The reference's cycles on level lc and below.
+template <typename T>
+static int launch_coarse(sg_uniform *c, int mode, int ncycle, int npre, int npost, double *resmax)
+{
+    const T *rhs = levels<T>(c).RHO[c->lc];
+    T *u = levels<T>(c).U[c->lc];
+    switch (c->nl[c->lc]) {
+    case 16: coarse_n<T, 16>(c, rhs, u, mode, ncycle, npre, npost, resmax); break;
+    case 8: coarse_n<T, 8>(c, rhs, u, mode, ncycle, npre, npost, resmax); break;
+    case 4: coarse_n<T, 4>(c, rhs, u, mode, ncycle, npre, npost, resmax); break;
+    default: coarse_n<T, 2>(c, rhs, u, mode, ncycle, npre, npost, resmax); break;
+    }
     SG_CHECK_LAUNCH();
     return SG_OK;
 }
 
-// U[lb] := exact solution for RHO[lb] (FP32): k_coarse when lb is the first level of <= 16^3
+// U[lb] := exact solution for RHO[lb] (FP32): k_coarse_exact when lb is the first level of <= 16^3
 // cells, else the three plane-parallel launches with U1[lb] as the intermediate array.
-static int exact_bottom(sg_uniform *c, int mode, int ncycle, int npre, int npost)
+static int exact_bottom(sg_uniform *c)
 {
     const int lb = c->lb, n = c->nl[lb];
-    SG_REQUIRE(c->coarse.exact, "exact coarse solve needs a level below the finest");
-    if (lb == c->lc) return launch_coarse_k(c, true, c->f.RHO[lb], c->f.U[lb], mode, ncycle, npre, npost, nullptr);
-    SG_REQUIRE(n <= kPlaneMaxN && n % 16 == 0 && c->d_qx && c->d_invx && c->U1[lb],
+    SG_REQUIRE(c->lc > 0, "exact coarse solve needs a level below the finest");
+    if (lb == c->lc) {
+        hipLaunchKernelGGL(k_coarse_exact, dim3(1), dim3(kCoarseThreads), 0, c->stream, (const float *)c->f.RHO[lb],
+                           c->f.U[lb], c->cexact);
+        SG_CHECK_LAUNCH();
+        return SG_OK;
+    }
+    SG_REQUIRE(n <= kPlaneMaxN && n % 16 == 0 && c->d_qx && c->d_invx && c->f.U1[lb],
                "plane-parallel exact solve not set up (n = %d)", n);
     const dim3 grid(n * plane_groups(n)), block(kSplitThreads);
-    hipLaunchKernelGGL(k_exact_xy_split, grid, block, 0, c->stream, (const float *)c->f.RHO[lb], c->U1[lb],
+    hipLaunchKernelGGL(k_exact_xy_split, grid, block, 0, c->stream, (const float *)c->f.RHO[lb], c->f.U1[lb],
                        (const float *)c->d_qx, n);
     SG_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_exact_z_split, grid, block, 0, c->stream, c->U1[lb], (const float *)c->d_qx,
+    hipLaunchKernelGGL(k_exact_z_split, grid, block, 0, c->stream, c->f.U1[lb], (const float *)c->d_qx,
                        (const float *)c->d_invx, n);
     SG_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_exact_xy_split, grid, block, 0, c->stream, (const float *)c->U1[lb], c->f.U[lb],
+    hipLaunchKernelGGL(k_exact_xy_split, grid, block, 0, c->stream, (const float *)c->f.U1[lb], c->f.U[lb],
                        (const float *)c->d_qx, n);
     SG_CHECK_LAUNCH();
     return SG_OK;
 }
 
-// mg_lin (mg.F90:106-218) in FP32 with fused kernels: the levels of <= 16^3 cells run inside one
+// mg_lin (mg.F90:106-218) with fused kernels: the levels of <= 16^3 cells run inside one
 // single-workgroup kernel (k_coarse); each fine-level visit of a V-cycle is npre + npost fused
 // sweeps, the last pre-sweep carrying the residual and its restriction, the first post-sweep the
-// prolongated correction.  With `exact` the cycle instead ends at level lb, solved exactly
-// (exact_bottom).  Same values as mg_lin<float> with the same `exact`, bit for bit.  *u0 receives
+// prolongated correction.  With `exact` (FP32) the cycle instead ends at level lb, solved exactly
+// (exact_bottom).  Same values as mg_lin<T> with the same `exact`, bit for bit.  *u0 receives
 // the buffer that holds the level-0 correction.  rhs1_ready: RHO[1] already holds the restriction
 // of RHO[0] (formed with the residual by k_update_resid).
-static int fast_mg_lin(sg_uniform *c, int ncycle, int npre, int npost, double *resmax, const float **u0,
-                       bool exact, bool rhs1_ready)
+template <typename T>
+static int fast_mg_lin(sg_uniform *c, int ncycle, int npre, int npost, double *resmax, const T **u0, bool exact,
+                       bool rhs1_ready)
 {
     SG_REQUIRE(npre >= 1 && npost >= 1, "fused path needs npre, npost >= 1");
-    Levels<float> &A = c->f;
+    Levels<T> &A = levels<T>(c);
     hipStream_t s = c->stream;
-    exact = exact && c->coarse.exact;
+    exact = exact && std::is_same<T, float>::value && c->lc > 0;
     const int lc = exact ? c->lb : c->lc;   // level of the coarse-grid solve
     int cur[kMaxLev] = {};
-    auto buf = [&](int l, int b) -> float * { return b ? c->U1[l] : A.U[l]; };
-    for (int l = rhs1_ready ? 2 : 1; l <= lc; ++l) SG_TRY(launch_restrict<float>(s, A.RHO[l], A.RHO[l - 1], c->nl[l]));
-    if (exact) SG_TRY(exact_bottom(c, 0, ncycle, npre, npost));
-    else SG_TRY(launch_coarse_k(c, false, A.RHO[lc], A.U[lc], 0, ncycle, npre, npost, lc == 0 ? resmax : nullptr));
+    auto buf = [&](int l, int b) -> T * { return b ? A.U1[l] : A.U[l]; };
+    auto bottom = [&](int mode) -> int {
+        if (exact) return exact_bottom(c);
+        return launch_coarse<T>(c, mode, ncycle, npre, npost, lc == 0 ? resmax : nullptr);
+    };
+    for (int l = rhs1_ready ? 2 : 1; l <= lc; ++l) SG_TRY(launch_restrict<T>(s, A.RHO[l], A.RHO[l - 1], c->nl[l]));
+    SG_TRY(bottom(0));
     cur[lc] = 0;
     for (int ml = lc - 1; ml >= 0; --ml) {
-        SG_TRY(launch_interp_cubic_tile(s, A.U[ml], buf(ml + 1, cur[ml + 1]), c->nl[ml]));
+        SG_TRY(launch_interp_cubic_tile<T>(s, A.U[ml], buf(ml + 1, cur[ml + 1]), c->nl[ml]));
         cur[ml] = 0;
         for (int jc = 0; jc < ncycle; ++jc) {
             for (int v = ml; v <= lc - 1; ++v) {
-                // npre sweeps in launches of up to tile_ns[v]; the first may start from zero, the
+                // npre sweeps in launches of up to level_ns(v); the first may start from zero, the
                 // last carries the residual restriction
                 for (int r = npre, first = 1; r > 0; first = 0) {
-                    const int k = std::min(r, c->tile_ns[v]);
+                    const int k = std::min(r, level_ns<T>(c, v));
                     const bool last = r == k;
-                    SG_TRY(launch_sweep(c, v, k, buf(v, cur[v]), buf(v, 1 - cur[v]), first && v > ml, false, last,
-                                        nullptr, last ? A.RHO[v + 1] : nullptr, nullptr));
+                    SG_TRY(launch_sweep<T>(c, v, k, buf(v, cur[v]), buf(v, 1 - cur[v]), first && v > ml, false, last,
+                                           nullptr, last ? A.RHO[v + 1] : nullptr, nullptr));
                     cur[v] ^= 1;
                     r -= k;
                 }
             }
-            if (exact) SG_TRY(exact_bottom(c, 1, ncycle, npre, npost));
-            else SG_TRY(launch_coarse_k(c, false, A.RHO[lc], A.U[lc], 1, ncycle, npre, npost, nullptr));
+            SG_TRY(bottom(1));
             cur[lc] = 0;
             for (int v = lc - 1; v >= ml; --v) {
                 // npost sweeps; the first launch adds the prolongated correction
                 for (int r = npost, first = 1; r > 0; first = 0) {
-                    const int k = std::min(r, c->tile_ns[v]);
+                    const int k = std::min(r, level_ns<T>(c, v));
                     const bool lastcall = (ml == 0 && jc == ncycle - 1 && v == 0 && r == k);
-                    SG_TRY(launch_sweep(c, v, k, buf(v, cur[v]), buf(v, 1 - cur[v]), false, first, false,
-                                        first ? buf(v + 1, cur[v + 1]) : nullptr, nullptr, lastcall ? resmax : nullptr));
+                    SG_TRY(launch_sweep<T>(c, v, k, buf(v, cur[v]), buf(v, 1 - cur[v]), false, first, false,
+                                           first ? buf(v + 1, cur[v + 1]) : nullptr, nullptr,
+                                           lastcall ? resmax : nullptr));
                     cur[v] ^= 1;
                     r -= k;
                 }
@@ -603,39 +623,58 @@ static int read_norms(sg_uniform *c, bool published = false)
     return SG_OK;
 }
 
+// Whether the outer step leaves the restricted residual in RHO[1] (the z-marching form, n >= 64).
+static bool restricts_residual(const sg_uniform *c) { return c->n >= 64; }
+
+// phi_out = phi_in + e and r = f - L phi_out into RHO[0] (FP32 or FP64), with the norms of r.
 // e == nullptr: the first residual (no update); pout, when given, receives a copy of pin, and with
 // fnorms max|src| and sum src^2 land in dnorm[3..4].
-static int launch_update_resid(sg_uniform *c, const double *pin, const float *e, double *pout, const double *src,
+template <typename T>
+static int launch_update_resid(sg_uniform *c, const double *pin, const T *e, double *pout, const double *src,
                                bool fnorms = false)
 {
     const int n = c->n, lg = ilog2(n);
     const long cells = n3(n);
-    // z chunk: about kNormBlocks patches of 512 cells per plane
-    int zc = (int)std::max<long>(4, std::min<long>(32, cells / (512L * kNormBlocks)));
-    zc = std::min(zc, n);
-    const bool wide = n % 256 == 0;  // 256 x 4 patches, else 64 x 8
-    const int tx = wide ? 256 : 64, ty = wide ? 4 : 8;
-    SG_REQUIRE(n >= 64 && n % tx == 0 && n % ty == 0 && n % zc == 0, "update+residual: bad n = %d", n);
-    const dim3 grid(n / tx, n / ty, n / zc), block(tx * ty);
-    const int nb = (int)(grid.x * grid.y * grid.z);
-    SG_REQUIRE(nb <= c->npart, "norm partial buffer too small");
-    SG_REQUIRE(c->nlev > 1 && zc % 2 == 0, "update+residual: no level to restrict into");
+    Levels<T> &A = levels<T>(c);
     const double h2i = 1.0 / (c->h * c->h);
-    // the residual restricted into RHO[1] here: the fused inner solve starts from it
     double *fpmax = fnorms ? c->pmax + c->npart : nullptr, *fpsum = fnorms ? c->psum + c->npart : nullptr;
-    if (e && wide)
-        hipLaunchKernelGGL((k_update_resid<true, 256, 4>), grid, block, 0, c->stream, pin, e, pout, src, c->f.RHO[0],
-                           lg, h2i, zc, c->pmax, c->psum, c->f.RHO[1], fpmax, fpsum);
-    else if (e)
-        hipLaunchKernelGGL((k_update_resid<true, 64, 8>), grid, block, 0, c->stream, pin, e, pout, src, c->f.RHO[0],
-                           lg, h2i, zc, c->pmax, c->psum, c->f.RHO[1], fpmax, fpsum);
-    else if (wide)
-        hipLaunchKernelGGL((k_update_resid<false, 256, 4>), grid, block, 0, c->stream, pin, e, pout, src, c->f.RHO[0],
-                           lg, h2i, zc, c->pmax, c->psum, c->f.RHO[1], fpmax, fpsum);
-    else
-        hipLaunchKernelGGL((k_update_resid<false, 64, 8>), grid, block, 0, c->stream, pin, e, pout, src, c->f.RHO[0],
-                           lg, h2i, zc, c->pmax, c->psum, c->f.RHO[1], fpmax, fpsum);
-    SG_CHECK_LAUNCH();
+    int nb;
+    if (!restricts_residual(c)) {
+        nb = (int)nblocks(cells);
+        SG_REQUIRE(nb <= c->npart, "norm partial buffer too small");
+        if (e)
+            hipLaunchKernelGGL((k_update_resid_cells<true, T>), dim3(nb), dim3(kBlock), 0, c->stream, pin, e, pout, src,
+                               A.RHO[0], lg, h2i, c->pmax, c->psum, fpmax, fpsum);
+        else
+            hipLaunchKernelGGL((k_update_resid_cells<false, T>), dim3(nb), dim3(kBlock), 0, c->stream, pin, e, pout, src,
+                               A.RHO[0], lg, h2i, c->pmax, c->psum, fpmax, fpsum);
+        SG_CHECK_LAUNCH();
+    } else {
+        // z chunk: about kNormBlocks patches of 512 cells per plane
+        int zc = (int)std::max<long>(4, std::min<long>(32, cells / (512L * kNormBlocks)));
+        zc = std::min(zc, n);
+        const bool wide = n % 256 == 0;  // 256 x 4 patches, else 64 x 8
+        const int tx = wide ? 256 : 64, ty = wide ? 4 : 8;
+        SG_REQUIRE(n >= 64 && n % tx == 0 && n % ty == 0 && n % zc == 0, "update+residual: bad n = %d", n);
+        const dim3 grid(n / tx, n / ty, n / zc), block(tx * ty);
+        nb = (int)(grid.x * grid.y * grid.z);
+        SG_REQUIRE(nb <= c->npart, "norm partial buffer too small");
+        SG_REQUIRE(c->nlev > 1 && zc % 2 == 0, "update+residual: no level to restrict into");
+        // the residual restricted into RHO[1] here: the fused inner solve starts from it
+        if (e && wide)
+            hipLaunchKernelGGL((k_update_resid<true, 256, 4, T>), grid, block, 0, c->stream, pin, e, pout, src, A.RHO[0],
+                               lg, h2i, zc, c->pmax, c->psum, A.RHO[1], fpmax, fpsum);
+        else if (e)
+            hipLaunchKernelGGL((k_update_resid<true, 64, 8, T>), grid, block, 0, c->stream, pin, e, pout, src, A.RHO[0],
+                               lg, h2i, zc, c->pmax, c->psum, A.RHO[1], fpmax, fpsum);
+        else if (wide)
+            hipLaunchKernelGGL((k_update_resid<false, 256, 4, T>), grid, block, 0, c->stream, pin, e, pout, src, A.RHO[0],
+                               lg, h2i, zc, c->pmax, c->psum, A.RHO[1], fpmax, fpsum);
+        else
+            hipLaunchKernelGGL((k_update_resid<false, 64, 8, T>), grid, block, 0, c->stream, pin, e, pout, src, A.RHO[0],
+                               lg, h2i, zc, c->pmax, c->psum, A.RHO[1], fpmax, fpsum);
+        SG_CHECK_LAUNCH();
+    }
     if (fnorms) {
         hipLaunchKernelGGL(k_norm_finalize, dim3(1), dim3(1024), 0, c->stream, (const double *)fpmax,
                            (const double *)fpsum, nb, c->dnorm + 3, (double *)nullptr);
@@ -647,38 +686,12 @@ static int launch_update_resid(sg_uniform *c, const double *pin, const float *e,
     return SG_OK;
 }
 
-// whether the mixed solve uses the fused update+residual step with a second phi buffer
-static bool pingpong(const sg_uniform *c, const sg_params *p)
+// whether the solve takes the fused kernels, with the update and the next residual in one step
+// between two phi buffers; else one kernel per reference loop nest (fused = 0, or a cycle without
+// pre- or post-smoothing, whose restriction and prolongation have no sweep to join)
+static bool fused_solve(const sg_uniform *c, const sg_params *p)
 {
-    return p->precision == SG_PREC_MIXED && p->fused && c->n >= 64 && c->psi_alt;
-}
-
-// One outer iteration after the first residual: inner solve on RHO[0] (= f - L phi), update
-// phi += U[0] (from pin into pout; in place when pin == pout), next residual with its norms into
-// dnorm[0..1].  Resmaxg lands in dnorm[2].
-static int outer_iteration(sg_uniform *c, const double *pin, double *pout, const double *src, const sg_params *p)
-{
-    // Resmaxg is only read by the reference stopping test; the true-residual test skips it.
-    double *resmax = p->stop_mode == SG_STOP_REFERENCE ? c->dnorm + 2 : nullptr;
-    SG_TRY(launch_fill<double>(c->stream, c->dnorm + 2, 1));
-    if (p->precision == SG_PREC_MIXED) {
-        const float *u0 = c->f.U[0];
-        const bool exact = p->coarse == SG_COARSE_EXACT;
-        // with pin != pout every residual came from launch_update_resid, which restricted it too
-        if (p->fused) SG_TRY(fast_mg_lin(c, p->ncycle, p->npre, p->npost, resmax, &u0, exact, pin != pout));
-        else SG_TRY(mg_lin<float>(c, p->ncycle, p->npre, p->npost, resmax, exact));
-        if (pin != pout) {
-            SG_TRY(launch_update_resid(c, pin, u0, pout, src));
-        } else {
-            SG_TRY(launch_update<float>(c, pout, u0));
-            SG_TRY((launch_resid<double, float>(c, c->f.RHO[0], pout, src, c->n, c->h, c->dnorm)));
-        }
-    } else {
-        SG_TRY(mg_lin<double>(c, p->ncycle, p->npre, p->npost, resmax));
-        SG_TRY(launch_update<double>(c, pout, c->d.U[0]));
-        SG_TRY((launch_resid<double, double>(c, c->d.RHO[0], pout, src, c->n, c->h, c->dnorm)));
-    }
-    return SG_OK;
+    return p->fused && p->npre >= 1 && p->npost >= 1 && c->psi_alt;
 }
 
 static void drop_graphs(sg_uniform *c)
@@ -689,20 +702,35 @@ static void drop_graphs(sg_uniform *c)
     }
 }
 
-static int run_outer_iteration(sg_uniform *c, const double *pin, double *pout, const double *src,
-                               const sg_params *p, int parity)
+// One inner solve: correction of the residual in RHO[0]; *u0 receives its buffer.  Resmaxg of the
+// last smoothing lands in dnorm[2] when the reference stopping test reads it.
+template <typename T> static int inner_solve(sg_uniform *c, const sg_params *p, const T **u0)
 {
-    if (!(p->use_graph && p->precision == SG_PREC_MIXED)) return outer_iteration(c, pin, pout, src, p);
-    sg_uniform::Graph &g = c->graph[parity & 1];
-    const bool same = g.exec && g.pin == pin && g.pout == pout && g.src == src && g.ncycle == p->ncycle &&
-                      g.npre == p->npre && g.npost == p->npost && g.fused == p->fused && g.stop == p->stop_mode &&
-                      g.coarse == p->coarse;
+    double *resmax = p->stop_mode == SG_STOP_REFERENCE ? c->dnorm + 2 : nullptr;
+    if (resmax) SG_TRY(launch_fill<double>(c->stream, resmax, 1));
+    const bool exact = p->coarse == SG_COARSE_EXACT;
+    *u0 = levels<T>(c).U[0];
+    if (fused_solve(c, p))
+        return fast_mg_lin<T>(c, p->ncycle, p->npre, p->npost, resmax, u0, exact, restricts_residual(c));
+    return mg_lin<T>(c, p->ncycle, p->npre, p->npost, resmax, exact);
+}
+
+// The inner solve replayed as a graph.  Not for a grid held by k_coarse alone (its inner solve is one
+// launch), nor for the FP64 solve without fused kernels (the plain form: every launch eager).
+template <typename T> static int run_inner_solve(sg_uniform *c, const sg_params *p, const T **u0)
+{
+    const bool fp64 = std::is_same<T, double>::value;
+    if (!p->use_graph || (fused_solve(c, p) ? c->lc == 0 : fp64)) return inner_solve<T>(c, p, u0);
+    sg_uniform::Graph &g = c->graph[fp64 ? 1 : 0];
+    const bool same = g.exec && g.ncycle == p->ncycle && g.npre == p->npre && g.npost == p->npost &&
+                      g.fused == p->fused && g.stop == p->stop_mode && g.coarse == p->coarse;
     if (!same) {
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
         g = sg_uniform::Graph();
         hipGraph_t graph = nullptr;
+        const T *u = nullptr;
         SG_HIP(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        const int rc = outer_iteration(c, pin, pout, src, p);
+        const int rc = inner_solve<T>(c, p, &u);
         const hipError_t e = hipStreamEndCapture(c->stream, &graph);
         if (rc != SG_OK) {
             if (graph) (void)hipGraphDestroy(graph);
@@ -712,9 +740,7 @@ static int run_outer_iteration(sg_uniform *c, const double *pin, double *pout, c
         const hipError_t e2 = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0);
         (void)hipGraphDestroy(graph);
         SG_HIP(e2);
-        g.pin = pin;
-        g.pout = pout;
-        g.src = src;
+        g.u0 = u;
         g.ncycle = p->ncycle;
         g.npre = p->npre;
         g.npost = p->npost;
@@ -722,8 +748,22 @@ static int run_outer_iteration(sg_uniform *c, const double *pin, double *pout, c
         g.coarse = p->coarse;
         g.stop = p->stop_mode;
     }
+    *u0 = static_cast<const T *>(g.u0);
     SG_HIP(hipGraphLaunch(g.exec, c->stream));
     return SG_OK;
+}
+
+// One outer iteration after the first residual: inner solve on RHO[0] (= f - L phi), update
+// phi += correction (from pin into pout; in place when pin == pout), next residual with its norms into
+// dnorm[0..1].
+template <typename T>
+static int outer_iteration(sg_uniform *c, const double *pin, double *pout, const double *src, const sg_params *p)
+{
+    const T *u0 = nullptr;
+    SG_TRY(run_inner_solve<T>(c, p, &u0));
+    if (pin != pout) return launch_update_resid<T>(c, pin, u0, pout, src);
+    SG_TRY(launch_update<T>(c, pout, u0));
+    return launch_resid<double, T>(c, levels<T>(c).RHO[0], pout, src, c->n, c->h, c->dnorm);
 }
 
 // mg.F90:42-94: FP64 defect correction psi += L^-1 (src - L psi) with the chosen inner solver.
@@ -744,13 +784,17 @@ static int uniform_cycle(sg_uniform *c, double *psi, const double *src, const sg
     std::memset(st, 0, sizeof(*st));
     const bool mixed = p->precision == SG_PREC_MIXED;
     SG_HIP(hipEventRecord(c->ev0, c->stream));
-    const bool pp = pingpong(c, p);
+    const bool pp = fused_solve(c, p);
     // With the fused update the iterations alternate between psi and psi_alt, so an odd count ends
     // in psi_alt and costs a final copy.  When the previous solve on this context took an odd
     // count, the first residual step also copies psi into psi_alt and the iterations start there.
     const bool start_alt = pp && c->last_odd;
-    if (pp) {
-        SG_TRY(launch_update_resid(c, psi, nullptr, start_alt ? c->psi_alt : nullptr, src, true));
+    SG_TRY(launch_fill<double>(c->stream, c->dnorm + 2, 1));   // Resmaxg, unless a sweep writes it
+    double *copy = start_alt ? c->psi_alt : nullptr;
+    if (pp && mixed) {
+        SG_TRY(launch_update_resid<float>(c, psi, nullptr, copy, src, true));
+    } else if (pp) {
+        SG_TRY(launch_update_resid<double>(c, psi, nullptr, copy, src, true));
     } else {
         SG_TRY(launch_norm(c, src, n3(c->n), c->dnorm + 3));
         if (mixed) SG_TRY((launch_resid<double, float>(c, c->f.RHO[0], psi, src, c->n, c->h, c->dnorm)));
@@ -778,7 +822,8 @@ static int uniform_cycle(sg_uniform *c, double *psi, const double *src, const sg
         }
         if (it >= p->maxit) break;
         double *next = pp ? (cur == psi ? c->psi_alt : psi) : cur;
-        SG_TRY(run_outer_iteration(c, cur, next, src, p, cur == psi ? 0 : 1));
+        if (mixed) SG_TRY(outer_iteration<float>(c, cur, next, src, p));
+        else SG_TRY(outer_iteration<double>(c, cur, next, src, p));
         cur = next;
         SG_TRY(read_norms(c, pp));
         ++it;
@@ -798,26 +843,26 @@ static int uniform_cycle(sg_uniform *c, double *psi, const double *src, const sg
 
 template <typename T> static int alloc_levels(sg_uniform *c, Levels<T> &A)
 {
-    for (int l = 0; l < c->nlev; ++l) {
-        const size_t bytes = sizeof(T) * (size_t)n3(c->nl[l]);
-        SG_HIP(hipMalloc(&A.U[l], bytes));
-        SG_HIP(hipMalloc(&A.RES[l], bytes));
-        SG_HIP(hipMalloc(&A.RHO[l], bytes));
-        SG_HIP(hipMemsetAsync(A.U[l], 0, bytes, c->stream));
-        SG_HIP(hipMemsetAsync(A.RES[l], 0, bytes, c->stream));
-        SG_HIP(hipMemsetAsync(A.RHO[l], 0, bytes, c->stream));
+    // one allocation for all levels, each array on a 256-byte boundary
+    size_t total = 0;
+    for (int pass = 0; pass < 2; ++pass) {
+        size_t at = 0;
+        for (int l = 0; l < c->nlev; ++l)
+            for (T **p : {&A.U[l], &A.RES[l], &A.RHO[l], &A.U1[l]}) {
+                if (pass) *p = reinterpret_cast<T *>(static_cast<char *>(A.mem) + at);
+                at += (sizeof(T) * (size_t)n3(c->nl[l]) + 255) / 256 * 256;
+            }
+        total = at;
+        if (!pass) SG_HIP(hipMalloc(&A.mem, total));
     }
+    SG_HIP(hipMemsetAsync(A.mem, 0, total, c->stream));
     return SG_OK;
 }
 
 template <typename T> static void free_levels(Levels<T> &A)
 {
-    for (int l = 0; l < kMaxLev; ++l) {
-        if (A.U[l]) (void)hipFree(A.U[l]);
-        if (A.RES[l]) (void)hipFree(A.RES[l]);
-        if (A.RHO[l]) (void)hipFree(A.RHO[l]);
-        A.U[l] = A.RES[l] = A.RHO[l] = nullptr;
-    }
+    if (A.mem) (void)hipFree(A.mem);
+    A = Levels<T>();
 }
 
 static void destroy(sg_uniform *c)
@@ -827,8 +872,6 @@ static void destroy(sg_uniform *c)
     drop_graphs(c);
     free_levels(c->d);
     free_levels(c->f);
-    for (int l = 0; l < kMaxLev; ++l)
-        if (c->U1[l]) (void)hipFree(c->U1[l]);
     if (c->psi_dev) (void)hipFree(c->psi_dev);
     if (c->psi_alt) (void)hipFree(c->psi_alt);
     if (c->d_qx) (void)hipFree(c->d_qx);
@@ -888,14 +931,9 @@ static int create(sg_uniform **out, int n, double h, int precisions)
             if (precisions & SG_PREC_FP64) SG_TRY(alloc_levels<double>(c, c->d));
             if (precisions & SG_PREC_MIXED) {
                 SG_TRY(alloc_levels<float>(c, c->f));
-                for (int l = 0; l < c->nlev; ++l) {
-                    const size_t bytes = sizeof(float) * (size_t)n3(c->nl[l]);
-                    SG_HIP(hipMalloc(&c->U1[l], bytes));
-                    SG_HIP(hipMemsetAsync(c->U1[l], 0, bytes, c->stream));
-                }
                 SG_TRY(autotune_tiles(c));
-                SG_HIP(hipMalloc(&c->psi_alt, sizeof(double) * (size_t)n3(n)));
             }
+            SG_HIP(hipMalloc(&c->psi_alt, sizeof(double) * (size_t)n3(n)));
             SG_HIP(hipStreamSynchronize(c->stream));
             return SG_OK;
         }()) != SG_OK)
@@ -1143,8 +1181,8 @@ int sg_uniform_time_smoother(sg_uniform *c, int prec, int reps, double *ms_per_s
             SG_TRY(sg::launch_relax<double>(c->stream, c->d.U[0], c->d.RHO[0], c->n, c->h, nullptr));
         else if (fused) {
             // the mixed path's fine-level sweep: U[0] -> U1[0] and back on alternate repetitions
-            float *a = (r & 1) ? c->U1[0] : c->f.U[0], *b = (r & 1) ? c->f.U[0] : c->U1[0];
-            SG_TRY(sg::launch_sweep_cfg(c->stream, c->tile_cfg[0], 1, c->tile_fs[0] != 0, a, b, c->f.RHO[0], c->n,
+            float *a = (r & 1) ? c->f.U1[0] : c->f.U[0], *b = (r & 1) ? c->f.U[0] : c->f.U1[0];
+            SG_TRY(sg::launch_sweep_cfg<float>(c->stream, c->tile_cfg[0], 1, c->tile_fs[0] != 0, a, b, c->f.RHO[0], c->n,
                                         c->h, false, false, false, nullptr, nullptr, nullptr));
         } else
             SG_TRY(sg::launch_relax<float>(c->stream, c->f.U[0], c->f.RHO[0], c->n, c->h, nullptr));
@@ -1162,7 +1200,7 @@ int sg_uniform_set_tile(sg_uniform *c, int level, int cfg, int ns, int fs)
     SG_REQUIRE(c && (c->precisions & SG_PREC_MIXED), "context lacks the mixed-precision arrays");
     SG_REQUIRE(level >= 0 && level < c->nlev && c->nl[level] > sg::kCoarseMaxN,
                "level %d is not a fused-sweep level", level);
-    SG_REQUIRE(cfg >= 0 && cfg < sg::kNumCfg && sg::cfg_fits(cfg, c->nl[level]) && sg::cfg_ok(cfg, ns, fs != 0),
+    SG_REQUIRE(cfg >= 0 && cfg < sg::kNumCfg && sg::cfg_fits(cfg, c->nl[level]) && sg::cfg_ok<float>(cfg, ns, fs != 0),
                "sweep configuration (%d, %d, %d) does not fit level %d (n = %d)", cfg, ns, fs, level, c->nl[level]);
     c->tile_cfg[level] = cfg;
     c->tile_ns[level] = ns;

@@ -142,14 +142,14 @@ __global__ void __launch_bounds__(256) k_resid(Tout *__restrict__ res, const Tin
     }
 }
 
-// Outer FP64 step of the mixed solve, fused: pout = pin + e (mg.F90:87) and
-// r = f - L pout (mg_poisson.F90:17-27) stored as FP32 for the next inner solve, with the norm
+// Outer FP64 step of the solve, fused: pout = pin + e (mg.F90:87) and r = f - L pout
+// (mg_poisson.F90:17-27) stored as Te (FP32: mixed, FP64: plain) for the next inner solve, with the norm
 // partials of r.  Neighbour values are formed as pin + e, exactly the values pout receives, so the
 // result equals the separate update and residual kernels bit for bit; pin and pout must differ.
 // UPD = false: r = f - L pin only, and pout (when given) a copy of pin.  With fpmax, the partials
-// of max|f| and sum f^2 as well.  With rc, the FP32 residual is also restricted into rc (the
+// of max|f| and sum f^2 as well.  With rc, the stored residual is also restricted into rc (the
 // next level's right-hand side, restriction.F90:132-147 operand order, as k_restrict forms it):
-// each plane's FP32 residuals go to one of four LDS planes, and the restriction of planes
+// each plane's stored residuals go to one of four LDS planes, and the restriction of planes
 // (k - 2, k - 1) runs at plane k, after its barrier.  A workgroup owns a 64 x 8 patch of (i, j) columns and marches
 // through zc planes: each thread forms its cell of the next plane (and, on the patch edge, one
 // halo cell in x and/or y) while the current plane sits in a double-buffered LDS plane with a
@@ -158,17 +158,17 @@ __global__ void __launch_bounds__(256) k_resid(Tout *__restrict__ res, const Tin
 // 64 x 8 columns, or 256 x 4 when n % 256 == 0: an x-halo cell costs a whole cache line of pin
 // and of e, so patches as wide as the grid (whose x neighbours wrap into the patch) trade those
 // for a second y-halo row per four.
-template <bool UPD, int TX, int TY>
-__global__ void __launch_bounds__(TX * TY) k_update_resid(const double *__restrict__ pin, const float *__restrict__ e,
+template <bool UPD, int TX, int TY, typename Te>
+__global__ void __launch_bounds__(TX * TY) k_update_resid(const double *__restrict__ pin, const Te *__restrict__ e,
                                                           double *__restrict__ pout, const double *__restrict__ f,
-                                                          float *__restrict__ r32, int lg, double h2i, int zc,
-                                                          double *pmax, double *psum, float *__restrict__ rc,
+                                                          Te *__restrict__ r0, int lg, double h2i, int zc,
+                                                          double *pmax, double *psum, Te *__restrict__ rc,
                                                           double *fpmax, double *fpsum)
 {
     constexpr int SP = TX + 2;
     static_assert(TY % 2 == 0 && TX % 2 == 0 && TX * TY <= 1024, "update+residual patch");
     __shared__ double sp[2][(TY + 2) * SP];
-    __shared__ float sr[4][TY * TX];
+    __shared__ Te sr[4][TY * TX];
     const int n = 1 << lg, m = n - 1;
     const int tx = (int)threadIdx.x % TX, ty = (int)threadIdx.x / TX;
     // XCD-aware patch numbering: the hardware deals consecutive workgroups round-robin to the 8
@@ -182,7 +182,7 @@ __global__ void __launch_bounds__(TX * TY) k_update_resid(const double *__restri
     const int z0 = pbz * zc;
     auto at = [&](int ii, int jj, int kk) { return (kk << (2 * lg)) | (jj << lg) | ii; };
     // pin, e, f and pout stream through once per outer iteration: non-temporal, so that the
-    // last-level cache keeps r32, which the next inner solve reads first
+    // last-level cache keeps r0, which the next inner solve reads first
     auto P = [&](int q) -> double {
         return UPD ? __builtin_nontemporal_load(pin + q) + (double)__builtin_nontemporal_load(e + q)
                    : __builtin_nontemporal_load(pin + q);
@@ -203,10 +203,10 @@ __global__ void __launch_bounds__(TX * TY) k_update_resid(const double *__restri
         const int t = (int)threadIdx.x;
         if (t < (TX / 2) * (TY / 2)) {
             const int cx = t % (TX / 2), cy = t / (TX / 2);
-            const float *a = sr[k0 & 3] + 2 * cy * TX + 2 * cx, *b = sr[(k0 + 1) & 3] + 2 * cy * TX + 2 * cx;
+            const Te *a = sr[k0 & 3] + 2 * cy * TX + 2 * cx, *b = sr[(k0 + 1) & 3] + 2 * cy * TX + 2 * cx;
             const int ic = pbx * (TX / 2) + cx, jc = pby * (TY / 2) + cy, kc = (k0 & m) >> 1;
             rc[(kc << (2 * lgc)) | (jc << lgc) | ic] =
-                restrict_value<float>(a[0], a[1], a[TX], b[0], a[TX + 1], b[1], b[TX], b[TX + 1]);
+                restrict_value<Te>(a[0], a[1], a[TX], b[0], a[TX + 1], b[1], b[TX], b[TX + 1]);
         }
     };
     for (int k = z0; k < z0 + zc; ++k) {
@@ -226,14 +226,14 @@ __global__ void __launch_bounds__(TX * TY) k_update_resid(const double *__restri
         const int c = at(i, j, k);
         __syncthreads();
         const double rv = resid_value<double>(zcen, s[sc + 1], s[sc - 1], s[sc + SP], s[sc - SP], zp, zm, fc, h2i);
-        r32[c] = (float)rv;
+        r0[c] = (Te)rv;
         if (pout) __builtin_nontemporal_store(zcen, pout + c);
         if (fpmax) {
             fmx = fmax(fmx, fabs(fc));
             fsm += fc * fc;
         }
         if (rc) {
-            sr[k & 3][ty * TX + tx] = (float)rv;
+            sr[k & 3][ty * TX + tx] = (Te)rv;
             if (((k - z0) & 1) == 0 && k >= z0 + 2) restrict_pair(k - 2);
         }
         mx = fmax(mx, fabs(rv));
@@ -259,6 +259,46 @@ __global__ void __launch_bounds__(TX * TY) k_update_resid(const double *__restri
         if (threadIdx.x == 0) {
             fpmax[b] = fmx;
             fpsum[b] = fsm;
+        }
+    }
+}
+
+// The same step, one thread per cell, for grids of any n = 2^lg (n < 64: too small to march): every
+// neighbour value formed as pin + e, no restriction.
+template <bool UPD, typename Te>
+__global__ void __launch_bounds__(256) k_update_resid_cells(const double *__restrict__ pin, const Te *__restrict__ e,
+                                                            double *__restrict__ pout, const double *__restrict__ f,
+                                                            Te *__restrict__ r0, int lg, double h2i, double *pmax,
+                                                            double *psum, double *fpmax, double *fpsum)
+{
+    const int n = 1 << lg, m = n - 1, c = blockIdx.x * blockDim.x + threadIdx.x;
+    double mx = 0.0, sm = 0.0, fmx = 0.0, fsm = 0.0;
+    if (c < (1 << (3 * lg))) {
+        const int i = c & m, j = (c >> lg) & m, k = c >> (2 * lg);
+        auto P = [&](int ii, int jj, int kk) -> double {
+            const int q = ((kk & m) << (2 * lg)) | ((jj & m) << lg) | (ii & m);
+            return UPD ? pin[q] + (double)e[q] : pin[q];
+        };
+        const double pc = P(i, j, k), fc = f[c];
+        const double rv = resid_value<double>(pc, P(i + 1, j, k), P(i - 1, j, k), P(i, j + 1, k), P(i, j - 1, k),
+                                              P(i, j, k + 1), P(i, j, k - 1), fc, h2i);
+        r0[c] = (Te)rv;
+        if (pout) pout[c] = pc;
+        mx = fabs(rv);
+        sm = rv * rv;
+        fmx = fabs(fc);
+        fsm = fc * fc;
+    }
+    block_max_sum(mx, sm);
+    if (threadIdx.x == 0) {
+        pmax[blockIdx.x] = mx;
+        psum[blockIdx.x] = sm;
+    }
+    if (fpmax) {
+        block_max_sum(fmx, fsm);
+        if (threadIdx.x == 0) {
+            fpmax[blockIdx.x] = fmx;
+            fpsum[blockIdx.x] = fsm;
         }
     }
 }

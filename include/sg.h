@@ -34,7 +34,7 @@ extern "C" {
 #define SG_STOP_TRUE_RESIDUAL 1 /* post-update max|f - L phi| / max|f| < tol, computed in FP64        */
 
 /* Arithmetic of the inner multigrid solve (outer residual and update are always FP64). */
-#define SG_PREC_FP64 1          /* plain: every kernel FP64, one launch per reference loop nest      */
+#define SG_PREC_FP64 1          /* plain: every kernel FP64, the reference's cycle and bits          */
 #define SG_PREC_MIXED 2         /* FP32 smoothing / restriction / prolongation inside FP64 refinement */
 
 /* Coarse-grid solve of the SG_PREC_MIXED inner cycle on the uniform and batched tiers (the FP64
@@ -53,8 +53,9 @@ typedef struct sg_params {
     int precision;    /* SG_PREC_*                                                  */
     int ncycle;       /* V-cycles per FMG level (mg.F90:123, 2)                     */
     int npre, npost;  /* smoothing sweeps (mg.F90:124-125, 2 and 2)                 */
-    int use_graph;    /* SG_PREC_MIXED only: replay the inner cycle as a hipGraph   */
-    int fused;        /* SG_PREC_MIXED only: fused LDS-tiled kernels (same values)  */
+    int use_graph;    /* replay the inner cycle as a hipGraph (AMR: SG_PREC_MIXED)  */
+    int fused;        /* fused LDS-tiled kernels (same values); uniform FP64 with 0: */
+                      /* one eager launch per reference loop nest                   */
     int coarse;       /* SG_PREC_MIXED only: SG_COARSE_* (default SG_COARSE_EXACT)  */
 } sg_params;
 
@@ -347,8 +348,9 @@ int sg_batch_destroy(sg_batch *ctx);
 /* psi[q], src[q]: device pointers to dense n[q]^3 FP64 arrays, i fastest (psi in = initial
  * guess, out = solution).  st[q]: per-problem statistics (ms is the whole batch's).  Stops each
  * problem on max|src - L psi| / max|src| < tol (SG_STOP_TRUE_RESIDUAL only); a converged problem
- * leaves the later launches.  SG_PREC_MIXED: fused FP32 inner solve with tile shapes chosen on the
- * first call; use_graph replays each outer iteration as a hipGraph.  Returns SG_OK when every
+ * leaves the later launches.  The inner solve runs the fused kernels in either precision
+ * (SG_PREC_MIXED: FP32, with tile shapes chosen on the first call); use_graph replays each outer
+ * iteration as a hipGraph.  Returns SG_OK when every
  * problem converged, else the status of a problem that did not. */
 int sg_batch_solve_dev(sg_batch *ctx, double *const *psi, const double *const *src, const sg_params *p,
                        sg_stats *st);

@@ -157,3 +157,22 @@ def test_uneven_48_problem_batch(gpu):
     print("192^3 mixed vs FFT", e, flush=True)
     assert e < 1e-9
     b.close()
+
+
+@pytest.mark.parametrize("sizes", [[96] * 10 + [48, 24, 128], [192, 192, 24, 48], [128, 96, 24], [24, 48, 64], [3, 6, 12, 24]])
+def test_fp64_sweep_shapes_do_not_change_values(gpu, sizes):
+    """The FP64 rule takes another sweep shape (streams of 64 x 16 and 32 x 32, tiles of one and two
+    sweeps) as the cells of a level add up, and the problems of a multiple of 32 apart from the
+    others: every problem equals its batch-of-one solve bit for bit, odd sweep counts included."""
+    for npre, npost in ((2, 2), (3, 1)):
+        srcs = rhs_list(sizes, seed=21)
+        b = BatchSolver(sizes, precisions=SG_PREC_FP64)
+        kw = dict(tol=1e-8, maxit=3, precision=SG_PREC_FP64, npre=npre, npost=npost, raise_on_fail=False)
+        psis, st = b.solve_host(srcs, **kw)
+        b.close()
+        for q in sorted({n: q for q, n in enumerate(sizes)}.values()):
+            one = BatchSolver([sizes[q]], precisions=SG_PREC_FP64)
+            p1, s1 = one.solve_host([srcs[q]], **kw)
+            one.close()
+            assert st[q]["iterations"] == s1[0]["iterations"] and st[q]["rel_linf"] == s1[0]["rel_linf"]
+            assert np.array_equal(psis[q], p1[0]), f"problem {q} (n = {sizes[q]})"

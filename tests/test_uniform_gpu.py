@@ -329,3 +329,29 @@ def test_fused_other_cycle_shapes_bitwise(gpu, npre, npost, ncycle):
     assert torch.equal(res[0][0], res[1][0])
     assert res[0][1]["resmaxg"] == res[1][1]["resmaxg"]
     s.close()
+
+
+@pytest.mark.parametrize("cycle", [(2, 2, 2), (1, 3, 1), (2, 1, 2)])
+@pytest.mark.parametrize("n", [2, 4, 8, 16, 32, 64, 128, 256])
+def test_fp64_fused_equals_plain(n, cycle, gpu):
+    """The fused FP64 solve (k_coarse below 16^3, every sweep shape of the rule: tiles of two sweeps at
+    32 and 64, a tile at 128, streams at 256; odd sweep counts) against one kernel per loop nest,
+    bit for bit, in both stopping modes, and again with other phi and source arrays (the graph is
+    the context's own)."""
+    import torch
+    s = UniformSolver(n, 1.0 / n, precisions=SG_PREC_FP64)
+    try:
+        for seed, stop in ((3, SG_STOP_TRUE_RESIDUAL), (4, SG_STOP_REFERENCE), (5, SG_STOP_TRUE_RESIDUAL)):
+            f = torch.tensor(problems.clumpy_rhs(n, seed=seed), device=gpu)
+            out = []
+            for fused in (True, False):
+                psi = torch.zeros_like(f)
+                st = s.cycle(psi, f, tol=1e-9, maxit=4, stop_mode=stop, precision=SG_PREC_FP64, ncycle=cycle[0],
+                             npre=cycle[1], npost=cycle[2], fused=fused, raise_on_fail=False)
+                out.append((psi, st))
+            (a, sa), (b, sb) = out
+            assert torch.equal(a, b)
+            assert sa["iterations"] == sb["iterations"] and sa["rel_linf"] == sb["rel_linf"]
+            assert sa["resmaxg"] == sb["resmaxg"] if stop == SG_STOP_REFERENCE else True
+    finally:
+        s.close()
