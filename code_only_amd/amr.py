@@ -87,13 +87,14 @@ class AmrSolver:
         return out
 
     def set_base_solver(self, chip):
-        """Base-grid mg_cycle of the plain FP64 solve, and the mixed solve's exact base solve, spread
-        over the chip (True, default) or in one workgroup (False); the values are the same."""
+        """Base-grid mg_cycle of the plain FP64 solve on the fused kernels (True, default) or the
+        reference's steps in one workgroup (False), and the mixed solve's exact base solve spread
+        over the chip or in one workgroup; the values are the same."""
         _lib.check(self._lib.sg_amr_set_base_solver(self._ctx, 1 if chip else 0))
 
     def set_fp64_refresh(self, fused):
-        """Plain FP64 solve with the staged refresh of the reference (False, default) or the mixed
-        solve's fused launch structure (True); the values are the same."""
+        """Plain FP64 solve with the mixed solve's fused launch structure (True, default) or the staged
+        refresh of the reference (False); the values are the same."""
         _lib.check(self._lib.sg_amr_set_fp64_refresh(self._ctx, 1 if fused else 0))
 
     def time_smoother(self, precision=SG_PREC_MIXED, reps=20):

@@ -16,6 +16,9 @@
 //    the coarse level's u in the same step;
 //  * the tricubic prolongation into 8^3 and larger runs as three separable passes with its weights
 //    tabulated once per launch.
+// Boundaries: periodic (ZERO false), or zero ghosts (ZERO: mg_boundary_fill0, with mg_boundary_extrap's
+// odd continuation, (-1)^g times the clamped interior cell for g ghost coordinates, before a
+// prolongation; mg.F90:735-771).
 // Per-cell values come from relax_value, resid_value, restrict_value, trilinear_value and cubic4 in the
 // order of the one-kernel-per-loop kernels, so both give the same bits.
 #pragma once
@@ -145,7 +148,7 @@ template <bool WAVE> struct CoarseTeam {
 };
 
 // one mg_relax call (mg_poisson.F90:55-74); a 1^3 level's cell belongs to the second pass
-template <typename T, int N, bool WAVE>
+template <typename T, int N, bool WAVE, bool ZERO>
 __device__ __forceinline__ void coarse_relax(CoarseLds<T> &S, T h2, double *resmax)
 {
     using C = CoarseTeam<WAVE>;
@@ -155,7 +158,10 @@ __device__ __forceinline__ void coarse_relax(CoarseLds<T> &S, T h2, double *resm
     double amax = 0.0;
     T s;
     if constexpr (N == 1) {
-        if (threadIdx.x == 0) u[0] = relax_value<T>(u[0], u[0], u[0], u[0], u[0], u[0], u[0], f[0], h2, &s);
+        if (threadIdx.x == 0) {
+            const T g = ZERO ? T(0) : u[0];
+            u[0] = relax_value<T>(u[0], g, g, g, g, g, g, f[0], h2, &s);
+        }
         C::sync();
         return;
     } else {
@@ -174,9 +180,16 @@ __device__ __forceinline__ void coarse_relax(CoarseLds<T> &S, T h2, double *resm
                     const int side = odd ? (ih + 1 == nh ? t + 1 - nh : t + 1) : (ih == 0 ? t + nh - 1 : t - 1);
                     const int yp = j + 1 == N ? t + nh - pl : t + nh, ym = j == 0 ? t - nh + pl : t - nh;
                     const int zp = k + 1 == N ? t + pl - half : t + pl, zm = k == 0 ? t - pl + half : t - pl;
-                    const T a = oth[t], b = oth[side];
-                    own[t] = relax_value<T>(own[t], odd ? b : a, odd ? a : b, oth[yp], oth[ym], oth[zp], oth[zm], fo[t],
-                                            h2, &s);
+                    const T a = oth[t];
+                    T b = oth[side], vyp = oth[yp], vym = oth[ym], vzp = oth[zp], vzm = oth[zm];
+                    if (ZERO) {
+                        if (odd ? ih + 1 == nh : ih == 0) b = T(0);
+                        if (j + 1 == N) vyp = T(0);
+                        if (j == 0) vym = T(0);
+                        if (k + 1 == N) vzp = T(0);
+                        if (k == 0) vzm = T(0);
+                    }
+                    own[t] = relax_value<T>(own[t], odd ? b : a, odd ? a : b, vyp, vym, vzp, vzm, fo[t], h2, &s);
                     amax = fmax(amax, fabs((double)s));
                 }
             }
@@ -195,7 +208,8 @@ __device__ __forceinline__ void coarse_relax(CoarseLds<T> &S, T h2, double *resm
 
 // residual of the level of width N (mg_poisson.F90:17-27) restricted into the next one's right-hand
 // side (restriction.F90:132-147), whose u is zeroed
-template <typename T, int N, bool WAVE> __device__ __forceinline__ void coarse_resid_restrict(CoarseLds<T> &S, T h2i)
+template <typename T, int N, bool WAVE, bool ZERO>
+__device__ __forceinline__ void coarse_resid_restrict(CoarseLds<T> &S, T h2i)
 {
     using C = CoarseTeam<WAVE>;
     using L = CoarseLevel<N>;
@@ -219,6 +233,11 @@ template <typename T, int N, bool WAVE> __device__ __forceinline__ void coarse_r
                 xo[o] = u[L::at(a ? ip : im, j + b, k + d)];
                 yo[o] = u[L::at(i + a, b ? jp : jm, k + d)];
                 zo[o] = u[L::at(i + a, j + b, d ? kp : km)];
+                if (ZERO) {
+                    if (a ? i + 2 == N : i == 0) xo[o] = T(0);
+                    if (b ? j + 2 == N : j == 0) yo[o] = T(0);
+                    if (d ? k + 2 == N : k == 0) zo[o] = T(0);
+                }
             }
             T r[8];
 #pragma unroll
@@ -256,9 +275,18 @@ template <typename T, int N, bool WAVE> __device__ __forceinline__ void coarse_r
     C::sync();
 }
 
+// interior cell and factor that coarse index c (-1 .. n) stands for
+template <typename T, bool ZERO> __device__ __forceinline__ int coarse_ghost(int c, int n, T &sign)
+{
+    sign = T(1);
+    if (!ZERO) return wrap_g(c, n);
+    if (c < 0 || c >= n) sign = T(-1);
+    return c < 0 ? 0 : (c >= n ? n - 1 : c);
+}
+
 // trilinear prolongation into the level of width N (interpolation.F90:226-245), added to u
 // (mg_addint) or stored
-template <typename T, int N, bool WAVE, bool ADD> __device__ __forceinline__ void coarse_linear(CoarseLds<T> &S)
+template <typename T, int N, bool WAVE, bool ADD, bool ZERO> __device__ __forceinline__ void coarse_linear(CoarseLds<T> &S)
 {
     using C = CoarseTeam<WAVE>;
     using L = CoarseLevel<N>;
@@ -272,11 +300,22 @@ template <typename T, int N, bool WAVE, bool ADD> __device__ __forceinline__ voi
             const int p = q / L::half, h = q % L::half;
             const int ic = h % nc, j = (h / nc) % N, k = h / L::pl, i = 2 * ic + ((j + k + p) & 1);
             const int jc = j >> 1, kc = k >> 1;
-            const int ic1 = wrap_g(ic + 2 * (i & 1) - 1, nc), jc1 = wrap_g(jc + 2 * (j & 1) - 1, nc),
-                      kc1 = wrap_g(kc + 2 * (k & 1) - 1, nc);
+            T sx, sy, sz;
+            const int ic1 = coarse_ghost<T, ZERO>(ic + 2 * (i & 1) - 1, nc, sx), jc1 = coarse_ghost<T, ZERO>(jc + 2 * (j & 1) - 1, nc, sy),
+                      kc1 = coarse_ghost<T, ZERO>(kc + 2 * (k & 1) - 1, nc, sz);
             auto V = [&](int a, int b, int d) { return S.u[K::off + K::at(a, b, d)]; };
-            const T v = trilinear_value<T>(V(ic, jc, kc), V(ic1, jc, kc), V(ic, jc1, kc), V(ic, jc, kc1),
-                                           V(ic, jc1, kc1), V(ic1, jc, kc1), V(ic1, jc1, kc), V(ic1, jc1, kc1));
+            T c[8] = {V(ic, jc, kc), V(ic1, jc, kc), V(ic, jc1, kc), V(ic, jc, kc1),
+                      V(ic, jc1, kc1), V(ic1, jc, kc1), V(ic1, jc1, kc), V(ic1, jc1, kc1)};
+            if (ZERO) {
+                c[1] = sx * c[1];
+                c[2] = sy * c[2];
+                c[3] = sz * c[3];
+                c[4] = (sy * sz) * c[4];
+                c[5] = (sx * sz) * c[5];
+                c[6] = (sx * sy) * c[6];
+                c[7] = (sx * sy * sz) * c[7];
+            }
+            const T v = trilinear_value<T>(c[0], c[1], c[2], c[3], c[4], c[5], c[6], c[7]);
             T &w = S.u[L::off + q];
             w = ADD ? w + v : v;
         }
@@ -286,14 +325,14 @@ template <typename T, int N, bool WAVE, bool ADD> __device__ __forceinline__ voi
 
 // FMG prolongation into the level of width N (mg.F90:608-633): tricubic, trilinear where the coarse
 // grid with ghosts is narrower than 4
-template <typename T, int N, bool WAVE> __device__ __forceinline__ void coarse_fmg_interp(CoarseLds<T> &S)
+template <typename T, int N, bool WAVE, bool ZERO> __device__ __forceinline__ void coarse_fmg_interp(CoarseLds<T> &S)
 {
     using C = CoarseTeam<WAVE>;
     using L = CoarseLevel<N>;
     using K = CoarseLevel<N / 2>;
     constexpr int nc = N / 2;
     if constexpr (nc + 2 < 4) {
-        coarse_linear<T, N, WAVE, false>(S);
+        coarse_linear<T, N, WAVE, false, ZERO>(S);
         return;
     } else {
         const T(*tw)[4] = S.tw + L::tab;
@@ -347,59 +386,59 @@ template <typename T, int N, bool WAVE> __device__ __forceinline__ void coarse_f
 // One V-cycle from the level of width N (depth D below the first held one) down and back.  Levels of
 // <= kWaveLevelN run in wavefront 0 (WAVE); the workgroup meets it at a barrier.  mg_slvsml
 // (mg.F90:540-546) at the bottom: two sweeps of a 1^3 level, the exact solve of a 3^3 one.
-template <typename T, int N, int D, bool WAVE>
+template <typename T, int N, int D, bool WAVE, bool ZERO>
 __device__ __forceinline__ void coarse_cycle(CoarseLds<T> &S, const CoarseCoef<T> &P, int npre, int npost, double *resmax)
 {
     static_assert(WAVE == (N <= kWaveLevelN), "levels of <= kWaveLevelN run in one wavefront");
     if constexpr (N == 1) {
-        for (int it = 0; it < 2; ++it) coarse_relax<T, 1, true>(S, P.h2[D], nullptr);
+        for (int it = 0; it < 2; ++it) coarse_relax<T, 1, true, ZERO>(S, P.h2[D], nullptr);
     } else if constexpr (N == 3) {
         if (threadIdx.x == 0) exact3<T>(S.u + CoarseLevel<3>::off, S.r + CoarseLevel<3>::off, P.q3, P.lam3);
         CoarseTeam<true>::sync();
     } else {
-        for (int p = 0; p < npre; ++p) coarse_relax<T, N, WAVE>(S, P.h2[D], nullptr);
-        coarse_resid_restrict<T, N, WAVE>(S, P.h2i[D]);
+        for (int p = 0; p < npre; ++p) coarse_relax<T, N, WAVE, ZERO>(S, P.h2[D], nullptr);
+        coarse_resid_restrict<T, N, WAVE, ZERO>(S, P.h2i[D]);
         constexpr int M = coarse_below(N);
         constexpr bool MW = M <= kWaveLevelN;
         if constexpr (MW && !WAVE) {
-            if (threadIdx.x < kWave) coarse_cycle<T, M, D + 1, true>(S, P, npre, npost, nullptr);
+            if (threadIdx.x < kWave) coarse_cycle<T, M, D + 1, true, ZERO>(S, P, npre, npost, nullptr);
             __syncthreads();
         } else {
-            coarse_cycle<T, M, D + 1, MW>(S, P, npre, npost, nullptr);
+            coarse_cycle<T, M, D + 1, MW, ZERO>(S, P, npre, npost, nullptr);
         }
-        coarse_linear<T, N, WAVE, true>(S);
-        for (int p = 0; p < npost; ++p) coarse_relax<T, N, WAVE>(S, P.h2[D], p == npost - 1 ? resmax : nullptr);
+        coarse_linear<T, N, WAVE, true, ZERO>(S);
+        for (int p = 0; p < npost; ++p) coarse_relax<T, N, WAVE, ZERO>(S, P.h2[D], p == npost - 1 ? resmax : nullptr);
     }
 }
 
 // FMG from the coarsest level up to the level of width N (mg.F90:142-215)
-template <typename T, int N, int D, bool WAVE>
+template <typename T, int N, int D, bool WAVE, bool ZERO>
 __device__ __forceinline__ void coarse_fmg(CoarseLds<T> &S, const CoarseCoef<T> &P, int ncycle, int npre, int npost,
                                            double *resmax)
 {
     if constexpr (N == 1 || N == 3) {
         if (threadIdx.x < N * N * N) S.u[CoarseLevel<N>::off + threadIdx.x] = T(0);
         CoarseTeam<true>::sync();
-        coarse_cycle<T, N, D, true>(S, P, npre, npost, nullptr);
+        coarse_cycle<T, N, D, true, ZERO>(S, P, npre, npost, nullptr);
     } else {
         constexpr int M = coarse_below(N);
         constexpr bool MW = M <= kWaveLevelN;
         coarse_restrict<T, N, WAVE>(S);
         if constexpr (MW && !WAVE) {
-            if (threadIdx.x < kWave) coarse_fmg<T, M, D + 1, true>(S, P, ncycle, npre, npost, nullptr);
+            if (threadIdx.x < kWave) coarse_fmg<T, M, D + 1, true, ZERO>(S, P, ncycle, npre, npost, nullptr);
             __syncthreads();
         } else {
-            coarse_fmg<T, M, D + 1, MW>(S, P, ncycle, npre, npost, nullptr);
+            coarse_fmg<T, M, D + 1, MW, ZERO>(S, P, ncycle, npre, npost, nullptr);
         }
-        coarse_fmg_interp<T, N, WAVE>(S);
+        coarse_fmg_interp<T, N, WAVE, ZERO>(S);
         for (int jc = 0; jc < ncycle; ++jc)
-            coarse_cycle<T, N, D, WAVE>(S, P, npre, npost, jc == ncycle - 1 ? resmax : nullptr);
+            coarse_cycle<T, N, D, WAVE, ZERO>(S, P, npre, npost, jc == ncycle - 1 ? resmax : nullptr);
     }
 }
 
 // tricubic stencils of the levels from width N whose coarse grid is wide enough, one fine index per
-// lane (q)
-template <typename T, int N> __device__ __forceinline__ void coarse_tables(CoarseLds<T> &S, int q)
+// lane (q).  A ghost cell's factor goes into its weight: w (-v) = (-w) v in every operation.
+template <typename T, int N, bool ZERO> __device__ __forceinline__ void coarse_tables(CoarseLds<T> &S, int q)
 {
     constexpr int M = coarse_below(N);
     if constexpr (M >= 2) {
@@ -409,11 +448,12 @@ template <typename T, int N> __device__ __forceinline__ void coarse_tables(Coars
             double a[4];
             cubic_stencil(f, -1, M, idx, a);
             for (int e = 0; e < 4; ++e) {
-                S.ti[q][e] = wrap_g(idx[e], M);
-                S.tw[q][e] = (T)a[e];
+                T sign;
+                S.ti[q][e] = coarse_ghost<T, ZERO>(idx[e], M, sign);
+                S.tw[q][e] = sign * (T)a[e];
             }
         }
-        coarse_tables<T, M>(S, q);
+        coarse_tables<T, M, ZERO>(S, q);
     }
 }
 
@@ -421,7 +461,7 @@ template <typename T, int N> __device__ __forceinline__ void coarse_tables(Coars
 // them); mode 1: one V-cycle from it with zero initial guess (mg.F90:179-210).  rhs_in, u_out: dense
 // N^3 arrays.  resmax receives max|resh2| of the last smoothing of the first level when non-null.
 // Every thread of a kCoarseThreads workgroup calls it.
-template <typename T, int N>
+template <typename T, int N, bool ZERO = false>
 __device__ __forceinline__ void coarse_solve(CoarseLds<T> &S, const CoarseCoef<T> &P, const T *__restrict__ rhs_in,
                                              T *__restrict__ u_out, int mode, int ncycle, int npre, int npost,
                                              double *resmax)
@@ -435,11 +475,11 @@ __device__ __forceinline__ void coarse_solve(CoarseLds<T> &S, const CoarseCoef<T
         S.r[d] = rhs_in[c];
         if (mode == 1) S.u[d] = T(0);
     }
-    if (mode == 0 && threadIdx.x >= kCoarseThreads - 64) coarse_tables<T, N>(S, (int)threadIdx.x - (kCoarseThreads - 64));
+    if (mode == 0 && threadIdx.x >= kCoarseThreads - 64) coarse_tables<T, N, ZERO>(S, (int)threadIdx.x - (kCoarseThreads - 64));
     __syncthreads();
     if (!W || threadIdx.x < kWave) {
-        if (mode == 0) coarse_fmg<T, N, 0, W>(S, P, ncycle, npre, npost, resmax);
-        else coarse_cycle<T, N, 0, W>(S, P, npre, npost, resmax);
+        if (mode == 0) coarse_fmg<T, N, 0, W, ZERO>(S, P, ncycle, npre, npost, resmax);
+        else coarse_cycle<T, N, 0, W, ZERO>(S, P, npre, npost, resmax);
     }
     if (W) __syncthreads();
     for (int c = threadIdx.x; c < L::len; c += kCoarseThreads) {

@@ -67,7 +67,7 @@ inline bool tile_fits(int cfg, int n)
 // One colour of the sweep over the LDS region shrunk by margin M: cells with
 // (gx + gy + gz) % 2 == colour, where colour 1 is the reference's first pass (ipass = 1).  The
 // source values are fetched for all of a thread's cells before any update.
-template <class TL, int LX, int LY, int LZ, int M, int H, bool FS, typename T>
+template <class TL, int LX, int LY, int LZ, int M, int H, bool FS, typename T, bool ZB>
 __device__ __forceinline__ void tile_colour(T *su, const T *sf, const T *__restrict__ f, int n, int x0,
                                             int y0, int z0, int colour, T h2, double &amax)
 {
@@ -91,6 +91,11 @@ __device__ __forceinline__ void tile_colour(T *su, const T *sf, const T *__restr
             const int d = (colour + x0 + M + y0 + y + z0 + z) & 1;
             const int x = M + 2 * xh + d;
             cv[it] = (z * LY + y) * LX + x;
+            if (ZB && ((unsigned)(x0 + x) >= (unsigned)n || (unsigned)(y0 + y) >= (unsigned)n ||
+                       (unsigned)(z0 + z) >= (unsigned)n)) {
+                cv[it] = -1;
+                continue;
+            }
             if (x >= H && x < H + TL::TX && y >= H && y < H + TL::TY && z >= H && z < H + TL::TZ) core |= 1u << it;
             if (FS) {
                 fv[it] = sf[cv[it]];
@@ -114,21 +119,21 @@ __device__ __forceinline__ void tile_colour(T *su, const T *sf, const T *__restr
 
 // Sweeps S .. NS-1 of a multi-sweep tile: sweep s updates the first colour on margin 2s+1 and the
 // second on margin 2s+2.  Only the last sweep feeds the max|resh2| (one mg_relax call's Resmaxg).
-template <class TL, int LX, int LY, int LZ, int H, int S, int NS, bool FS, typename T> struct TileSweeps {
+template <class TL, int LX, int LY, int LZ, int H, int S, int NS, bool FS, typename T, bool ZB> struct TileSweeps {
     static __device__ __forceinline__ void run(T *su, const T *sf, const T *__restrict__ f, int n, int x0,
                                                int y0, int z0, T h2, double &amax)
     {
         double dummy = 0.0;
         double &acc = (S == NS - 1) ? amax : dummy;
-        tile_colour<TL, LX, LY, LZ, 2 * S + 1, H, FS, T>(su, sf, f, n, x0, y0, z0, 1, h2, acc);
+        tile_colour<TL, LX, LY, LZ, 2 * S + 1, H, FS, T, ZB>(su, sf, f, n, x0, y0, z0, 1, h2, acc);
         __syncthreads();
-        tile_colour<TL, LX, LY, LZ, 2 * S + 2, H, FS, T>(su, sf, f, n, x0, y0, z0, 0, h2, acc);
+        tile_colour<TL, LX, LY, LZ, 2 * S + 2, H, FS, T, ZB>(su, sf, f, n, x0, y0, z0, 0, h2, acc);
         __syncthreads();
-        TileSweeps<TL, LX, LY, LZ, H, S + 1, NS, FS, T>::run(su, sf, f, n, x0, y0, z0, h2, amax);
+        TileSweeps<TL, LX, LY, LZ, H, S + 1, NS, FS, T, ZB>::run(su, sf, f, n, x0, y0, z0, h2, amax);
     }
 };
-template <class TL, int LX, int LY, int LZ, int H, int NS, bool FS, typename T>
-struct TileSweeps<TL, LX, LY, LZ, H, NS, NS, FS, T> {
+template <class TL, int LX, int LY, int LZ, int H, int NS, bool FS, typename T, bool ZB>
+struct TileSweeps<TL, LX, LY, LZ, H, NS, NS, FS, T, ZB> {
     static __device__ __forceinline__ void run(T *, const T *, const T *__restrict__, int, int, int, int, T, double &)
     {
     }
@@ -153,8 +158,10 @@ template <class TL, int NS, bool FS, typename T = float> constexpr bool sweep_fi
 // NS full sweeps (temporal blocking: halo 2 per sweep, +1 for the residual).  FS stages the source
 // on the same LDS region as u, loaded together with u, so the colour passes touch LDS only.
 // Body of the fused sweep for tile t of an n^3 level (n even, divisible by the tile extents);
-// called by every thread of a workgroup with the same t.
-template <class TL, int NS, bool ZERO, bool PROLONG, bool RESID, bool FS, typename T = float>
+// called by every thread of a workgroup with the same t.  ZB: zero ghosts instead of periodic ones
+// (coarse_levels.h): cells outside the grid hold zero and are never updated, a coarse cell outside
+// its grid is the odd continuation.
+template <class TL, int NS, bool ZERO, bool PROLONG, bool RESID, bool FS, typename T = float, bool ZB = false>
 __device__ __forceinline__ void sweep_tile(const T *__restrict__ uin, T *__restrict__ uout,
                                            const T *__restrict__ f, int n, T h2, T h2i,
                                            const T *__restrict__ uc, T *__restrict__ rc, double *resmax, int t)
@@ -189,6 +196,9 @@ __device__ __forceinline__ void sweep_tile(const T *__restrict__ uin, T *__restr
                     const int x = q % LX, y = (q / LX) % LY, z = q / (LX * LY);
                     const int g = (wrapn(z0 + z, n) * n + wrapn(y0 + y, n)) * n + wrapn(x0 + x, n);
                     if (!ZERO) v[it] = uin[g];
+                    if (!ZERO && ZB && ((unsigned)(x0 + x) >= (unsigned)n || (unsigned)(y0 + y) >= (unsigned)n ||
+                                        (unsigned)(z0 + z) >= (unsigned)n))
+                        v[it] = T(0);
                     if (FS) fvl[FS ? it : 0] = f[g];
                 }
             }
@@ -200,7 +210,11 @@ __device__ __forceinline__ void sweep_tile(const T *__restrict__ uin, T *__restr
                 const int q = threadIdx.x + it * NT;
                 if (CNTC % NT == 0 || q < CNTC) {
                     const int x = q % CX, y = (q / CX) % CY, z = q / (CX * CY);
-                    cvl[it] = uc[(wrapn(cz0 + z, nc) * nc + wrapn(cy0 + y, nc)) * nc + wrapn(cx0 + x, nc)];
+                    T sx, sy, sz;
+                    const int a = coarse_ghost<T, ZB>(cx0 + x, nc, sx), b = coarse_ghost<T, ZB>(cy0 + y, nc, sy),
+                              d = coarse_ghost<T, ZB>(cz0 + z, nc, sz);
+                    cvl[it] = uc[(d * nc + b) * nc + a];
+                    if (ZB) cvl[it] = (sx * sy * sz) * cvl[it];
                 }
             }
 #pragma unroll
@@ -231,6 +245,9 @@ __device__ __forceinline__ void sweep_tile(const T *__restrict__ uin, T *__restr
                 const int ic = (x >> 1) + 1, jc = (y >> 1) + 1, kc = (z >> 1) + 1;
                 const int ic1 = ic + 2 * (x & 1) - 1, jc1 = jc + 2 * (y & 1) - 1, kc1 = kc + 2 * (z & 1) - 1;
                 auto C = [&](int a, int b, int d) { return sc[(d * CY + b) * CX + a]; };
+                if (ZB && ((unsigned)(x0 + x) >= (unsigned)n || (unsigned)(y0 + y) >= (unsigned)n ||
+                           (unsigned)(z0 + z) >= (unsigned)n))
+                    continue;
                 su[q] = su[q] + trilinear_value<T>(C(ic, jc, kc), C(ic1, jc, kc), C(ic, jc1, kc), C(ic, jc, kc1),
                                                        C(ic, jc1, kc1), C(ic1, jc, kc1), C(ic1, jc1, kc),
                                                        C(ic1, jc1, kc1));
@@ -239,7 +256,7 @@ __device__ __forceinline__ void sweep_tile(const T *__restrict__ uin, T *__restr
         __syncthreads();
     }
     double amax = 0.0;
-    TileSweeps<TL, LX, LY, LZ, H, 0, NS, FS, T>::run(su, sf, f, n, x0, y0, z0, h2, amax);
+    TileSweeps<TL, LX, LY, LZ, H, 0, NS, FS, T, ZB>::run(su, sf, f, n, x0, y0, z0, h2, amax);
     {
         constexpr int CNT = TX * TY * TZ, IT = (CNT + NT - 1) / NT;
 #pragma unroll
@@ -297,7 +314,7 @@ __device__ __forceinline__ void sweep_tile(const T *__restrict__ uin, T *__restr
     if (resmax) block_atomic_max(resmax, amax);
 }
 
-template <class TL, int NS, bool ZERO, bool PROLONG, bool RESID, bool FS, typename T = float>
+template <class TL, int NS, bool ZERO, bool PROLONG, bool RESID, bool FS, typename T = float, bool ZB = false>
 __global__ void __launch_bounds__(TL::NT)
 k_sweep_tile(const T *__restrict__ uin, T *__restrict__ uout, const T *__restrict__ f, int n, T h2,
              T h2i, const T *__restrict__ uc, T *__restrict__ rc, double *resmax)
@@ -305,7 +322,7 @@ k_sweep_tile(const T *__restrict__ uin, T *__restrict__ uout, const T *__restric
     const int ntiles = (n / TL::TX) * (n / TL::TY) * (n / TL::TZ);
     const int t = xcd_tile(ntiles);
     if (t >= ntiles) return;  // uniform per workgroup, before any barrier
-    sweep_tile<TL, NS, ZERO, PROLONG, RESID, FS, T>(uin, uout, f, n, h2, h2i, uc, rc, resmax, t);
+    sweep_tile<TL, NS, ZERO, PROLONG, RESID, FS, T, ZB>(uin, uout, f, n, h2, h2i, uc, rc, resmax, t);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -772,7 +789,7 @@ inline void cand_decode(int cand, int &cfg, int &ns, bool &fs)
 // as the reference's bufx / bufxy sweeps.  Fine tile FX*FY*FZ, nf >= FX, nf % FY == nf % FZ == 0.
 // T = float (mixed path) or double (plain path): the weights are rounded to T as k_interp_cubic
 // rounds them, and every value is formed in the same operand order, so both give its results.
-template <int FX, int FY, int FZ, int NT, typename T = float>
+template <int FX, int FY, int FZ, int NT, typename T = float, bool ZB = false>
 __device__ __forceinline__ void interp_cubic_tile(T *__restrict__ uf, const T *__restrict__ uc, int nf, int t)
 {
     constexpr int CX = FX / 2 + 4, CY = FY / 2 + 4, CZ = FZ / 2 + 4;
@@ -792,7 +809,11 @@ __device__ __forceinline__ void interp_cubic_tile(T *__restrict__ uf, const T *_
             const int q = threadIdx.x + it * NT;
             if (CNT % NT == 0 || q < CNT) {
                 const int x = q % CX, y = (q / CX) % CY, z = q / (CX * CY);
-                v[it] = uc[(wrapn(bzo + z, nc) * nc + wrapn(byo + y, nc)) * nc + wrapn(bxo + x, nc)];
+                T sx, sy, sz;
+                const int a = coarse_ghost<T, ZB>(bxo + x, nc, sx), b = coarse_ghost<T, ZB>(byo + y, nc, sy),
+                          d = coarse_ghost<T, ZB>(bzo + z, nc, sz);
+                v[it] = uc[(d * nc + b) * nc + a];
+                if (ZB) v[it] = (sx * sy * sz) * v[it];
             }
         }
 #pragma unroll
@@ -845,26 +866,26 @@ __device__ __forceinline__ void interp_cubic_tile(T *__restrict__ uf, const T *_
     }
 }
 
-template <int FX, int FY, int FZ, int NT, typename T = float>
+template <int FX, int FY, int FZ, int NT, typename T = float, bool ZB = false>
 __global__ void __launch_bounds__(NT) k_interp_cubic_tile(T *__restrict__ uf, const T *__restrict__ uc, int nf)
 {
     const int ntiles = (nf / FX) * (nf / FY) * (nf / FZ);
     const int t = xcd_tile(ntiles);
     if (t >= ntiles) return;
-    interp_cubic_tile<FX, FY, FZ, NT, T>(uf, uc, nf, t);
+    interp_cubic_tile<FX, FY, FZ, NT, T, ZB>(uf, uc, nf, t);
 }
 
 // ------------------------------------------------------------------------------------------------
 // Single-workgroup solvers of the first level of <= 16^3 cells: the reference's cycles from there down
 // (coarse_levels.h), or its exact solve.
 // ------------------------------------------------------------------------------------------------
-template <typename T, int N>
+template <typename T, int N, bool ZERO = false>
 __global__ void __launch_bounds__(kCoarseThreads)
 k_coarse(const T *__restrict__ rhs_in, T *__restrict__ u_out, CoarseCoef<T> P, int mode, int ncycle, int npre, int npost,
          double *resmax)
 {
     __shared__ CoarseLds<T> S;
-    coarse_solve<T, N>(S, P, rhs_in, u_out, mode, ncycle, npre, npost, resmax);
+    coarse_solve<T, N, ZERO>(S, P, rhs_in, u_out, mode, ncycle, npre, npost, resmax);
 }
 
 struct CoarseExact {

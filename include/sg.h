@@ -222,16 +222,16 @@ int sg_amr_info(sg_amr *ctx, int *info, int n);
  * where not yet timed: the FP32 ones are timed at the first mixed-precision solve). */
 int sg_amr_tile_info(sg_amr *ctx, int which, int *choice, float *ms, int nms);
 /* How the plain FP64 solve runs the base grid's mg_cycle (vmg_slvsml -> mg_cycle, vmg.F90:387-432):
- * chip = 1 (default) the finest base level's steps as multi-workgroup launches and the coarser
- * levels' stretches in one workgroup each; chip = 0 the whole mg_cycle in one workgroup.  The
- * mixed solve's exact base solve likewise: six multi-workgroup transform passes, or one workgroup.
- * Same values either way. */
+ * chip = 1 (default) the fused kernels of the uniform tier (base grids of up to 16^3 cells: the whole
+ * mg_cycle with its stopping test in one launch); chip = 0 the reference's steps on ghosted arrays in
+ * one workgroup.  The mixed solve's exact base solve: six multi-workgroup transform passes, or one
+ * workgroup.  Same values either way. */
 int sg_amr_set_base_solver(sg_amr *ctx, int chip);
-/* How the plain FP64 solve refreshes ghosts (no reference counterpart): fused = 0 (default) the
- * reference's staged sequence (c2p, fmg_ghostcell_fix level by level and direction by direction,
- * reflux) before every colour pass; fused = 1 the mixed solve's launch structure in FP64 -- one
- * table-driven refresh per pass, halo-free colour passes, merged VMG steps -- with the same values
- * (so that the mixed solve's speed-up over it is the part that precision buys). */
+/* How the plain FP64 solve refreshes ghosts (no reference counterpart): fused = 1 (default) the mixed
+ * solve's launch structure in FP64 -- one table-driven refresh per pass, halo-free colour passes,
+ * merged VMG steps, fmg_lin replayed as graphs (use_graph); fused = 0 the reference's staged sequence
+ * (c2p, fmg_ghostcell_fix level by level and direction by direction, reflux) before every colour pass,
+ * launched eagerly.  Same values either way. */
 int sg_amr_set_fp64_refresh(sg_amr *ctx, int fused);
 /* Adjoint of the sphere-boundary AMR solve (no reference counterpart: the reference has no
  * derivatives).  The converged solve maps the source linearly to the potential: the source's

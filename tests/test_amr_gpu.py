@@ -570,3 +570,54 @@ def test_fp64_fused_refresh_equals_staged(which, gpu):
         assert np.array_equal(ps, pf) and np.array_equal(gs, gf)
     finally:
         g.close()
+
+
+@pytest.mark.parametrize("bc", [ah.PERIODIC, ah.SPHERE])
+@pytest.mark.parametrize("base", [1, 2, 4, 8, 16, 32])
+def test_base_cycle_widths(base, bc, gpu):
+    """The base-grid mg_cycle on the fused kernels against the one-workgroup form, bit for bit, for every
+    width it dispatches on (2^3 ... 16^3 in one launch, 32^3 and 64^3 over the chip), both boundaries."""
+    refine = [] if base < 4 else [{(1, 1, 1), (2, 1, 1)}]
+    if base == 1 and bc == ah.PERIODIC:
+        refine = []
+    h = ah.build((base,) * 3, refine, bc=bc)
+    src = problems.amr_source(h, seed=5)
+    out = []
+    g = AmrSolver(h)
+    try:
+        for chip in (True, False):
+            g.set_base_solver(chip)
+            out.append(g.solve_host(src, tol=1e-8, maxit=3, raise_on_fail=False))
+    finally:
+        g.close()
+    assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
+    assert out[0][2]["hist"] == out[1][2]["hist"]
+
+
+@pytest.mark.parametrize("which", ["nested-sphere-8", "nested-sphere-16", "random-periodic", "random-sphere"])
+def test_fp64_default_equals_staged(which, gpu):
+    """The plain FP64 solve's default (fused refresh, fmg_lin replayed as graphs: one, or stretches
+    between base solves at a 32^3 base grid) against the reference's staged sequence, bit for bit: as
+    recorded and replayed, eagerly, with another source, and after the settings a graph holds changed."""
+    h = {"nested-sphere-8": lambda: ah.nested(base=8, levels=3, bc=ah.SPHERE),
+         "nested-sphere-16": lambda: ah.nested(base=16, levels=2, bc=ah.SPHERE),
+         "random-periodic": lambda: ah.random_hierarchy(4, 3, 0.35, seed=7, bc=ah.PERIODIC),
+         "random-sphere": lambda: ah.random_hierarchy(4, 3, 0.35, seed=3, bc=ah.SPHERE)}[which]()
+    g = AmrSolver(h)
+    kw = dict(tol=1e-9, maxit=4, raise_on_fail=False)
+    try:
+        for seed in (41, 42):
+            src = problems.amr_source(h, seed=seed)
+            g.set_fp64_refresh(False)
+            ref = g.solve_host(src, **kw)
+            g.set_fp64_refresh(True)
+            runs = [g.solve_host(src, **kw), g.solve_host(src, use_graph=False, **kw)]
+            g.set_base_solver(False)
+            runs.append(g.solve_host(src, **kw))
+            g.set_base_solver(True)
+            runs.append(g.solve_host(src, **kw))
+            for psi, acc, st in runs:
+                assert st["hist"] == ref[2]["hist"] and st["resmaxg"] == ref[2]["resmaxg"]
+                assert np.array_equal(psi, ref[0]) and np.array_equal(acc, ref[1])
+    finally:
+        g.close()
