@@ -31,7 +31,6 @@ k_base_small(double *Au, const double *__restrict__ Arhs, const int *__restrict_
              double tol, int maxit)
 {
     using L = CoarseLevel<N>;
-    constexpr bool W = N <= kWaveLevelN;
     constexpr int IT = (L::len + kCoarseThreads - 1) / kCoarseThreads;
     __shared__ CoarseLds<double> S;
     __shared__ double psi[L::len];
@@ -76,7 +75,7 @@ k_base_small(double *Au, const double *__restrict__ Arhs, const int *__restrict_
         if (it == 0) block_atomic_max(&s_max[0], mx);
         if (threadIdx.x == 0) s_max[1] = 0.0;
         __syncthreads();
-        if (!W || threadIdx.x < kWave) coarse_fmg<double, N, 0, W, ZERO>(S, P, 2, 2, 2, &s_max[1]);
+        coarse_run<double, N, ZERO>(S, P, true, 2, 2, 2, &s_max[1]);
         __syncthreads();
 #pragma unroll
         for (int m = 0; m < IT; ++m) {

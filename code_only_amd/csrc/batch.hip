@@ -295,7 +295,7 @@ template <typename T> int op_coarse(sg_batch *c, const Pairs &pl, int mode, int 
         int cnt, tot;
         SG_TRY(take(c, ex, [](int, int) { return 1; }, &d, &cnt, &tot));
         if (cnt) {
-            hipLaunchKernelGGL(kb_coarse_exact, dim3(tot), dim3(kCoarseThreads), 0, c->stream, bl<float>(c, d, cnt),
+            hipLaunchKernelGGL(kb_coarse_exact, dim3(tot), dim3(kCoarseExactThreads), 0, c->stream, bl<float>(c, d, cnt),
                                (const CoarseDesc<float> *)c->d_desc);
             SG_CHECK_LAUNCH();
         }

@@ -364,7 +364,7 @@ kb_coarse(BL<T> L, const CoarseDesc<T> *descs, int mode, int ncycle, int npre, i
 }
 
 // The exact solve of the first held level (coarse_exact) of every item.
-static __global__ void __launch_bounds__(kCoarseThreads) kb_coarse_exact(BL<float> L, const CoarseDesc<float> *descs)
+static __global__ void __launch_bounds__(kCoarseExactThreads) kb_coarse_exact(BL<float> L, const CoarseDesc<float> *descs)
 {
     Cell<float> c;
     if (!locate(L, (int)blockIdx.x, c)) return;

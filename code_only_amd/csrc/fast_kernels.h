@@ -888,6 +888,119 @@ k_coarse(const T *__restrict__ rhs_in, T *__restrict__ u_out, CoarseCoef<T> P, i
     coarse_solve<T, N, ZERO>(S, P, rhs_in, u_out, mode, ncycle, npre, npost, resmax);
 }
 
+// mg_cycle (mg.F90:42-94) of a grid held by the coarse levels alone (N <= 16) in one launch: FP64
+// residual and update around the inner solve in T, both stopping tests.  A 16^3 solve of 4 iterations
+// is 4 inner solves of 57 us; as launches (inner solve, update + residual, norm) with a host read of the
+// norms per iteration it took 400 us, this 300 us.  psi stays in LDS, its source and the
+// cells' places in registers.  rec (pinned host memory): what the host's statistics need.
+struct SmallRecord {
+    double fmax, fsum;             // max|f|, sum f^2
+    double rmax, rsum, resmax;     // last residual's max and sum of squares; last max|resh2|
+    int iterations, status;
+    double hist[SG_HIST];          // max|r| per iteration
+};
+
+template <typename T, int N>
+__global__ void __launch_bounds__(kCoarseThreads)
+k_cycle_small(double *__restrict__ psi_io, const double *__restrict__ src, CoarseCoef<T> P, double h, double h2i,
+              double tol, int maxit, int stop_mode, int ncycle, int npre, int npost, SmallRecord *rec)
+{
+    using L = CoarseLevel<N>;
+    constexpr int IT = (L::len + kCoarseThreads - 1) / kCoarseThreads;
+    constexpr bool full = L::len % kCoarseThreads == 0;
+    __shared__ CoarseLds<T> S;
+    __shared__ double psi[L::len];
+    __shared__ double s_norm[5];   // max|f|, sum f^2, max|r|, sum r^2, max|resh2|
+    double f[IT];
+    double mx = 0.0, sm = 0.0;
+#pragma unroll
+    for (int m = 0; m < IT; ++m) {
+        const int c = (int)threadIdx.x + m * kCoarseThreads;
+        f[m] = 0.0;
+        if (full || c < L::len) {
+            int i, j, k;
+            L::decode(c, i, j, k);
+            psi[L::at(i, j, k)] = psi_io[c];
+            f[m] = src[c];
+            mx = fmax(mx, fabs(f[m]));
+            sm += f[m] * f[m];
+        }
+    }
+    if (threadIdx.x >= kCoarseThreads - 64) coarse_tables<T, N, false>(S, (int)threadIdx.x - (kCoarseThreads - 64));
+    block_max_sum(mx, sm);
+    if (threadIdx.x == 0) {
+        s_norm[0] = mx;
+        s_norm[1] = sm;
+        s_norm[4] = 0.0;
+    }
+    __syncthreads();
+    int it = 0, status = SG_ERR_NOT_CONVERGED;
+    double rhomax = 0.0;
+    for (;;) {
+        mx = sm = 0.0;
+#pragma unroll
+        for (int m = 0; m < IT; ++m) {
+            const int c = (int)threadIdx.x + m * kCoarseThreads;
+            if (full || c < L::len) {
+                int i, j, k;
+                L::decode(c, i, j, k);
+                auto U = [&](int a, int b, int d) { return psi[L::at((a + N) % N, (b + N) % N, (d + N) % N)]; };
+                const double r = resid_value<double>(U(i, j, k), U(i + 1, j, k), U(i - 1, j, k), U(i, j + 1, k), U(i, j - 1, k),
+                                                     U(i, j, k + 1), U(i, j, k - 1), f[m], h2i);
+                S.r[L::off + L::at(i, j, k)] = (T)r;
+                mx = fmax(mx, fabs(r));
+                sm += r * r;
+            }
+        }
+        block_max_sum(mx, sm);
+        if (threadIdx.x == 0) {
+            s_norm[2] = mx;
+            s_norm[3] = sm;
+        }
+        __syncthreads();
+        // every thread takes the same decision, in the order of the host's loop
+        const double fm = s_norm[0], rm = s_norm[2], resmaxg = s_norm[4] / (h * h);
+        const double rel = fm > 0 ? rm / fm : 0.0;
+        if (it == 0) rhomax = rm;
+        if (threadIdx.x == 0 && it < SG_HIST) rec->hist[it] = rm;
+        if (!isfinite(rm) || !isfinite(s_norm[3])) { status = SG_ERR_NONFINITE; break; }
+        if (stop_mode == SG_STOP_TRUE_RESIDUAL && rel < tol) { status = SG_OK; break; }
+        if (it > 0 && stop_mode == SG_STOP_REFERENCE && (rhomax > 0 ? resmaxg / rhomax : 0.0) < tol) { status = SG_OK; break; }
+        if (it >= maxit) break;
+        __syncthreads();
+        if (threadIdx.x == 0) s_norm[4] = 0.0;
+        __syncthreads();
+        coarse_run<T, N, false>(S, P, true, ncycle, npre, npost,
+                                stop_mode == SG_STOP_REFERENCE ? &s_norm[4] : (double *)nullptr);
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < IT; ++m) {
+            const int c = (int)threadIdx.x + m * kCoarseThreads;
+            if (full || c < L::len) psi[c] = psi[c] + (double)S.u[L::off + c];
+        }
+        ++it;
+        __syncthreads();
+    }
+#pragma unroll
+    for (int m = 0; m < IT; ++m) {
+        const int c = (int)threadIdx.x + m * kCoarseThreads;
+        if (full || c < L::len) {
+            int i, j, k;
+            L::decode(c, i, j, k);
+            psi_io[c] = psi[L::at(i, j, k)];
+        }
+    }
+    if (threadIdx.x == 0) {
+        rec->fmax = s_norm[0];
+        rec->fsum = s_norm[1];
+        rec->rmax = s_norm[2];
+        rec->rsum = s_norm[3];
+        rec->resmax = s_norm[4];
+        rec->iterations = it;
+        rec->status = status;
+    }
+}
+
 struct CoarseExact {
     int n;                                                 // cells per side, <= 16
     float Q[kCoarseMaxN * kCoarseMaxN], lam[kCoarseMaxN];  // Hartley basis and eigenvalues
@@ -919,7 +1032,8 @@ inline void hartley_basis(int n, double h, double *Q, double *lam)
 // for all six passes, and the four threads of a line sit in adjacent lanes, so the line's reads
 // are broadcasts.  Each output is accumulated k = 0 .. n-1 in order with fused multiply-adds.
 constexpr int kCeParts = 4;
-static_assert(kCoarseMaxN * kCoarseMaxN * kCeParts <= kCoarseThreads, "one thread per (line, part)");
+constexpr int kCoarseExactThreads = 1024;
+static_assert(kCoarseMaxN * kCoarseMaxN * kCeParts <= kCoarseExactThreads, "one thread per (line, part)");
 static_assert(kCoarseMaxN <= 4 * kCeParts, "four outputs per thread");
 
 __device__ inline void ce_basis(float (&q)[4][kCoarseMaxN], const float *Q, int n)
@@ -971,9 +1085,9 @@ __device__ inline void coarse_exact(float *g, float *s, const float *Qg, const f
 {
     const int P = n + 1, n3 = n * n * n;
     float *Qs = s, *lam = s + n * n;
-    for (int t = threadIdx.x; t < n * n; t += kCoarseThreads) Qs[t] = Qg[t];
-    for (int t = threadIdx.x; t < n; t += kCoarseThreads) lam[t] = lamg[t];
-    for (int c = threadIdx.x; c < n3; c += kCoarseThreads) {
+    for (int t = threadIdx.x; t < n * n; t += kCoarseExactThreads) Qs[t] = Qg[t];
+    for (int t = threadIdx.x; t < n; t += kCoarseExactThreads) lam[t] = lamg[t];
+    for (int c = threadIdx.x; c < n3; c += kCoarseExactThreads) {
         const int i = c % n, j = (c / n) % n, k = c / (n * n);
         g[(k * n + j) * P + i] = rhs_in[c];
     }
@@ -981,7 +1095,7 @@ __device__ inline void coarse_exact(float *g, float *s, const float *Qg, const f
     float q[4][kCoarseMaxN];
     ce_basis(q, Qs, n);
     for (int a = 0; a < 3; ++a) ce_pass(g, q, n, a);
-    for (int c = threadIdx.x; c < n3; c += kCoarseThreads) {
+    for (int c = threadIdx.x; c < n3; c += kCoarseExactThreads) {
         const int i = c % n, j = (c / n) % n, k = c / (n * n);
         const float den = (lam[i] + lam[j]) + lam[k];
         float &v = g[(k * n + j) * P + i];
@@ -989,13 +1103,13 @@ __device__ inline void coarse_exact(float *g, float *s, const float *Qg, const f
     }
     __syncthreads();
     for (int a = 0; a < 3; ++a) ce_pass(g, q, n, a);
-    for (int c = threadIdx.x; c < n3; c += kCoarseThreads) {
+    for (int c = threadIdx.x; c < n3; c += kCoarseExactThreads) {
         const int i = c % n, j = (c / n) % n, k = c / (n * n);
         u_out[c] = g[(k * n + j) * P + i];
     }
 }
 
-static __global__ void __launch_bounds__(kCoarseThreads)
+static __global__ void __launch_bounds__(kCoarseExactThreads)
 k_coarse_exact(const float *__restrict__ rhs_in, float *__restrict__ u_out, CoarseExact E)
 {
     __shared__ float g[kCoarseMaxN * kCoarseMaxN * (kCoarseMaxN + 1)], q[kCoarseMaxN * kCoarseMaxN + kCoarseMaxN];

@@ -520,7 +520,7 @@ static int exact_bottom(sg_uniform *c)
     const int lb = c->lb, n = c->nl[lb];
     SG_REQUIRE(c->lc > 0, "exact coarse solve needs a level below the finest");
     if (lb == c->lc) {
-        hipLaunchKernelGGL(k_coarse_exact, dim3(1), dim3(kCoarseThreads), 0, c->stream, (const float *)c->f.RHO[lb],
+        hipLaunchKernelGGL(k_coarse_exact, dim3(1), dim3(kCoarseExactThreads), 0, c->stream, (const float *)c->f.RHO[lb],
                            c->f.U[lb], c->cexact);
         SG_CHECK_LAUNCH();
         return SG_OK;
@@ -766,6 +766,43 @@ static int outer_iteration(sg_uniform *c, const double *pin, double *pout, const
     return launch_resid<double, T>(c, levels<T>(c).RHO[0], pout, src, c->n, c->h, c->dnorm);
 }
 
+// The whole solve of a grid of n <= 16 in one launch (k_cycle_small).
+template <typename T, int N> static void small_n(sg_uniform *c, double *psi, const double *src, const sg_params *p)
+{
+    hipLaunchKernelGGL((k_cycle_small<T, N>), dim3(1), dim3(kCoarseThreads), 0, c->stream, psi, src, coarse_coef<T>(c->h),
+                       c->h, 1.0 / (c->h * c->h), p->tol, p->maxit, p->stop_mode, p->ncycle, p->npre, p->npost,
+                       reinterpret_cast<SmallRecord *>(c->hnorm_dev));
+}
+
+template <typename T> static int small_cycle(sg_uniform *c, double *psi, const double *src, const sg_params *p, sg_stats *st)
+{
+    switch (c->n) {
+    case 16: small_n<T, 16>(c, psi, src, p); break;
+    case 8: small_n<T, 8>(c, psi, src, p); break;
+    case 4: small_n<T, 4>(c, psi, src, p); break;
+    default: small_n<T, 2>(c, psi, src, p); break;
+    }
+    SG_CHECK_LAUNCH();
+    SG_HIP(hipEventRecord(c->ev1, c->stream));
+    hipError_t q;
+    while ((q = hipEventQuery(c->ev1)) == hipErrorNotReady) {
+    }
+    SG_HIP(q);
+    const SmallRecord &R = *reinterpret_cast<const SmallRecord *>(c->hnorm);
+    const double fl2 = std::sqrt(R.fsum);
+    for (int it = 0; it <= R.iterations && it < SG_HIST; ++it) st->hist[it] = R.fmax > 0 ? R.hist[it] / R.fmax : 0.0;
+    st->rel_linf = R.fmax > 0 ? R.rmax / R.fmax : 0.0;
+    st->rel_l2 = fl2 > 0 ? std::sqrt(R.rsum) / fl2 : 0.0;
+    st->rel_h2 = st->rel_linf;
+    st->resmaxg = R.resmax / (c->h * c->h);
+    float ms = 0.f;
+    SG_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
+    st->ms = ms;
+    st->iterations = R.iterations;
+    st->status = R.status;
+    return R.status;
+}
+
 // mg.F90:42-94: FP64 defect correction psi += L^-1 (src - L psi) with the chosen inner solver.
 static int uniform_cycle(sg_uniform *c, double *psi, const double *src, const sg_params *p, sg_stats *st)
 {
@@ -785,6 +822,7 @@ static int uniform_cycle(sg_uniform *c, double *psi, const double *src, const sg
     const bool mixed = p->precision == SG_PREC_MIXED;
     SG_HIP(hipEventRecord(c->ev0, c->stream));
     const bool pp = fused_solve(c, p);
+    if (pp && c->lc == 0) return mixed ? small_cycle<float>(c, psi, src, p, st) : small_cycle<double>(c, psi, src, p, st);
     // With the fused update the iterations alternate between psi and psi_alt, so an odd count ends
     // in psi_alt and costs a final copy.  When the previous solve on this context took an odd
     // count, the first residual step also copies psi into psi_alt and the iterations start there.
@@ -925,7 +963,7 @@ static int create(sg_uniform **out, int n, double h, int precisions)
             SG_HIP(hipMalloc(&c->psum, sizeof(double) * 2 * c->npart));
             SG_HIP(hipMalloc(&c->dnorm, sizeof(double) * 8));
             SG_HIP(hipMemsetAsync(c->dnorm, 0, sizeof(double) * 8, c->stream));
-            SG_HIP(hipHostMalloc(&c->hnorm, sizeof(double) * 8, hipHostMallocDefault));
+            SG_HIP(hipHostMalloc(&c->hnorm, std::max(sizeof(double) * 8, sizeof(SmallRecord)), hipHostMallocDefault));
             SG_HIP(hipHostGetDevicePointer((void **)&c->hnorm_dev, c->hnorm, 0));
             SG_TRY(coarse_levels(c));
             if (precisions & SG_PREC_FP64) SG_TRY(alloc_levels<double>(c, c->d));

@@ -355,3 +355,30 @@ def test_fp64_fused_equals_plain(n, cycle, gpu):
             assert sa["resmaxg"] == sb["resmaxg"] if stop == SG_STOP_REFERENCE else True
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("n", [2, 4, 8, 16])
+def test_small_grid_mixed_equals_unfused(n, gpu):
+    """The one-launch mixed solve of n <= 16 against one kernel per loop nest, bit for bit, from a
+    non-zero guess, with maxit 0, a zero source and a NaN in it."""
+    import torch
+    s = UniformSolver(n, 1.0 / n, precisions=SG_PREC_MIXED)
+    f = torch.tensor(problems.clumpy_rhs(n, seed=8), device=gpu)
+    guess = torch.tensor(np.random.default_rng(9).standard_normal((n, n, n)), device=gpu)
+    bad = f.clone()
+    bad[0, 0, 0] = float("nan")
+    try:
+        for src, start, kw in ((f, None, {}), (f, guess, {}), (f, guess, dict(stop_mode=SG_STOP_REFERENCE, tol=1e-2)),
+                               (f, guess, dict(maxit=0)), (torch.zeros_like(f), None, {}), (bad, None, {})):
+            out = []
+            for fused in (True, False):
+                psi = torch.zeros_like(f) if start is None else start.clone()
+                st = s.cycle(psi, src, precision=SG_PREC_MIXED, fused=fused, raise_on_fail=False,
+                             **dict(dict(tol=1e-9, maxit=6), **kw))
+                out.append((psi, st))
+            (a, sa), (b, sb) = out
+            assert torch.equal(torch.nan_to_num(a, nan=7.0), torch.nan_to_num(b, nan=7.0))
+            assert sa["iterations"] == sb["iterations"] and sa["status"] == sb["status"]
+            assert sa["hist"] == sb["hist"] or sa["status"] == 4
+    finally:
+        s.close()
