@@ -527,7 +527,7 @@ static int exact_bottom(sg_uniform *c)
     }
     SG_REQUIRE(n <= kPlaneMaxN && n % 16 == 0 && c->d_qx && c->d_invx && c->f.U1[lb],
                "plane-parallel exact solve not set up (n = %d)", n);
-    const dim3 grid(n * plane_groups(n)), block(kSplitThreads);
+    const dim3 grid(n * plane_groups(n)), block(kPlaneThreads);
     hipLaunchKernelGGL(k_exact_xy_split, grid, block, 0, c->stream, (const float *)c->f.RHO[lb], c->f.U1[lb],
                        (const float *)c->d_qx, n);
     SG_CHECK_LAUNCH();
