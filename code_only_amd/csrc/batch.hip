@@ -197,22 +197,30 @@ void sweep_ns(sg_batch *c, int ns, bool fs, const BL<T> &L, int tot, int cin, in
     }
 }
 
+template <class SS, int NS, bool ZERO, bool PROLONG, bool RESID, typename T>
+void stream_one(sg_batch *c, const BL<T> &L, int tot, int cin, int cout, int cuc)
+{
+    const dim3 grid(8 * ((tot + 7) / 8)), block(StreamGeom<SS, NS, PROLONG, RESID, T>::NT);
+    hipLaunchKernelGGL((kb_stream<SS, NS, ZERO, PROLONG, RESID, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+}
+
+template <class SS, int NS, typename T>
+void stream_ns(sg_batch *c, const BL<T> &L, int tot, int cin, int cout, int cuc, bool zero, bool prolong, bool resid)
+{
+    if (resid && zero) stream_one<SS, NS, true, false, true, T>(c, L, tot, cin, cout, cuc);
+    else if (resid) stream_one<SS, NS, false, false, true, T>(c, L, tot, cin, cout, cuc);
+    else if (prolong) stream_one<SS, NS, false, true, false, T>(c, L, tot, cin, cout, cuc);
+    else if (zero) stream_one<SS, NS, true, false, false, T>(c, L, tot, cin, cout, cuc);
+    else stream_one<SS, NS, false, false, false, T>(c, L, tot, cin, cout, cuc);
+}
+
 template <class SS, typename T>
-void stream_variant(sg_batch *c, const BL<T> &L, int tot, int cin, int cout, int cuc, bool zero, bool prolong,
+void stream_variant(sg_batch *c, int ns, const BL<T> &L, int tot, int cin, int cout, int cuc, bool zero, bool prolong,
                     bool resid)
 {
     if constexpr (stream_built<SS, T>()) {
-        const dim3 grid(8 * ((tot + 7) / 8)), block(SS::NT);
-        if (resid && zero)
-            hipLaunchKernelGGL((kb_stream<SS, true, false, true, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
-        else if (resid)
-            hipLaunchKernelGGL((kb_stream<SS, false, false, true, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
-        else if (prolong)
-            hipLaunchKernelGGL((kb_stream<SS, false, true, false, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
-        else if (zero)
-            hipLaunchKernelGGL((kb_stream<SS, true, false, false, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
-        else
-            hipLaunchKernelGGL((kb_stream<SS, false, false, false, T>), grid, block, 0, c->stream, L, tot, cin, cout, cuc);
+        if (ns == 2) stream_ns<SS, 2, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid);
+        else stream_ns<SS, 1, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid);
     }
 }
 
@@ -240,15 +248,15 @@ int op_sweep_cfg(sg_batch *c, const Pairs &pl, int cfg, int ns, bool fs, int cin
     if (!cnt) return SG_OK;
     const BL<T> L = bl<T>(c, d, cnt);
     switch (cfg) {
-    case kNumTiles + 0: stream_variant<Stream0, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 1: stream_variant<Stream1, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 2: stream_variant<Stream2, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 3: stream_variant<Stream3, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 4: stream_variant<Stream4, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 5: stream_variant<Stream5, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 6: stream_variant<Stream6, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 7: stream_variant<Stream7, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 8: stream_variant<Stream8, T>(c, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 0: stream_variant<Stream0, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 1: stream_variant<Stream1, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 2: stream_variant<Stream2, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 3: stream_variant<Stream3, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 4: stream_variant<Stream4, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 5: stream_variant<Stream5, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 6: stream_variant<Stream6, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 7: stream_variant<Stream7, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 8: stream_variant<Stream8, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case 0: sweep_ns<Tile0, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case 1: sweep_ns<Tile1, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case 2: sweep_ns<Tile2, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
@@ -346,10 +354,7 @@ int op_exact_planes(sg_batch *c, const Pairs &pl)
 template <typename T> int level_ns(sg_batch *c, int v)
 {
     if constexpr (std::is_same<T, float>::value) return c->tile_ns[v];
-    long m = 0;
-    for (int p = 0; p < c->np; ++p)
-        if (c->lc[p] > v) m += cells(c->n[p] >> v);
-    return fp64_two_sweeps(m) ? 2 : 1;
+    else return kMaxSweepsPerLaunch;
 }
 
 // ns sweeps of level v of the listed problems.  FP32: one launch with the autotuned shape.  FP64: the
@@ -362,7 +367,6 @@ int op_sweep(sg_batch *c, const Pairs &pl, int v, int ns, int cin, int cout, int
     if constexpr (std::is_same<T, float>::value) {
         return op_sweep_cfg<T>(c, pl, c->tile_cfg[v], ns, c->tile_fs[v] != 0, cin, cout, cuc, zero, prolong, resid);
     } else {
-        const bool two = level_ns<T>(c, v) == 2;
         for (int cls = 0; cls < 2; ++cls) {
             Pairs w;
             int unit = 64;
@@ -374,7 +378,7 @@ int op_sweep(sg_batch *c, const Pairs &pl, int v, int ns, int cin, int cout, int
                 m += cells(n);
                 w.push_back(q);
             }
-            SG_TRY(op_sweep_cfg<T>(c, w, fp64_sweep_shape(unit, m, two), ns, false, cin, cout, cuc, zero, prolong, resid));
+            SG_TRY(op_sweep_cfg<T>(c, w, fp64_sweep_shape(unit, m), ns, false, cin, cout, cuc, zero, prolong, resid));
         }
         return SG_OK;
     }

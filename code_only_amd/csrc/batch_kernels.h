@@ -304,15 +304,16 @@ __global__ void __launch_bounds__(TL::NT) kb_sweep(BL<T> L, int total, int cin, 
                                                  RESID ? (&q + 1)->a[CRHS] : nullptr, nullptr, c.lb);
 }
 
-// The streaming form of the same sweep (one launch = one sweep).
-template <class SS, bool ZERO, bool PROLONG, bool RESID, typename T>
-__global__ void __launch_bounds__(SS::NT) kb_stream(BL<T> L, int total, int cin, int cout, int cuc)
+// The streaming form of the same sweeps.
+template <class SS, int NS, bool ZERO, bool PROLONG, bool RESID, typename T>
+__global__ void __launch_bounds__((StreamGeom<SS, NS, PROLONG, RESID, T>::NT))
+kb_stream(BL<T> L, int total, int cin, int cout, int cuc)
 {
     Cell<T> c;
     if (!locate(L, xcd_block(total), c)) return;
     const PL<T> &q = *c.q;
     const int l = c.it->l;
-    sweep_stream<SS, ZERO, PROLONG, RESID, T>(q.a[cin], q.a[cout], q.a[CRHS], q.n, q.h2, q.h2i,
+    sweep_stream<SS, NS, ZERO, PROLONG, RESID, T>(q.a[cin], q.a[cout], q.a[CRHS], q.n, q.h2, q.h2i,
                                            PROLONG ? coarse_src(q, l, cuc) : nullptr,
                                            RESID ? (&q + 1)->a[CRHS] : nullptr, nullptr, c.lb);
 }

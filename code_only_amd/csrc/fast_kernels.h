@@ -12,6 +12,7 @@
 //    owner's arithmetic exactly, so the result equals the two-launch colour sweep bit for bit.
 //    Tile shape and workgroup size are template parameters; the host picks one per level size by
 //    timing (all shapes give identical values).
+//  * k_sweep_stream: the same, two sweeps per launch, marching up a column (pair_stream.h).
 //  * k_interp_cubic_tile: the FMG tricubic prolongation (interpolation.F90:98-217) as the
 //    reference's three separable passes, on an LDS-staged coarse tile.
 //  * k_coarse: every level of <= 16^3 cells in one workgroup's LDS (coarse_levels.h): the FMG part of
@@ -26,21 +27,10 @@
 #include <cmath>
 
 #include "coarse_levels.h"
+#include "pair_stream.h"
 #include "uniform_kernels.h"
 
 namespace sg {
-
-__device__ __forceinline__ int wrapn(int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); }
-
-// Tile index with XCD-aware placement: consecutive workgroups are dealt round-robin to the 8
-// XCDs, so workgroup b is given tile (b % 8) * per + b / 8 -- each XCD works through a contiguous
-// range of tiles (z-slabs), and the halos its tiles share stay in that XCD's L2.
-__device__ __forceinline__ int xcd_tile(int ntiles)
-{
-    const int per = (ntiles + 7) / 8;
-    const int b = (int)blockIdx.x;
-    return (b % 8) * per + b / 8;
-}
 
 template <int TX_, int TY_, int TZ_, int NT_> struct Tile {
     static constexpr int TX = TX_, TY = TY_, TZ = TZ_, NT = NT_;
@@ -325,355 +315,21 @@ k_sweep_tile(const T *__restrict__ uin, T *__restrict__ uout, const T *__restric
     sweep_tile<TL, NS, ZERO, PROLONG, RESID, FS, T, ZB>(uin, uout, f, n, h2, h2i, uc, rc, resmax, t);
 }
 
-// ------------------------------------------------------------------------------------------------
-// Streaming form of the fused sweep: a workgroup owns an SX x SY column of the grid and a chunk of
-// ZC planes, and marches up the chunk with the planes it needs in an LDS ring of R planes (u and
-// f).  Step p:
-//   1. first colour (i+j+k odd, the reference's ipass 1) of plane p, on the column with margin 1;
-//   -- barrier --
-//   2. plane p + 2 (fetched into registers one step earlier, with the trilinear correction added
-//      for PROLONG) into the slot of plane p - 3 (p - 4 with RESID), plane p + 3 fetched into the
-//      registers; second colour of plane p - 1, margin 2, whose first-colour neighbours on planes
-//      p - 2, p - 1 and p are all new: plane p - 1 is final;
-//   -- barrier --
-//   3. plane p - 1 stored; with RESID, the residual of plane p - 2 (final, as are p - 3 and
-//      p - 1), restricted pairwise (restriction.F90:132-147 operand order).
-// Phase 3 overlaps the next step's first colour, which touches none of its planes.  Every
-// thread's cells and global offsets are fixed for the whole march and computed once; the march is
-// unrolled by R, so the ring slots are immediate LDS offsets.  Halo: H = 2 cells in x and y, H
-// planes below and above the chunk (H = 3 with RESID).  max|resh2| is kept in FP32 only when
-// asked for (the max of the FP32 values, widened once, equals the max of their widened values).
-// Every cell update sees the same operands as the two-launch colour passes, so the values are
-// those of the tile kernel, bit for bit.
-// ------------------------------------------------------------------------------------------------
-template <int SX_, int SY_, int ZC_, int NT_> struct StreamShape {
-    static constexpr int SX = SX_, SY = SY_, ZC = ZC_, NT = NT_;
-};
-
-template <class SS, bool PROLONG, bool RESID, typename T = float> struct StreamGeom {
-    static constexpr int H = RESID ? 3 : 2;
-    static constexpr int PX = SS::SX + 2 * H, PY = SS::SY + 2 * H, PP = PX * PY;
-    static constexpr int R = RESID ? 6 : 5;                    // ring slots
-    static constexpr int CX = PX / 2 + 2, CY = PY / 2 + 2, CP = CX * CY;  // staged coarse plane
-    static constexpr int CR = 8;                               // coarse ring slots
-    static constexpr int IL = (PP + SS::NT - 1) / SS::NT;      // ring cells per thread
-    static constexpr int ICL = (CP + SS::NT - 1) / SS::NT;     // coarse cells per thread
-    static constexpr int IS = (SS::SX * SS::SY + SS::NT - 1) / SS::NT;  // core cells per thread
-    static constexpr int RX1 = (PX - 2) / 2, RY1 = PY - 2, C1 = RX1 * RY1, I1 = (C1 + SS::NT - 1) / SS::NT;
-    static constexpr int RX2 = (PX - 4) / 2, RY2 = PY - 4, C2 = RX2 * RY2, I2 = (C2 + SS::NT - 1) / SS::NT;
-    static constexpr int lds_bytes = (int)sizeof(T) * (2 * R * PP + (PROLONG ? CR * CP : 0) + (RESID ? SS::SX * SS::SY : 0));
-    static_assert(IL <= 32 && I1 <= 32 && I2 <= 32 && IS <= 32, "per-thread bit masks hold 32 cells");
-};
-
-template <class SS, bool PROLONG, bool RESID, typename T = float> constexpr bool stream_fits_lds()
-{
-    return StreamGeom<SS, PROLONG, RESID, T>::lds_bytes + 1024 <= 163840;
-}
-
-__device__ __forceinline__ int pmod(int a, int m) { const int r = a % m; return r < 0 ? r + m : r; }
-__device__ __forceinline__ int fdiv2(int a) { return a >> 1; }  // floor(a / 2), arithmetic shift
-
-// Cells of one colour pass (margin M) owned by this thread: base offset y PX + M + 2 xh (the cell
-// is base + (y + k) % 2 on plane k, since x0, y0 and colour + M are even), y parity, and for
-// either x parity whether the cell is in the column's core.
-template <int N> struct PassCells {
-    int cb[N];
-    unsigned yb = 0u, valid = 0u, core0 = 0u, core1 = 0u;
-};
-
-template <int N, int RX, int RY, int CNT, int NT, int PX, int M, int H, int SX, int SY>
-__device__ __forceinline__ void pass_cells(PassCells<N> &P, int tid)
-{
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const int q = tid + i * NT;
-        const int xh = q % RX, y = M + q / RX;
-        P.cb[i] = y * PX + M + 2 * xh;
-        if (q < CNT) P.valid |= 1u << i;
-        if (y & 1) P.yb |= 1u << i;
-        const bool yc = y >= H && y < H + SY;
-        if (yc && M + 2 * xh >= H && M + 2 * xh < H + SX) P.core0 |= 1u << i;
-        if (yc && M + 2 * xh + 1 >= H && M + 2 * xh + 1 < H + SX) P.core1 |= 1u << i;
-    }
-}
-
-template <class SS, bool ZERO, bool PROLONG, bool RESID, typename T = float>
-__device__ __forceinline__ void sweep_stream(const T *__restrict__ uin, T *__restrict__ uout,
-                                             const T *__restrict__ f, int n, T h2, T h2i,
-                                             const T *__restrict__ uc, T *__restrict__ rc, double *resmax, int t)
-{
-    using G = StreamGeom<SS, PROLONG, RESID, T>;
-    constexpr int SX = SS::SX, SY = SS::SY, ZC = SS::ZC, NT = SS::NT;
-    constexpr int H = G::H, PX = G::PX, PP = G::PP, R = G::R, CX = G::CX, CP = G::CP, CR = G::CR;
-    static_assert(SX % 2 == 0 && SY % 2 == 0 && ZC % 2 == 0, "stream shape");
-    static_assert(!PROLONG || H % 2 == 0, "the coarse-value window starts on an even fine plane");
-    __shared__ T su[R * PP];
-    __shared__ T sf[R * PP];
-    __shared__ T scz[PROLONG ? CR * CP : 1];
-    __shared__ T srp[RESID ? SX * SY : 1];
-    const int ntx = n / SX, nty = n / SY;
-    const int tx = t % ntx, ty = (t / ntx) % nty, tz = t / (ntx * nty);
-    const int x0 = tx * SX, y0 = ty * SY, z0 = tz * ZC;
-    const int nc = n >> 1;
-    const int tid = threadIdx.x;
-    const bool want = resmax != nullptr;
-    T amax = T(0);
-
-    // ---- per-thread geometry, fixed for the whole march ----
-    int goff[G::IL];         // global (y, x) offset of ring cell tid + it NT
-    int coff[PROLONG ? G::IL : 1][4];  // its trilinear stencil in the staged coarse plane
-#pragma unroll
-    for (int it = 0; it < G::IL; ++it) {
-        const int q = tid + it * NT;
-        const int x = q % PX, y = q / PX;
-        goff[it] = wrapn(y0 - H + y, n) * n + wrapn(x0 - H + x, n);
-        if (PROLONG) {
-            const int ic = (x >> 1) + 1, jc = (y >> 1) + 1;
-            const int ic1 = ic + 2 * (x & 1) - 1, jc1 = jc + 2 * (y & 1) - 1;
-            coff[PROLONG ? it : 0][0] = jc * CX + ic;
-            coff[PROLONG ? it : 0][1] = jc * CX + ic1;
-            coff[PROLONG ? it : 0][2] = jc1 * CX + ic;
-            coff[PROLONG ? it : 0][3] = jc1 * CX + ic1;
-        }
-    }
-    int cgoff[PROLONG ? G::ICL : 1];  // global (y, x) offset of coarse staged cell tid + it NT
-    if (PROLONG) {
-#pragma unroll
-        for (int it = 0; it < G::ICL; ++it) {
-            const int q = tid + it * NT;
-            const int x = q % CX, y = q / CX;
-            cgoff[PROLONG ? it : 0] = wrapn(fdiv2(y0 - H) - 1 + y, nc) * nc + wrapn(fdiv2(x0 - H) - 1 + x, nc);
-        }
-    }
-    PassCells<G::I1> P1;
-    PassCells<G::I2> P2;
-    pass_cells<G::I1, G::RX1, G::RY1, G::C1, NT, PX, 1, H, SX, SY>(P1, tid);
-    pass_cells<G::I2, G::RX2, G::RY2, G::C2, NT, PX, 2, H, SX, SY>(P2, tid);
-    int soff[G::IS], sl[G::IS];  // core cells: global (y, x) offset, ring offset
-#pragma unroll
-    for (int it = 0; it < G::IS; ++it) {
-        const int q = tid + it * NT;
-        const int x = q % SX, y = q / SX;
-        soff[it] = (y0 + y) * n + x0 + x;
-        sl[it] = (y + H) * PX + x + H;
-    }
-
-    T ru[G::IL], rf[G::IL], rcz[PROLONG ? G::ICL : 1];
-    auto fetch = [&](int k) {
-        const int base = wrapn(k, n) * n * n;
-#pragma unroll
-        for (int it = 0; it < G::IL; ++it) {
-            if (PP % NT == 0 || tid + it * NT < PP) {
-                ru[it] = ZERO ? T(0) : uin[base + goff[it]];
-                rf[it] = f[base + goff[it]];
-            }
-        }
-    };
-    auto fetch_coarse = [&](int c) {
-        const int base = wrapn(c, nc) * nc * nc;
-#pragma unroll
-        for (int it = 0; it < G::ICL; ++it)
-            if (CP % NT == 0 || tid + it * NT < CP) rcz[PROLONG ? it : 0] = uc[base + cgoff[PROLONG ? it : 0]];
-    };
-    auto put_coarse = [&](int c) {
-        T *dst = scz + (c & (CR - 1)) * CP;
-#pragma unroll
-        for (int it = 0; it < G::ICL; ++it)
-            if (CP % NT == 0 || tid + it * NT < CP) dst[tid + it * NT] = rcz[PROLONG ? it : 0];
-    };
-    // PROLONG: the four coarse values of each ring cell's trilinear stencil on the two coarse
-    // planes a put reads, held in registers: win[0] plane m, win[1] plane m + 1 for the fine
-    // planes 2m + 1 and 2m + 2, so each coarse plane is read from LDS once per thread, not 4 times
-    constexpr int WI = PROLONG ? G::IL : 1;
-    T win[2][WI][4];
-    auto win_load = [&](int w, int c) {
-        const T *src = scz + (c & (CR - 1)) * CP;
-#pragma unroll
-        for (int it = 0; it < WI; ++it)
-            if (PP % NT == 0 || tid + it * NT < PP)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) win[w][it][e] = src[coff[PROLONG ? it : 0][e]];
-    };
-    // the fetched plane k into ring slot `slot` (adding the trilinear correction with PROLONG:
-    // coarse planes kc = floor(k / 2) and kc1 = kc - 1 (k even) or kc + 1 (k odd))
-    auto put = [&](int k, int slot) {
-        T *du = su + slot * PP, *df = sf + slot * PP;
-        const bool odd = (k & 1) != 0;
-        if (PROLONG && odd) {
-#pragma unroll
-            for (int it = 0; it < WI; ++it)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) win[0][it][e] = win[1][it][e];
-            win_load(1, fdiv2(k) + 1);
-        }
-#pragma unroll
-        for (int it = 0; it < G::IL; ++it) {
-            const int q = tid + it * NT;
-            if (PP % NT == 0 || q < PP) {
-                T v = ru[it];
-                if (PROLONG) {
-                    const int w = PROLONG ? it : 0;
-                    T a[4], b[4];  // plane kc, plane kc1
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        a[e] = odd ? win[0][w][e] : win[1][w][e];
-                        b[e] = odd ? win[1][w][e] : win[0][w][e];
-                    }
-                    v = v + trilinear_value<T>(a[0], a[1], a[2], b[0], b[2], b[1], a[3], b[3]);
-                }
-                du[q] = v;
-                df[q] = rf[it];
-            }
-        }
-    };
-    // one colour pass over the cells P on plane k: u (slot of k), um / up (k - 1 / k + 1), fk
-    auto colour = [&](auto &P, int k, T *u, const T *um, const T *up, const T *fk, bool out) {
-        constexpr int N = sizeof(P.cb) / sizeof(int);
-        const unsigned kb = (unsigned)(k & 1);
-#pragma unroll
-        for (int i = 0; i < N; ++i) {
-            if (((P.valid >> i) & 1u) == 0u) continue;
-            const unsigned d = ((P.yb >> i) & 1u) ^ kb;
-            const int c = P.cb[i] + (int)d;
-            T s;
-            u[c] = relax_value<T>(u[c], u[c + 1], u[c - 1], u[c + PX], u[c - PX], up[c], um[c], fk[c], h2, &s);
-            if (want && out && ((((d ? P.core1 : P.core0) >> i) & 1u) != 0u)) amax = fmax(amax, fabs(s));
-        }
-    };
-    auto resid_at = [&](int slot, int slotm, int slotp, int x, int y) {
-        const T *u = su + slot * PP, *um = su + slotm * PP, *up = su + slotp * PP;
-        const T *fk = sf + slot * PP;
-        const int c = (y + H) * PX + x + H;
-        return resid_value<T>(u[c], u[c + 1], u[c - 1], u[c + PX], u[c - PX], up[c], um[c], fk[c], h2i);
-    };
-
-    const int zlo = z0 - H, zhi = z0 + ZC + H - 1;  // planes held at some point
-    // ---- prologue: coarse planes for fine planes zlo .. zlo + 3, fine planes zlo .. zlo + 2 into
-    // slots 0 .. 2, plane zlo + 3 (and the next coarse plane) into registers ----
-    auto cneed = [&](int k) { return fdiv2(k) + 1; };  // highest coarse plane put(k) reads
-    int cmax = 0;
-    if (PROLONG) {
-        for (int c = fdiv2(zlo) - 1; c <= cneed(zlo + 3); ++c) {
-            fetch_coarse(c);
-            put_coarse(c);
-        }
-        cmax = cneed(zlo + 3);
-        __syncthreads();
-    }
-    if (PROLONG) {
-        // zlo is even (H = 2, z0 a multiple of the even ZC): put(zlo) reads planes zlo/2 - 1, zlo/2
-        win_load(0, fdiv2(zlo) - 1);
-        win_load(1, fdiv2(zlo));
-    }
-    for (int k = zlo; k <= zlo + 2; ++k) {
-        fetch(k);
-        put(k, k - zlo);
-    }
-    fetch(zlo + 3);
-    bool cpend = false;  // a coarse plane (cmax + 1) waits in the registers
-    if (PROLONG && cneed(zlo + 4) > cmax) {
-        fetch_coarse(cmax + 1);
-        cpend = true;
-    }
-    __syncthreads();
-    for (int pb = zlo + 1; pb <= zhi - 1; pb += R) {
-#pragma unroll
-        for (int uu = 0; uu < R; ++uu) {
-            const int pa = pb + uu;
-            if (pa > zhi - 1) break;  // uniform per workgroup
-            // ring slot of plane pa + delta: (pa + delta - zlo) mod R, pa - zlo = 1 + uu (mod R)
-            auto S = [&](int delta) { return ((1 + uu + delta) % R + R) % R; };
-            // 1. first colour of plane pa (margin 1)
-            colour(P1, pa, su + S(0) * PP, su + S(-1) * PP, su + S(1) * PP, sf + S(0) * PP, pa >= z0 && pa < z0 + ZC);
-            __syncthreads();
-            // 2. coarse plane for the next step's put, plane pa + 2 into its slot, fetches
-            if (PROLONG && cpend) {
-                put_coarse(cmax + 1);
-                ++cmax;
-                cpend = false;
-            }
-            if (pa + 2 <= zhi) put(pa + 2, S(2));
-            if (pa + 3 <= zhi) fetch(pa + 3);
-            if (PROLONG && pa + 3 <= zhi && cneed(pa + 4 <= zhi ? pa + 4 : zhi) > cmax) {
-                fetch_coarse(cmax + 1);
-                cpend = true;
-            }
-            //    second colour of plane pa - 1 (margin 2): final
-            if (pa - 1 >= zlo + 2 && pa - 1 <= zhi - 2)
-                colour(P2, pa - 1, su + S(-1) * PP, su + S(-2) * PP, su + S(0) * PP, sf + S(-1) * PP,
-                       pa - 1 >= z0 && pa - 1 < z0 + ZC);
-            __syncthreads();
-            // 3. store plane pa - 1; residual of plane pa - 2
-            if (pa - 1 >= z0 && pa - 1 < z0 + ZC) {
-                const T *u = su + S(-1) * PP;
-                const int gz = wrapn(pa - 1, n) * n * n;
-#pragma unroll
-                for (int it = 0; it < G::IS; ++it)
-                    if ((SX * SY) % NT == 0 || tid + it * NT < SX * SY) uout[gz + soff[it]] = u[sl[it]];
-            }
-            if (RESID) {
-                const int kq = pa - 2;
-                if (kq >= z0 && kq < z0 + ZC) {
-                    if ((kq & 1) == 0) {
-                        for (int q = tid; q < SX * SY; q += NT) srp[q] = resid_at(S(-2), S(-3), S(-1), q % SX, q / SX);
-                    } else {
-                        // coarse cell (cx, cy) of the pair (kq - 1, kq), shared by two adjacent lanes:
-                        // lane b forms the two residuals of row 2 cy + b on the odd plane and takes
-                        // that row's two of the even plane from srp; the pair swaps its four values
-                        // and lane 0 restricts the eight (NT is a multiple of the wave size, so both
-                        // lanes of a pair are in one wave and in the same loop trip)
-                        for (int q = tid; q < SX * SY / 2; q += NT) {
-                            const int b = q & 1, cx = (q >> 1) % (SX / 2), cy = (q >> 1) / (SX / 2);
-                            const int y = 2 * cy + b;
-                            const T e0 = srp[y * SX + 2 * cx], e1 = srp[y * SX + 2 * cx + 1];
-                            const T o0 = resid_at(S(-2), S(-3), S(-1), 2 * cx, y);
-                            const T o1 = resid_at(S(-2), S(-3), S(-1), 2 * cx + 1, y);
-                            const T pe0 = __shfl_xor(e0, 1), pe1 = __shfl_xor(e1, 1);
-                            const T po0 = __shfl_xor(o0, 1), po1 = __shfl_xor(o1, 1);
-                            if (b == 0) {
-                                // r[a + 2 b + 4 dz]: own row is b = 0, the partner's b = 1
-                                const T r[8] = {e0, e1, pe0, pe1, o0, o1, po0, po1};
-                                const int gcx = x0 / 2 + cx, gcy = y0 / 2 + cy, gcz = wrapn(kq, n) / 2;
-                                rc[(gcz * nc + gcy) * nc + gcx] =
-                                    restrict_value<T>(r[0], r[1], r[2], r[4], r[3], r[5], r[6], r[7]);
-                            }
-                        }
-                    }
-                }
-            }
-        }
-    }
-    if (want) block_atomic_max(resmax, (double)amax);
-}
-
-template <class SS, bool ZERO, bool PROLONG, bool RESID, typename T = float>
-__global__ void __launch_bounds__(SS::NT)
-k_sweep_stream(const T *__restrict__ uin, T *__restrict__ uout, const T *__restrict__ f, int n, T h2,
-               T h2i, const T *__restrict__ uc, T *__restrict__ rc, double *resmax)
-{
-    const int ntiles = (n / SS::SX) * (n / SS::SY) * (n / SS::ZC);
-    const int t = xcd_tile(ntiles);
-    if (t >= ntiles) return;
-    sweep_stream<SS, ZERO, PROLONG, RESID, T>(uin, uout, f, n, h2, h2i, uc, rc, resmax, t);
-}
-
-// Streaming shapes the autotuners choose from beside the tiles (one sweep per launch, source always
-// staged): column SX x SY, chunk of ZC planes, NT threads.
-using Stream0 = StreamShape<64, 16, 32, 512>;
-using Stream1 = StreamShape<64, 16, 16, 512>;
-using Stream2 = StreamShape<64, 32, 32, 512>;
-using Stream3 = StreamShape<32, 16, 32, 256>;
-using Stream4 = StreamShape<128, 16, 32, 512>;
-using Stream5 = StreamShape<32, 16, 16, 256>;
-using Stream6 = StreamShape<32, 8, 16, 256>;
-using Stream7 = StreamShape<32, 32, 32, 512>;
-using Stream8 = StreamShape<16, 16, 16, 256>;
+// Streaming shapes (pair_stream.h) the autotuners choose from beside the tiles, with two sweeps per launch
+// (one where a single sweep is left): column SX x SY, chunk of ZC planes.  A longer chunk spends less on
+// its halo planes, a shorter one makes more workgroups: 512^3 is fastest with 128 planes, 256^3 with 64.
+using Stream0 = StreamShape<64, 16, 32>;
+using Stream1 = StreamShape<64, 16, 64>;
+using Stream2 = StreamShape<64, 16, 128>;
+using Stream3 = StreamShape<32, 32, 32>;
+using Stream4 = StreamShape<32, 32, 64>;
+using Stream5 = StreamShape<32, 16, 16>;
+using Stream6 = StreamShape<32, 16, 64>;
+using Stream7 = StreamShape<16, 16, 16>;
+using Stream8 = StreamShape<16, 8, 8>;
 constexpr int kNumStream = 9;
-static const int kStreamDims[kNumStream][4] = {
-    {64, 16, 32, 512}, {64, 16, 16, 512}, {64, 32, 32, 512}, {32, 16, 32, 256}, {128, 16, 32, 512},
-    {32, 16, 16, 256}, {32, 8, 16, 256},  {32, 32, 32, 512}, {16, 16, 16, 256}};
-static_assert(stream_fits_lds<Stream2, true, false>() && stream_fits_lds<Stream2, false, true>(), "stream LDS");
-static_assert(stream_fits_lds<Stream4, true, false>() && stream_fits_lds<Stream4, false, true>(), "stream LDS");
+static const int kStreamDims[kNumStream][3] = {{64, 16, 32}, {64, 16, 64}, {64, 16, 128}, {32, 32, 32}, {32, 32, 64},
+                                               {32, 16, 16}, {32, 16, 64}, {16, 16, 16},  {16, 8, 8}};
 
 // sweep configurations: 0 .. kNumTiles-1 tiles, kNumTiles .. kNumTiles+kNumStream-1 streams
 constexpr int kNumCfg = kNumTiles + kNumStream;
@@ -693,41 +349,39 @@ inline bool cfg_fits(int cfg, int n)
 template <class TL, int NS, bool FS, typename T> constexpr bool sweep_built()
 {
     if (sizeof(T) == sizeof(float)) return sweep_fits_lds<TL, NS, FS, T>();
-    return !FS && ((TL::NT == 1024 && NS == 1) || (TL::TX == 16 && TL::NT == 1024) || (TL::TX == 16 && NS == 1) || TL::TX == 8);
+    return !FS && ((TL::TX == 16 && TL::NT == 1024) || TL::TX == 8);
 }
 template <class SS, typename T> constexpr bool stream_built()
 {
-    if (sizeof(T) == sizeof(float)) return stream_fits_lds<SS, true, false, T>() && stream_fits_lds<SS, false, true, T>();
-    return SS::ZC == 32 && SS::NT == 512 && (SS::SX == 64 ? SS::SY == 16 : SS::SX == 32);
+    return sizeof(T) == sizeof(float) || (SS::SX == 32 && SS::SY == 16);
+}
+template <class SS, typename T> constexpr bool stream_built_fits()
+{
+    return !stream_built<SS, T>() || (StreamGeom<SS, 2, true, false, T>::fits && StreamGeom<SS, 2, false, true, T>::fits);
 }
 template <class TL, int NS, bool FS, typename T> constexpr bool sweep_built_fits()
 {
     return !sweep_built<TL, NS, FS, T>() || sweep_fits_lds<TL, NS, FS, T>();
 }
-static_assert(sweep_built_fits<Tile0, 1, false, double>() && sweep_built_fits<Tile1, 2, false, double>() &&
-                  sweep_built_fits<Tile2, 1, false, double>() && sweep_built_fits<Tile4, 2, false, double>() &&
-                  stream_fits_lds<Stream0, true, false, double>() && stream_fits_lds<Stream0, false, true, double>() &&
-                  stream_fits_lds<Stream7, true, false, double>() && stream_fits_lds<Stream7, false, true, double>(),
+static_assert(sweep_built_fits<Tile1, 2, false, double>() && sweep_built_fits<Tile4, 2, false, double>() &&
+                  stream_built_fits<Stream5, double>() && stream_built_fits<Stream6, double>(),
               "FP64 sweep shapes exceed the LDS");
+static_assert(stream_built_fits<Stream0, float>() && stream_built_fits<Stream3, float>() &&
+                  stream_built_fits<Stream5, float>() && stream_built_fits<Stream7, float>(),
+              "FP32 streaming shapes exceed the LDS or a workgroup");
 
-// The FP64 sweep shape of a launch over levels whose widths are all multiples of `unit` (64, 32, 16 or
-// 8) with `cells` cells in all: the largest shape that still makes 256 workgroups, one per CU, since a
-// workgroup's halo costs less the larger its tile; below that the levels are bound by latency, and two
-// sweeps per launch halve the launches (two_sweeps: the caller's choice for all launches of the level,
-// fp64_two_sweeps).  One V(2,2) visit of one grid, us: 512^3 stream 64 x 16 z32 3358, 32 x 32 z32
-// 3605, tile 32 x 16 x 16 4383; 256^3 426, 448, 522; 128^3 tile 32 x 16 x 16 64, stream 78, tile
-// 16 x 8 x 8 76; 64^3 tile 16 x 8 x 8 with two sweeps 20.3, with one 21.0, tile 8^3 22.1; 32^3 tile 8^3
-// with two sweeps 14.6, with one 16.4, tile 16 x 8 x 8 18.1.
+// The FP64 sweep shape of a launch, always of two sweeps where two are left, over levels whose widths are
+// all multiples of `unit` (64, 32, 16 or 8) with `cells` cells in all: the largest shape that still makes
+// 256 workgroups, one per CU, since a workgroup's halo costs less the larger its shape; below that the
+// levels are bound by latency.  One V(2,2) visit of one grid, us: 512^3 stream 32 x 16 z64 2457 (one sweep
+// per launch in 64 x 16 z64 3062); 256^3 357 (374); 128^3 stream 32 x 16 z16 55, tile 32 x 16 x 16 with
+// one sweep 64; 64^3 tile 16 x 8 x 8 20.3, stream 16 x 8 z8 25.4, tile 8^3 22.1; 32^3 tile 8^3 14.6, tile
+// 16 x 8 x 8 18.1.
 constexpr long kSweepCUs = 256;
-inline bool fp64_two_sweeps(long cells) { return cells < kSweepCUs * 32 * 16 * 16; }
-inline int fp64_sweep_shape(int unit, long cells, bool two_sweeps)
+inline int fp64_sweep_shape(int unit, long cells)
 {
-    if (!two_sweeps) {
-        if (unit >= 64 && cells >= kSweepCUs * 64 * 16 * 32) return kNumTiles + 0;
-        if (unit >= 32 && cells >= kSweepCUs * 32 * 32 * 32) return kNumTiles + 7;
-        if (unit >= 32) return 0;
-        return unit >= 16 ? 2 : 4;
-    }
+    if (unit >= 64 && cells >= kSweepCUs * 32 * 16 * 64) return kNumTiles + 6;
+    if (unit >= 32 && cells >= kSweepCUs * 32 * 16 * 16) return kNumTiles + 5;
     return unit >= 16 && cells >= kSweepCUs * 16 * 8 * 8 ? 1 : 4;
 }
 
@@ -749,12 +403,11 @@ template <typename T> inline bool cand_ok(int cfg, int ns, bool fs)
     }
 }
 
-// whether configuration cfg with (ns, fs) exists: streams take one sweep per launch and always
-// stage the source (reported as fs = 0)
+// whether configuration cfg with (ns, fs) exists: streams hold the source in registers (fs = 0)
 template <typename T> inline bool cfg_ok(int cfg, int ns, bool fs)
 {
     if (cfg < kNumTiles) return cand_ok<T>(cfg, ns, fs);
-    if (ns != 1 || fs) return false;
+    if (ns < 1 || ns > kMaxSweepsPerLaunch || fs) return false;
     switch (cfg - kNumTiles) {
     case 0: return stream_built<Stream0, T>();
     case 1: return stream_built<Stream1, T>();
@@ -779,7 +432,7 @@ inline void cand_decode(int cand, int &cfg, int &ns, bool &fs)
         fs = cand % 2;
     } else {
         cfg = kNumTiles + (cand - nt);
-        ns = 1;
+        ns = kMaxSweepsPerLaunch;
         fs = false;
     }
 }

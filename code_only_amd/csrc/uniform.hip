@@ -306,28 +306,39 @@ static void sweep_ns(hipStream_t s, int ns, bool fs, const T *uin, T *uout, cons
     }
 }
 
-// ns (1 or 2) fused red-black sweeps of a fine level (n >= 32) with tile shape cfg, the source
-// staged in LDS when fs: uin -> uout.
+template <class SS, int NS, bool ZERO, bool PROLONG, bool RESID, typename T>
+static void stream_one(hipStream_t s, const T *uin, T *uout, const T *f, int n, T h2, T h2i, const T *uc, T *rc,
+                       double *resmax)
+{
+    const int ntiles = (n / SS::SX) * (n / SS::SY) * (n / SS::ZC);
+    const dim3 grid(8 * ((ntiles + 7) / 8)), block(StreamGeom<SS, NS, PROLONG, RESID, T>::NT);
+    hipLaunchKernelGGL((k_sweep_stream<SS, NS, ZERO, PROLONG, RESID, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc,
+                       rc, resmax);
+}
+
+template <class SS, int NS, typename T>
+static void stream_ns(hipStream_t s, const T *uin, T *uout, const T *f, int n, T h2, T h2i, bool zero, bool prolong,
+                      bool resid, const T *uc, T *rc, double *resmax)
+{
+    if (resid && zero) stream_one<SS, NS, true, false, true, T>(s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+    else if (resid) stream_one<SS, NS, false, false, true, T>(s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+    else if (prolong) stream_one<SS, NS, false, true, false, T>(s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+    else if (zero) stream_one<SS, NS, true, false, false, T>(s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+    else stream_one<SS, NS, false, false, false, T>(s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+}
+
 template <class SS, typename T>
-static void stream_variant(hipStream_t s, const T *uin, T *uout, const T *f, int n, T h2, T h2i,
-                           bool zero, bool prolong, bool resid, const T *uc, T *rc, double *resmax)
+static void stream_variant(hipStream_t s, int ns, const T *uin, T *uout, const T *f, int n, T h2, T h2i, bool zero,
+                           bool prolong, bool resid, const T *uc, T *rc, double *resmax)
 {
     if constexpr (stream_built<SS, T>()) {
-        const int ntiles = (n / SS::SX) * (n / SS::SY) * (n / SS::ZC);
-        const dim3 grid(8 * ((ntiles + 7) / 8)), block(SS::NT);
-        if (resid && zero)
-            hipLaunchKernelGGL((k_sweep_stream<SS, true, false, true, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
-        else if (resid)
-            hipLaunchKernelGGL((k_sweep_stream<SS, false, false, true, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
-        else if (prolong)
-            hipLaunchKernelGGL((k_sweep_stream<SS, false, true, false, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
-        else if (zero)
-            hipLaunchKernelGGL((k_sweep_stream<SS, true, false, false, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
-        else
-            hipLaunchKernelGGL((k_sweep_stream<SS, false, false, false, T>), grid, block, 0, s, uin, uout, f, n, h2, h2i, uc, rc, resmax);
+        if (ns == 2) stream_ns<SS, 2, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax);
+        else stream_ns<SS, 1, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax);
     }
 }
 
+// ns (1 or 2) fused red-black sweeps of a fine level (n >= 32) with shape cfg, the source staged in LDS
+// when fs (tiles): uin -> uout.
 template <typename T>
 static int launch_sweep_cfg(hipStream_t s, int cfg, int ns, bool fs, const T *uin, T *uout, const T *f,
                             int n, double h, bool zero, bool prolong, bool resid, const T *uc, T *rc,
@@ -338,15 +349,15 @@ static int launch_sweep_cfg(hipStream_t s, int cfg, int ns, bool fs, const T *ui
     SG_REQUIRE(cfg_ok<T>(cfg, ns, fs), "sweep shape %d with %d sweeps (staged %d) does not exist", cfg, ns, (int)fs);
     const T h2 = (T)(h * h), h2i = (T)(1.0 / (h * h));
     switch (cfg) {
-    case kNumTiles + 0: stream_variant<Stream0, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 1: stream_variant<Stream1, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 2: stream_variant<Stream2, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 3: stream_variant<Stream3, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 4: stream_variant<Stream4, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 5: stream_variant<Stream5, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 6: stream_variant<Stream6, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 7: stream_variant<Stream7, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 8: stream_variant<Stream8, T>(s, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 0: stream_variant<Stream0, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 1: stream_variant<Stream1, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 2: stream_variant<Stream2, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 3: stream_variant<Stream3, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 4: stream_variant<Stream4, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 5: stream_variant<Stream5, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 6: stream_variant<Stream6, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 7: stream_variant<Stream7, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 8: stream_variant<Stream8, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case 0: sweep_ns<Tile0, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case 1: sweep_ns<Tile1, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case 2: sweep_ns<Tile2, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
@@ -368,7 +379,7 @@ static int level_of(const sg_uniform *c, int n)
 template <typename T> static int level_ns(sg_uniform *c, int l)
 {
     if constexpr (std::is_same<T, float>::value) return c->tile_ns[l];
-    else return fp64_two_sweeps(n3(c->nl[l])) ? 2 : 1;
+    else return kMaxSweepsPerLaunch;
 }
 
 template <typename T>
@@ -379,7 +390,7 @@ static int launch_sweep(sg_uniform *c, int l, int ns, const T *uin, T *uout, boo
     int cfg = c->tile_cfg[l];
     bool fs = c->tile_fs[l] != 0;
     if constexpr (std::is_same<T, double>::value) {
-        cfg = fp64_sweep_shape(n >= 64 ? 64 : n, n3(n), fp64_two_sweeps(n3(n)));
+        cfg = fp64_sweep_shape(n >= 64 ? 64 : n, n3(n));
         fs = false;
     }
     return launch_sweep_cfg<T>(c->stream, cfg, ns, fs, uin, uout, levels<T>(c).RHO[l], n, c->hl[l], zero, prolong,

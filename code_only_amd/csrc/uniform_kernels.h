@@ -23,6 +23,18 @@ template <> struct Consts<float> {
     static __device__ __forceinline__ float sixth() { return 1.0f / 6.0f; }
 };
 
+__device__ __forceinline__ int wrapn(int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); }
+
+// Tile index with XCD-aware placement: consecutive workgroups are dealt round-robin to the 8
+// XCDs, so workgroup b is given tile (b % 8) * per + b / 8 -- each XCD works through a contiguous
+// range of tiles (z-slabs), and the halos its tiles share stay in that XCD's L2.
+__device__ __forceinline__ int xcd_tile(int ntiles)
+{
+    const int per = (ntiles + 7) / 8;
+    const int b = (int)blockIdx.x;
+    return (b % 8) * per + b / 8;
+}
+
 // ---- per-cell arithmetic shared by every kernel (plain, fused, single-workgroup) -------------
 // Operand order is the reference's: x+, x-, y+, y-, z+, z- neighbours, then -6u, then the source.
 

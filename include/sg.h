@@ -140,7 +140,7 @@ int sg_uniform_time_smoother(sg_uniform *ctx, int prec, int reps, double *ms_per
  * cycle (two sweeps ending with the residual restriction, two starting with the prolongated
  * correction) of every candidate (-1 where it does not fit): 29 candidates, the LDS tiles first,
  * indexed tile * 4 + (sweeps - 1) * 2 + staged (cfg 0..4), then the nine streaming shapes
- * (cfg 5..13, one sweep per launch). */
+ * (cfg 5..13, timed with two sweeps per launch). */
 int sg_uniform_tile_info(sg_uniform *ctx, int level, int *cfg, int *ns, int *fs, float *ms, int nms);
 /* Override the autotuner's choice for fused-sweep level `level` (same meaning of cfg / ns / fs;
  * values do not depend on the choice). */

@@ -280,7 +280,7 @@ def test_exact_coarse_solve_contracts_at_least_as_well(gpu, n):
     s.close()
 
 
-STREAM_CFGS = list(range(5, 14))   # streaming sweep shapes (one or two planes per step)
+STREAM_CFGS = list(range(5, 14))   # streaming sweep shapes
 
 
 @pytest.mark.parametrize("n", [32, 64, 128])
@@ -314,6 +314,37 @@ def test_every_sweep_shape_bitwise(gpu, n, cfg):
     s.close()
 
 
+@pytest.mark.parametrize("npre,npost", [(2, 2), (3, 1)])
+@pytest.mark.parametrize("n", [32, 64, 128])
+@pytest.mark.parametrize("cfg", STREAM_CFGS)
+def test_streams_of_two_sweeps_bitwise(gpu, n, cfg, npre, npost):
+    """The streaming shapes with two sweeps per launch (and the odd sweep alone), forced where they
+    fit, against the unfused FP32 solve, bit for bit; columns that meet their own periodic images
+    (n equal to the shape's width) included."""
+    s = UniformSolver(n, precisions=SG_PREC_MIXED)
+    ft = T(problems.clumpy_rhs(n, seed=14), gpu)
+    forced, lev, m = 0, 0, n
+    while m > 16:
+        try:
+            s.set_tile(lev, cfg, 2, 0)
+            forced += 1
+        except Exception:
+            pass
+        lev += 1
+        m //= 2
+    if not forced:
+        pytest.skip(f"configuration {cfg} fits no level of n = {n}")
+    res = []
+    for fused in (False, True):
+        psi = torch.zeros_like(ft)
+        st = s.cycle(psi, ft, tol=1e-10, maxit=30, precision=SG_PREC_MIXED, fused=fused, npre=npre, npost=npost,
+                     stop_mode=SG_STOP_REFERENCE, raise_on_fail=False)
+        res.append((psi, st))
+    assert torch.equal(res[0][0], res[1][0])
+    assert res[0][1]["resmaxg"] == res[1][1]["resmaxg"]
+    s.close()
+
+
 @pytest.mark.parametrize("npre,npost,ncycle", [(1, 1, 1), (3, 2, 2), (2, 3, 1)])
 def test_fused_other_cycle_shapes_bitwise(gpu, npre, npost, ncycle):
     n = 64
@@ -335,7 +366,7 @@ def test_fused_other_cycle_shapes_bitwise(gpu, npre, npost, ncycle):
 @pytest.mark.parametrize("n", [2, 4, 8, 16, 32, 64, 128, 256])
 def test_fp64_fused_equals_plain(n, cycle, gpu):
     """The fused FP64 solve (k_coarse below 16^3, every sweep shape of the rule: tiles of two sweeps at
-    32 and 64, a tile at 128, streams at 256; odd sweep counts) against one kernel per loop nest,
+    32 and 64, streams of two sweeps at 128 and 256; odd sweep counts) against one kernel per loop nest,
     bit for bit, in both stopping modes, and again with other phi and source arrays (the graph is
     the context's own)."""
     import torch
