@@ -393,7 +393,7 @@ template <int N, typename T> int prep_n(sg_amr &s, int L, int ju)
 {
     constexpr int H = N / 2;
     const int ncov = s.prep_ncov[L], ncf = (int)s.cf.size();
-    const long work = (long)ncov + (long)ncf * H * H;
+    const long work = prep_quads(ncov) + 4 * (long)ncf * H * H;
     LevelScalars hil{};
     for (int l = 0; l < kMaxLev; ++l) hil.v[l] = s.hil[L][l];
     if constexpr (N == 8 && std::is_same<T, float>::value) {

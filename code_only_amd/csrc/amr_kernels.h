@@ -501,24 +501,25 @@ template <int N, typename T> __device__ __forceinline__ T rstr_at(const T *A, lo
     return s * (T)(1.0 / 8.0);
 }
 
-template <int N, typename T> __device__ __forceinline__ T src_val(const T *A, int s)
-{
-    return s >= 0 ? A[s] : rstr_at<N, T>(A, -(long)s - 1);
-}
-
-
 // One launch per refresh.  Items [0, ncov): the covered blocks' face layers that same-level leaf
-// neighbours read (cov[t] = {destination, restriction origin}).  Items [ncov, + ncf H^2): one coarse
-// face cell (c1, c2) of coarse-fine face e each: the four fine ghost cells behind it
+// neighbours read (cov[t] = {destination, restriction origin}).  Items from prep_quads(ncov) on, 4 ncf H^2:
+// one fine ghost cell (q1, q2) behind coarse face cell (c1, c2) of coarse-fine face e each
 // (fmg_ghfix_parentlev: bilinear (9,3,3,1)/16 tangentially, then (10 u0 + 8 uH - 3 uN)/15 normally,
-// the operand order of k_ghost) and the reflux override of the coarse neighbour there (the 2x2
-// average of the fine face fluxes, the order of k_reflux).  rec[e] = {fine block, face + 8 octant,
-// override slot, AMR level}; src + e (H+2)^2 holds the sources of the coarse neighbour's face layer
-// at tangential coarse positions -1..H (the fine block's quarter of it, ghosts included).
-// Reads only leaf interiors and physical ghost cells, which no item writes.
+// the operand order of k_ghost); the four lanes of a face cell then form the reflux override of the
+// coarse neighbour there (the 2x2 average of the fine face fluxes, the order of k_reflux).  rec[e] =
+// {fine block, face + 8 octant, override slot, AMR level}; src + e (H+2)^2 holds the sources of the coarse
+// neighbour's face layer at tangential coarse positions -1..H (the fine block's quarter of it, ghosts
+// included).  Reads only leaf interiors and physical ghost cells, which no item writes.
+// Bound by its chain of dependent loads (source index, value, store) on launches of few items, so a lane
+// takes one ghost cell and its four sources are loaded together, the restricted ones after a branch that
+// few waves take; with one lane per coarse face cell, nine sources by branches and four ghost cells one
+// after the other, a launch took 6.9 us (FP32 4^3) and 6.1 (8^3 compact): an adjoint pass over an 8^3-block
+// hierarchy of two levels (1 590 such launches) 42.7 -> 36.8 ms, the mixed solve of 20 480 blocks 21.2 -> 20.5.
 // CC: the compact level-0 form of the inner solve (N = 8, T = float; A the compact interiors by
 // active-list position, the tables of build_compact_tables): covered items write their value to the
 // ghost store gs at cov[t].x, the fine ghosts go there too (aidx: the blocks' active positions).
+__host__ __device__ constexpr long prep_quads(long ncov) { return (ncov + 3) / 4 * 4; }
+
 template <int N, typename T, bool CC = false>
 __global__ void k_prep(T *A, T *ov, const int2 *cov, int ncov, const int4 *rec, const int *src, int ncf,
                        LevelScalars hil, T *gs = nullptr, const int *aidx = nullptr)
@@ -527,7 +528,8 @@ __global__ void k_prep(T *A, T *ov, const int2 *cov, int ncov, const int4 *rec, 
     constexpr int H = N / 2, S = H + 2;
     static_assert(!CC || (N == 8 && std::is_same<T, float>::value), "the compact form is FP32 8^3");
     long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < ncov) {
+    if (t < prep_quads(ncov)) {
+        if (t >= ncov) return;
         const int2 p = cov[t];
         if constexpr (CC) {
             gs[p.x] = rstr_cc(A, p.y);
@@ -536,54 +538,57 @@ __global__ void k_prep(T *A, T *ov, const int2 *cov, int ncov, const int4 *rec, 
         A[p.x] = rstr_at<N, T>(A, p.y);
         return;
     }
-    t -= ncov;
+    t -= prep_quads(ncov);
+    const int q1 = (int)(t & 1), q2 = (int)((t >> 1) & 1);   // a face cell's four lanes are in one wave
+    t >>= 2;
     if (t >= (long)ncf * H * H) return;
     const int c1 = (int)(t % H), c2 = (int)((t / H) % H), e = (int)(t / (H * H));
-    const int *sr = src + (long)e * S * S;
-    // the 3x3 coarse neighbourhood the four fine ghosts interpolate from
-    T w[3][3];
-#pragma unroll
-    for (int y = 0; y < 3; ++y)
-#pragma unroll
-        for (int x = 0; x < 3; ++x) {
-            const int so = sr[(c2 + y) * S + (c1 + x)];
-            if constexpr (CC) {
-                w[y][x] = so >= 0 ? A[so] : (so == -1 ? (T)0 : rstr_cc(A, -so - 2));
-            } else {
-                w[y][x] = src_val<N, T>(A, so);
-            }
-        }
+    // sources: the coarse cell behind the ghost, and its neighbours one coarse cell down (q = 0) or up (q = 1)
+    const int *sr = src + (long)e * S * S + (c2 + 1) * S + c1 + 1;
+    const int n1 = 2 * q1 - 1, n2 = (2 * q2 - 1) * S;
+    const int so[4] = {sr[0], sr[n2 + n1], sr[n2], sr[n1]};
     const int4 r = rec[e];
     const int b = r.x, f = r.y & 7, o = r.y >> 3, d = f >> 1, lr = f & 1;
     const int ag = lr ? N : -1, inner = lr ? -1 : 1;
     const int ab = CC ? aidx[b] : b;   // the block's position in A
     T *u = A + (long)ab * (CC ? 512 : B::LEN);
-    const T hi = (T)hil.v[r.w];
-    T ffv[2][2];
+    const int s1 = 2 * c1 + q1, s2 = 2 * c2 + q2;
+    const T u0 = u[CC ? cc_rot(d, ag + inner, s1, s2) : B::rot(d, ag + inner, s1, s2)];
+    const T uN = u[CC ? cc_rot(d, ag + 2 * inner, s1, s2) : B::rot(d, ag + 2 * inner, s1, s2)];
+    T w[4];
 #pragma unroll
-    for (int q2 = 0; q2 < 2; ++q2)
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (CC) w[i] = so[i] >= 0 ? A[so[i]] : (T)0;
+        else w[i] = A[so[i] >= 0 ? (long)so[i] : -(long)so[i] - 1];
+    }
+    if (min(min(so[0], so[1]), min(so[2], so[3])) < (CC ? -1 : 0)) {
 #pragma unroll
-        for (int q1 = 0; q1 < 2; ++q1) {
-            const int s1 = 2 * c1 + q1, s2 = 2 * c2 + q2;
-            // buf(cc, cc) is w[1][1]; the near neighbour is one coarse cell down (q = 0) or up (q = 1)
-            const int n1 = 2 * q1, n2 = 2 * q2;
-            T Sv = (T)9.0 * w[1][1] + w[n2][n1];
-            Sv = Sv + (T)3.0 * w[n2][1];
-            Sv = Sv + (T)3.0 * w[1][n1];
-            const T uH = Sv / (T)16.0;
-            const T u0 = u[CC ? cc_rot(d, ag + inner, s1, s2) : B::rot(d, ag + inner, s1, s2)];
-            const T uN = u[CC ? cc_rot(d, ag + 2 * inner, s1, s2) : B::rot(d, ag + 2 * inner, s1, s2)];
-            T q = (T)10.0 * u0 + (T)8.0 * uH;
-            q = q - (T)3.0 * uN;
-            const T g = q / (T)15.0;
-            if constexpr (CC) gs[((long)ab * 6 + f) * 64 + gs_cell(f, s1, s2)] = g;
-            else u[B::rot(d, ag, s1, s2)] = g;
-            // face flux (u(af + 1) - u(af)) hi with af = -1 (left face) or N - 1 (right face)
-            ffv[q1][q2] = lr ? (g - u0) * hi : (u0 - g) * hi;
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (CC) {
+                if (so[i] < -1) w[i] = rstr_cc(A, -so[i] - 2);
+            } else {
+                if (so[i] < 0) w[i] = rstr_at<N, T>(A, -(long)so[i] - 1);
+            }
         }
-    T v = ffv[0][0] + ffv[0][1];
-    v = v + ffv[1][0];
-    v = v + ffv[1][1];
+    }
+    T Sv = (T)9.0 * w[0] + w[1];
+    Sv = Sv + (T)3.0 * w[2];
+    Sv = Sv + (T)3.0 * w[3];
+    const T uH = Sv / (T)16.0;
+    T q = (T)10.0 * u0 + (T)8.0 * uH;
+    q = q - (T)3.0 * uN;
+    const T g = q / (T)15.0;
+    if constexpr (CC) gs[((long)ab * 6 + f) * 64 + gs_cell(f, s1, s2)] = g;
+    else u[B::rot(d, ag, s1, s2)] = g;
+    // face flux (u(af + 1) - u(af)) hi with af = -1 (left face) or N - 1 (right face)
+    const T hi = (T)hil.v[r.w];
+    const T ff = lr ? (g - u0) * hi : (u0 - g) * hi;
+    // (q1, q2) = (0, 0), (0, 1), (1, 0), (1, 1): lanes 0, 2, 1, 3
+    const T f01 = __shfl_xor(ff, 2), f10 = __shfl_xor(ff, 1), f11 = __shfl_xor(ff, 3);
+    if (q1 | q2) return;
+    T v = ff + f01;
+    v = v + f10;
+    v = v + f11;
     const int ta = d == 0 ? 1 : 0, tb = d == 2 ? 1 : 2;
     const int off1 = ((o >> ta) & 1) * H, off2 = ((o >> tb) & 1) * H;
     ov[(long)r.z * N * N + (off1 + c1) + N * (off2 + c2)] = v * (T)0.25;
