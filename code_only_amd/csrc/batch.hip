@@ -231,7 +231,7 @@ template <typename T>
 int op_sweep_cfg(sg_batch *c, const Pairs &pl, int cfg, int ns, bool fs, int cin, int cout, int cuc, bool zero,
                  bool prolong, bool resid)
 {
-    SG_REQUIRE(cfg >= 0 && cfg < kNumCfg && cfg_ok<T>(cfg, ns, fs), "bad sweep configuration %d/%d/%d", cfg, ns, (int)fs);
+    SG_REQUIRE(cfg >= 0 && cfg < kNumCfg && cfg_timed(cfg) && cfg_ok<T>(cfg, ns, fs), "bad sweep configuration %d/%d/%d", cfg, ns, (int)fs);
     const int *td = cfg < kNumTiles ? kTileDims[cfg] : kStreamDims[cfg - kNumTiles];
     for (auto &q : pl) {
         SG_REQUIRE(q.second < c->lc[q.first], "batch schedule: fused sweep on a coarse-kernel level");
@@ -249,14 +249,14 @@ int op_sweep_cfg(sg_batch *c, const Pairs &pl, int cfg, int ns, bool fs, int cin
     const BL<T> L = bl<T>(c, d, cnt);
     switch (cfg) {
     case kNumTiles + 0: stream_variant<Stream0, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 1: stream_variant<Stream1, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case kNumTiles + 2: stream_variant<Stream2, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 3: stream_variant<Stream3, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case kNumTiles + 4: stream_variant<Stream4, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case kNumTiles + 5: stream_variant<Stream5, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
-    case kNumTiles + 6: stream_variant<Stream6, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case kNumTiles + 7: stream_variant<Stream7, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case kNumTiles + 8: stream_variant<Stream8, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 9: stream_variant<Stream9, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 10: stream_variant<Stream10, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
+    case kNumTiles + 11: stream_variant<Stream11, T>(c, ns, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case 0: sweep_ns<Tile0, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case 1: sweep_ns<Tile1, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
     case 2: sweep_ns<Tile2, T>(c, ns, fs, L, tot, cin, cout, cuc, zero, prolong, resid); break;
@@ -591,7 +591,7 @@ int autotune(sg_batch *c)
             int cfg, ns;
             bool fs;
             cand_decode(cand, cfg, ns, fs);
-            bool fits = cfg_ok<float>(cfg, ns, fs);
+            bool fits = cfg_timed(cfg) && cfg_ok<float>(cfg, ns, fs);
             for (auto &q : Mv) fits = fits && cfg_fits(cfg, c->h_pl32[q.first * kBLev + v].n);
             c->tune_ms[v][cand] = -1.f;
             if (!fits) continue;

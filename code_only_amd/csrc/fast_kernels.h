@@ -318,23 +318,35 @@ k_sweep_tile(const T *__restrict__ uin, T *__restrict__ uout, const T *__restric
 // Streaming shapes (pair_stream.h) the autotuners choose from beside the tiles, with two sweeps per launch
 // (one where a single sweep is left): column SX x SY, chunk of ZC planes.  A longer chunk spends less on
 // its halo planes, a shorter one makes more workgroups: 512^3 is fastest with 128 planes, 256^3 with 64.
+// A shape's number is public (sg_uniform_set_tile) and fixes the widths it takes, the multiples of its
+// largest extent: shapes are appended, never renumbered.  Numbers 2 and 4 (Stream2, Stream4) once named
+// columns of 64 x 32 and 128 x 16, whose pairs exceed a workgroup, and take their widths (4 also 64).  Numbers 1, 3
+// and 6 are there for callers that hold them; the autotuners do not time them (their longer or wider
+// neighbours spend less on halos at the same widths).
 using Stream0 = StreamShape<64, 16, 32>;
-using Stream1 = StreamShape<64, 16, 64>;
-using Stream2 = StreamShape<64, 16, 128>;
-using Stream3 = StreamShape<32, 32, 32>;
+using Stream1 = StreamShape<64, 16, 16>;
+using Stream2 = StreamShape<64, 16, 64>;
+using Stream3 = StreamShape<32, 16, 32>;
 using Stream4 = StreamShape<32, 32, 64>;
 using Stream5 = StreamShape<32, 16, 16>;
-using Stream6 = StreamShape<32, 16, 64>;
-using Stream7 = StreamShape<16, 16, 16>;
-using Stream8 = StreamShape<16, 8, 8>;
-constexpr int kNumStream = 9;
-static const int kStreamDims[kNumStream][3] = {{64, 16, 32}, {64, 16, 64}, {64, 16, 128}, {32, 32, 32}, {32, 32, 64},
-                                               {32, 16, 16}, {32, 16, 64}, {16, 16, 16},  {16, 8, 8}};
+using Stream6 = StreamShape<32, 8, 16>;
+using Stream7 = StreamShape<32, 32, 32>;
+using Stream8 = StreamShape<16, 16, 16>;
+using Stream9 = StreamShape<64, 16, 128>;
+using Stream10 = StreamShape<32, 16, 64>;
+using Stream11 = StreamShape<16, 8, 8>;
+constexpr int kNumStream = 12;
+static const int kStreamDims[kNumStream][3] = {
+    {64, 16, 32}, {64, 16, 16}, {64, 16, 64}, {32, 16, 32}, {32, 32, 64},  {32, 16, 16},
+    {32, 8, 16},  {32, 32, 32}, {16, 16, 16}, {64, 16, 128}, {32, 16, 64}, {16, 8, 8}};
 
 // sweep configurations: 0 .. kNumTiles-1 tiles, kNumTiles .. kNumTiles+kNumStream-1 streams
 constexpr int kNumCfg = kNumTiles + kNumStream;
 constexpr int kNumCand = kNumTiles * kMaxSweepsPerLaunch * 2 + kNumStream;
 static_assert(kNumCand <= 32, "autotuner timing tables hold 32 candidates");
+
+// whether the autotuners time configuration cfg
+inline bool cfg_timed(int cfg) { return cfg != kNumTiles + 1 && cfg != kNumTiles + 3 && cfg != kNumTiles + 6; }
 
 inline bool cfg_fits(int cfg, int n)
 {
@@ -353,7 +365,7 @@ template <class TL, int NS, bool FS, typename T> constexpr bool sweep_built()
 }
 template <class SS, typename T> constexpr bool stream_built()
 {
-    return sizeof(T) == sizeof(float) || (SS::SX == 32 && SS::SY == 16);
+    return sizeof(T) == sizeof(float) || (SS::SX == 32 && SS::SY == 16 && SS::ZC != 32);
 }
 template <class SS, typename T> constexpr bool stream_built_fits()
 {
@@ -364,10 +376,10 @@ template <class TL, int NS, bool FS, typename T> constexpr bool sweep_built_fits
     return !sweep_built<TL, NS, FS, T>() || sweep_fits_lds<TL, NS, FS, T>();
 }
 static_assert(sweep_built_fits<Tile1, 2, false, double>() && sweep_built_fits<Tile4, 2, false, double>() &&
-                  stream_built_fits<Stream5, double>() && stream_built_fits<Stream6, double>(),
+                  stream_built_fits<Stream5, double>() && stream_built_fits<Stream10, double>(),
               "FP64 sweep shapes exceed the LDS");
-static_assert(stream_built_fits<Stream0, float>() && stream_built_fits<Stream3, float>() &&
-                  stream_built_fits<Stream5, float>() && stream_built_fits<Stream7, float>(),
+static_assert(stream_built_fits<Stream0, float>() && stream_built_fits<Stream5, float>() &&
+                  stream_built_fits<Stream7, float>() && stream_built_fits<Stream8, float>(),
               "FP32 streaming shapes exceed the LDS or a workgroup");
 
 // The FP64 sweep shape of a launch, always of two sweeps where two are left, over levels whose widths are
@@ -380,7 +392,7 @@ static_assert(stream_built_fits<Stream0, float>() && stream_built_fits<Stream3, 
 constexpr long kSweepCUs = 256;
 inline int fp64_sweep_shape(int unit, long cells)
 {
-    if (unit >= 64 && cells >= kSweepCUs * 32 * 16 * 64) return kNumTiles + 6;
+    if (unit >= 64 && cells >= kSweepCUs * 32 * 16 * 64) return kNumTiles + 10;
     if (unit >= 32 && cells >= kSweepCUs * 32 * 16 * 16) return kNumTiles + 5;
     return unit >= 16 && cells >= kSweepCUs * 16 * 8 * 8 ? 1 : 4;
 }
@@ -418,6 +430,9 @@ template <typename T> inline bool cfg_ok(int cfg, int ns, bool fs)
     case 6: return stream_built<Stream6, T>();
     case 7: return stream_built<Stream7, T>();
     case 8: return stream_built<Stream8, T>();
+    case 9: return stream_built<Stream9, T>();
+    case 10: return stream_built<Stream10, T>();
+    case 11: return stream_built<Stream11, T>();
     default: return false;
     }
 }

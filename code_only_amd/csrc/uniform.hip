@@ -358,6 +358,9 @@ static int launch_sweep_cfg(hipStream_t s, int cfg, int ns, bool fs, const T *ui
     case kNumTiles + 6: stream_variant<Stream6, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case kNumTiles + 7: stream_variant<Stream7, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case kNumTiles + 8: stream_variant<Stream8, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 9: stream_variant<Stream9, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 10: stream_variant<Stream10, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 11: stream_variant<Stream11, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case 0: sweep_ns<Tile0, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case 1: sweep_ns<Tile1, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case 2: sweep_ns<Tile2, T>(s, ns, fs, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
@@ -418,7 +421,7 @@ static int autotune_tiles(sg_uniform *c)
             bool fs;
             cand_decode(cand, cfg, ns, fs);
             c->tune_ms[l][cand] = -1.f;
-            if (!cfg_fits(cfg, n) || !cfg_ok<float>(cfg, ns, fs)) continue;
+            if (!cfg_timed(cfg) || !cfg_fits(cfg, n) || !cfg_ok<float>(cfg, ns, fs)) continue;
             const int reps = n >= 256 ? 3 : 6;  // timed visits, after one untimed
             int flip = 0;
             auto launch = [&](int k, bool prolong, bool resid) {

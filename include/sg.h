@@ -138,12 +138,15 @@ int sg_uniform_time_smoother(sg_uniform *ctx, int prec, int reps, double *ms_per
  * chosen for MG level `level` of a context created with SG_PREC_MIXED (cfg -1 for levels solved
  * inside the single-workgroup coarse kernel) and the measured ms per fine-level visit of a V(2,2)
  * cycle (two sweeps ending with the residual restriction, two starting with the prolongated
- * correction) of every candidate (-1 where it does not fit): 29 candidates, the LDS tiles first,
- * indexed tile * 4 + (sweeps - 1) * 2 + staged (cfg 0..4), then the nine streaming shapes
- * (cfg 5..13, timed with two sweeps per launch). */
+ * correction) of every candidate (-1 where it does not fit or is not timed): 32 candidates, the LDS
+ * tiles first, indexed tile * 4 + (sweeps - 1) * 2 + staged (cfg 0..4), then the twelve streaming
+ * shapes at 20 + cfg - 5, timed with two sweeps per launch: column and planes, cfg 5 64x16x32, 6
+ * 64x16x16 (not timed), 7 64x16x64, 8 32x16x32 (not timed), 9 32x32x64, 10 32x16x16, 11 32x8x16 (not
+ * timed), 12 32x32x32, 13 16x16x16, 14 64x16x128, 15 32x16x64, 16 16x8x8. */
 int sg_uniform_tile_info(sg_uniform *ctx, int level, int *cfg, int *ns, int *fs, float *ms, int nms);
-/* Override the autotuner's choice for fused-sweep level `level` (same meaning of cfg / ns / fs;
- * values do not depend on the choice). */
+/* Override the autotuner's choice for fused-sweep level `level` (same meaning of cfg / ns / fs; values
+ * do not depend on the choice).  A cfg fits the levels whose width is a multiple of its largest extent;
+ * the numbers keep that meaning (a shape may be replaced by one that fits the same widths). */
 int sg_uniform_set_tile(sg_uniform *ctx, int level, int cfg, int ns, int fs);
 
 /* ---------------------------------------------------------------------------------------------
@@ -357,7 +360,8 @@ int sg_batch_solve_dev(sg_batch *ctx, double *const *psi, const double *const *s
 
 /* Chosen fused-sweep shape of fine level `level` (configuration index as sg_uniform_tile_info's,
  * sweeps per launch, source staged in LDS), tricubic tile x extent, and the timings (ms per
- * fine-level visit of a V(2,2) cycle, -1 = did not fit) of the 29 candidates. */
+ * fine-level visit of a V(2,2) cycle, -1 = did not fit) of the candidates of
+ * sg_uniform_tile_info. */
 int sg_batch_tile_info(sg_batch *ctx, int level, int *cfg, int *ns, int *fs, int *cubic_fx, float *ms, int nms);
 /* Number of levels of problem `prob` and its first level held by the coarse kernel. */
 int sg_batch_levels(sg_batch *ctx, int prob, int *nlev, int *first_coarse);

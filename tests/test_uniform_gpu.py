@@ -11,6 +11,7 @@ import torch
 import oracle
 from oracle import fft_poisson as fp
 from code_only_amd import problems
+from code_only_amd._lib import SgError
 from code_only_amd.uniform import (SG_COARSE_EXACT, SG_COARSE_VCYCLE, SG_PREC_FP64, SG_PREC_MIXED,
                                    SG_STOP_REFERENCE, SG_STOP_TRUE_RESIDUAL, UniformSolver)
 
@@ -314,9 +315,24 @@ def test_every_sweep_shape_bitwise(gpu, n, cfg):
     s.close()
 
 
+@pytest.mark.parametrize("cfg", STREAM_CFGS)
+def test_stream_numbers_keep_their_widths(gpu, cfg):
+    """A streaming shape's number takes every level width it has taken, whatever shape stands behind it."""
+    narrowest = {5: 64, 6: 64, 7: 64, 8: 32, 9: 64, 10: 32, 11: 32, 12: 32, 13: 32}[cfg]
+    s = UniformSolver(128, precisions=SG_PREC_MIXED)
+    for lev, m in ((0, 128), (1, 64), (2, 32)):
+        if m >= narrowest:
+            s.set_tile(lev, cfg, 1, 0)
+            assert s.tile_info(lev)["cfg"] == cfg
+        else:
+            with pytest.raises(SgError):
+                s.set_tile(lev, cfg, 1, 0)
+    s.close()
+
+
 @pytest.mark.parametrize("npre,npost", [(2, 2), (3, 1)])
 @pytest.mark.parametrize("n", [32, 64, 128])
-@pytest.mark.parametrize("cfg", STREAM_CFGS)
+@pytest.mark.parametrize("cfg", STREAM_CFGS + [14, 15, 16])
 def test_streams_of_two_sweeps_bitwise(gpu, n, cfg, npre, npost):
     """The streaming shapes with two sweeps per launch (and the odd sweep alone), forced where they
     fit, against the unfused FP32 solve, bit for bit; columns that meet their own periodic images
