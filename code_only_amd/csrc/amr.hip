@@ -185,16 +185,17 @@ struct sg_amr {
     sg_blockmem bml{};
     int have_bm = 0;
     int *d_slot_u = nullptr, *d_slot_u1 = nullptr, *d_slot_u2 = nullptr;
-    // the hydro steps' item tables (build_hydro_tables, on first use): exchange items per (level,
+    // the hydro steps' item tables (each kind built by its first call): exchange items per (level,
     // direction), restriction items per fine level, refluxing items per coarse level grouped in
     // rounds of disjoint coarse cells
-    int hydro_ready = 0;
+    int hx_ready = 0, fg_ready = 0, rf_ready = 0;
     int4 *d_hx = nullptr, *d_fg = nullptr, *d_rf = nullptr;
     std::vector<int> hx_off, fg_off;
-    // the same exchanges resolved per ghost region (k_hx_fill), 27 entries per block: [0] a level's own
-    // exchange, [1] its same-level part on all arrays; hx_one: levels where the resolved form holds
-    int2 *d_hxe[2] = {};
-    std::vector<int> hx_one[2];
+    // the exchanges resolved per ghost region (k_hx_fill): 27 entries per block for a level's own exchange,
+    // then 27 per block for its same-level part on all arrays, then per form and level whether it takes the
+    // staged passes (items of those levels only in d_hx)
+    int2 *d_hxe = nullptr;
+    std::vector<int> hx_staged;
     std::vector<std::vector<int>> rf_rounds;   // per coarse level: offsets of its rounds, + end
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1810,7 +1811,7 @@ void release(sg_amr *s)
     for (int *q : ip) if (q) (void)hipFree(q);
     if (s->d_crop) (void)hipFree(s->d_crop);
     for (int4 *q : {s->d_hx, s->d_fg, s->d_rf}) if (q) (void)hipFree(q);
-    for (int2 *q : s->d_hxe) if (q) (void)hipFree(q);
+    if (s->d_hxe) (void)hipFree(s->d_hxe);
     if (s->rhs0c) (void)hipFree(s->rhs0c);
     for (float *q : {s->u0c, s->res0c, s->gs0}) if (q) (void)hipFree(q);
     for (long *q : {s->d_at_ptr, s->d_bt_ptr}) if (q) (void)hipFree(q);
@@ -2843,75 +2844,34 @@ int sg_amr_op(sg_amr *ctx, int opc, int fmglev, int a, int b, int c, int flag, d
 namespace {
 int upload4(sg_amr &s, int4 **dptr, const std::vector<int4> &v)
 {
+    if (*dptr) (void)hipFree(*dptr);   // of a call that failed after it
+    *dptr = nullptr;
     SG_HIP(hipMalloc((void **)dptr, std::max<size_t>(1, v.size()) * sizeof(int4)));
     if (!v.empty()) SG_HIP(hipMemcpy(*dptr, v.data(), v.size() * sizeof(int4), hipMemcpyHostToDevice));
     return SG_OK;
 }
 
-// What face f of block b holds for the exchange: 0 nothing, 1 a same-level neighbour, 2 the coarse grid
-// of the parent's face (interpolation; nothing with same_only); *src: that grid.
-int hx_face(const sg_amr &s, int b, int f, int same_only, int *src)
+// The exchange's tables, on its first call for a hierarchy: the source of every ghost region by k_hx_table
+// from the block tables on the device, and the pass items of the levels that keep the staged passes.
+int build_exchange_tables(sg_amr &s)
 {
-    const int l = s.level[b], m = s.nbr[6 * b + f];
-    if (m >= 0 && s.level[m] == l) {
-        *src = m;
-        return 1;
-    }
-    if (l == 0 || same_only) return 0;
-    const int g = s.nbr[6 * s.parent[b] + f];
-    *src = g;
-    return g >= 0 && s.level[g] == l - 1 ? 2 : 0;
-}
-
-// The source of ghost region `side` (-1, 0, 1 per axis) of block b after the x, y, z passes, as
-// k_hx_fill reads it.  Returns 0 where the chain ends at a ghost cell that a pass of the same launch
-// writes (an inner corner of the refined region in the same-level part): the staged passes then
-// see an older value there.
-int hx_resolve(const sg_amr &s, int b, const int side[3], int same_only, int2 *out)
-{
-    int q = b, src = -1, moved = 0;
-    for (int d = 2; d >= 0; --d) {
-        if (side[d] == 0) continue;
-        const int lr = side[d] > 0, kind = hx_face(s, q, 2 * d + lr, same_only, &src);
-        if (kind == 2) {
-            *out = make_int2(src, moved | 8 | (d << 4) | (lr << 6) | (s.octant[q] << 7));
-            return 1;
-        }
-        if (kind == 1) {
-            q = src;
-            moved |= 1 << d;
-        }
-    }
-    if (!moved) {
-        *out = make_int2(-1, 0);
-        return 1;
-    }
-    for (int d = 0; d < 3; ++d)
-        if (side[d] != 0 && !((moved >> d) & 1) && hx_face(s, q, 2 * d + (side[d] > 0), same_only, &src)) return 0;
-    *out = make_int2(q, moved);
-    return 1;
-}
-
-int build_hydro_tables(sg_amr &s)
-{
-    if (s.hydro_ready) return SG_OK;
-    for (int so = 0; so < 2; ++so) {
-        std::vector<int2> ent((size_t)27 * s.nblk, make_int2(-1, 0));
-        s.hx_one[so].assign(s.nlev, 1);
-        for (int b = 0; b < s.nblk; ++b)
-            for (int r = 0; r < 27; ++r) {
-                const int side[3] = {r % 3 - 1, (r / 3) % 3 - 1, r / 9 - 1};
-                if (!hx_resolve(s, b, side, so, &ent[(size_t)27 * b + r])) s.hx_one[so][s.level[b]] = 0;
-            }
-        SG_HIP(hipMalloc((void **)&s.d_hxe[so], ent.size() * sizeof(int2)));
-        SG_HIP(hipMemcpy(s.d_hxe[so], ent.data(), ent.size() * sizeof(int2), hipMemcpyHostToDevice));
-    }
+    if (s.hx_ready) return SG_OK;
     const int nl = s.nlev;
-    std::vector<int4> hx, fg, rf;
+    const size_t ne = (size_t)2 * 27 * s.nblk;
+    if (!s.d_hxe) SG_HIP(hipMalloc((void **)&s.d_hxe, ne * sizeof(int2) + 2 * nl * sizeof(int)));
+    int *staged = (int *)(s.d_hxe + ne);
+    SG_HIP(hipMemsetAsync(staged, 0, 2 * nl * sizeof(int), s.stream));
+    SG_TRY(go(s, k_hx_table, (long)ne, s.d_hxe, staged, s.nblk, nl,
+              HxBlocks{s.d_level, s.d_nbr, s.d_parent, s.d_octant}));
+    s.hx_staged.assign(2 * nl, 0);
+    SG_HIP(hipMemcpyAsync(s.hx_staged.data(), staged, 2 * nl * sizeof(int), hipMemcpyDeviceToHost, s.stream));
+    SG_HIP(hipStreamSynchronize(s.stream));
+    std::vector<int4> hx;
     s.hx_off.assign(3 * nl + 1, 0);
     for (int l = 0; l < nl; ++l)
         for (int d = 0; d < 3; ++d) {
             s.hx_off[3 * l + d] = (int)hx.size();
+            if (!s.hx_staged[l] && !s.hx_staged[nl + l]) continue;
             for (int b = s.lev_start[l]; b < s.lev_start[l + 1]; ++b)
                 for (int lr = 0; lr < 2; ++lr) {
                     const int f = 2 * d + lr, m = s.nbr[6 * b + f];
@@ -2924,6 +2884,16 @@ int build_hydro_tables(sg_amr &s)
                 }
         }
     s.hx_off[3 * nl] = (int)hx.size();
+    if (!hx.empty()) SG_TRY(upload4(s, &s.d_hx, hx));
+    s.hx_ready = 1;
+    return SG_OK;
+}
+
+int build_restriction_tables(sg_amr &s)
+{
+    if (s.fg_ready) return SG_OK;
+    const int nl = s.nlev;
+    std::vector<int4> fg;
     s.fg_off.assign(nl + 1, 0);
     for (int l = 0; l < nl; ++l) {
         s.fg_off[l] = (int)fg.size();
@@ -2931,6 +2901,16 @@ int build_hydro_tables(sg_amr &s)
             for (int b = s.lev_start[l]; b < s.lev_start[l + 1]; ++b) fg.push_back(make_int4(b, s.parent[b], s.octant[b], 0));
     }
     s.fg_off[nl] = (int)fg.size();
+    SG_TRY(upload4(s, &s.d_fg, fg));
+    s.fg_ready = 1;
+    return SG_OK;
+}
+
+int build_reflux_tables(sg_amr &s)
+{
+    if (s.rf_ready) return SG_OK;
+    const int nl = s.nlev;
+    std::vector<int4> rf;
     // refluxing: items in the reference's order, each in the round after the last one that
     // corrected any of its coarse cells
     s.rf_rounds.assign(nl, {});
@@ -2975,10 +2955,8 @@ int build_hydro_tables(sg_amr &s)
         }
         off.push_back((int)rf.size());
     }
-    SG_TRY(upload4(s, &s.d_hx, hx));
-    SG_TRY(upload4(s, &s.d_fg, fg));
     SG_TRY(upload4(s, &s.d_rf, rf));
-    s.hydro_ready = 1;
+    s.rf_ready = 1;
     return SG_OK;
 }
 
@@ -3099,7 +3077,7 @@ int sg_amr_hydro_boundary_dev(sg_amr *ctx, double *pool, int level, int mode)
                s.bml.ng);
     SG_REQUIRE(level == 0 || (s.d_slot_u1 && s.d_slot_u2),
                "sg_amr_hydro_boundary_dev: the parent level's pass needs the predictor and past slots");
-    SG_TRY(build_hydro_tables(s));
+    SG_TRY(build_exchange_tables(s));
     const long W = 8 + 2 * s.bml.ng, slab = (long)s.bml.ng * W * W * s.bml.ncomp;
     SG_REQUIRE(3 * slab <= 65535L * 256, "sg_amr_hydro_boundary_dev: ncomp too large for the launch shape");
     auto pass = [&](int l, int d, int ntab, int same_only) -> int {
@@ -3115,14 +3093,14 @@ int sg_amr_hydro_boundary_dev(sg_amr *ctx, double *pool, int level, int mode)
     // one launch per level where every ghost region's source is known beforehand, else the three
     // staged passes (an inner corner of the refined region in the same-level part)
     auto exchange = [&](int l, int ntab, int same_only) -> int {
-        const long wide = (long)(s.lev_start[l + 1] - s.lev_start[l]) * ntab;
-        if (!s.hx_one[same_only][l] || wide > 0x7fffffffL) {
+        if (s.hx_staged[same_only * s.nlev + l]) {
             for (int d = 0; d < 3; ++d) SG_TRY(pass(l, d, ntab, same_only));
             return SG_OK;
         }
         const int b0 = s.lev_start[l], nb = s.lev_start[l + 1] - b0;
-        const unsigned groups = (unsigned)wide;
-        const int2 *ent = s.d_hxe[same_only] + (size_t)27 * b0;
+        SG_REQUIRE((long)nb * ntab <= 0x7fffffffL, "sg_amr_hydro_boundary_dev: level %d too large for one launch", l);
+        const unsigned groups = (unsigned)(nb * ntab);
+        const int2 *ent = s.d_hxe + (size_t)27 * ((size_t)same_only * s.nblk + b0);
         const int *su = s.d_slot_u, *s1 = s.d_slot_u1, *s2 = s.d_slot_u2;
         if (s.bml.ng == 2)
             hipLaunchKernelGGL(k_hx_fill<2>, dim3(groups), dim3(256), 0, s.stream, pool, ent, b0, nb, su,
@@ -3148,7 +3126,7 @@ int sg_amr_fg2cg_dev(sg_amr *ctx, double *pool, int level, double gamma)
     SG_REQUIRE(level >= 0 && level < s.nlev, "sg_amr_fg2cg_dev: level %d outside 0..%d", level, s.nlev - 1);
     SG_REQUIRE(std::isfinite(gamma) && gamma != 1.0, "sg_amr_fg2cg_dev: bad gamma");
     if (level < 1) return SG_OK;   // fg2cg.F90:25
-    SG_TRY(build_hydro_tables(s));
+    SG_TRY(build_restriction_tables(s));
     const int a = s.fg_off[level], n = s.fg_off[level + 1] - a;
     SG_TRY(go(s, k_fg2cg, (long)n * 64, pool, (const int4 *)(s.d_fg + a), n, (const int *)s.d_slot_u, s.bml, gamma));
     SG_HIP(hipStreamSynchronize(s.stream));
@@ -3163,7 +3141,7 @@ int sg_amr_fluxcorrection_dev(sg_amr *ctx, double *pool, const double *fb, int l
     SG_REQUIRE(is_hd9(s.bml), "sg_amr_fluxcorrection_dev: the ideal-gas refluxing takes the nine-component layout");
     SG_REQUIRE(std::isfinite(gamma) && gamma != 1.0, "sg_amr_fluxcorrection_dev: bad gamma");
     if (level < 0 || level >= s.nlev - 1) return SG_OK;   // reflux.F90:118-119
-    SG_TRY(build_hydro_tables(s));
+    SG_TRY(build_reflux_tables(s));
     const double hf = s.hl[0][level + 1], hc = s.hl[0][level];
     const double dsf = hf * hf, dsc = hc * hc, dv = hc * hc * hc;   // get_ds, get_dv (grid.F90:405-421)
     const std::vector<int> &off = s.rf_rounds[level];
