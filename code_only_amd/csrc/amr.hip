@@ -3098,16 +3098,20 @@ int sg_amr_hydro_boundary_dev(sg_amr *ctx, double *pool, int level, int mode)
             return SG_OK;
         }
         const int b0 = s.lev_start[l], nb = s.lev_start[l + 1] - b0;
-        SG_REQUIRE((long)nb * ntab <= 0x7fffffffL, "sg_amr_hydro_boundary_dev: level %d too large for one launch", l);
-        const unsigned groups = (unsigned)(nb * ntab);
+        if (nb == 0) return SG_OK;
+        // all components in one workgroup where the grids alone fill the chip, else shared out
+        const int M = s.bml.ncomp, want = (int)std::min<long>(M, (kHxGroups + (long)nb * ntab - 1) / ((long)nb * ntab));
+        const int per = (M + want - 1) / want, parts = (M + per - 1) / per;
+        SG_REQUIRE((long)nb * ntab * parts <= 0x7fffffffL, "sg_amr_hydro_boundary_dev: level %d too large for one launch", l);
+        const dim3 grid((unsigned)(nb * ntab * parts));
         const int2 *ent = s.d_hxe + (size_t)27 * ((size_t)same_only * s.nblk + b0);
         const int *su = s.d_slot_u, *s1 = s.d_slot_u1, *s2 = s.d_slot_u2;
         if (s.bml.ng == 2)
-            hipLaunchKernelGGL(k_hx_fill<2>, dim3(groups), dim3(256), 0, s.stream, pool, ent, b0, nb, su,
-                               s1, s2, mode, s.bml);
+            hipLaunchKernelGGL(k_hx_fill<2>, grid, dim3(256), 0, s.stream, (const double *)pool, pool, ent, b0, nb, su, s1,
+                               s2, mode, s.bml, per, parts);
         else
-            hipLaunchKernelGGL(k_hx_fill<0>, dim3(groups), dim3(256), 0, s.stream, pool, ent, b0, nb, su,
-                               s1, s2, mode, s.bml);
+            hipLaunchKernelGGL(k_hx_fill<0>, grid, dim3(256), 0, s.stream, (const double *)pool, pool, ent, b0, nb, su, s1,
+                               s2, mode, s.bml, per, parts);
         SG_CHECK_LAUNCH();
         return SG_OK;
     };

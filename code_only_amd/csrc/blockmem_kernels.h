@@ -307,99 +307,107 @@ __global__ void k_hx_table(int2 *ent, int *staged, int nblk, int nlev, HxBlocks 
 // reads a ghost cell soon, and the neighbours' lines stay in L2 (4 % on the whole step).  Measured
 // slower: one or three components per workgroup (10 %), cells taken row by row with the interior's
 // lanes idle (7 %).
+// Levels of fewer grids are bound by the latency of a workgroup's loop over the components, so they are
+// shared out over workgroups until kHxGroups of them, the eight of 256 threads that each CU holds, and
+// the interpolated cells, which sit in a few regions, are dealt to all threads.  Without either the
+// exchange of a random hierarchy's finest level fell behind the passes (288 blocks of three levels 0.082 ms
+// with the passes, 0.101 without, 0.076 here; 2 008 blocks 0.479, 0.497, 0.466; nested, 192 blocks: 0.066,
+// 0.072, 0.037).  With 512 or 1 024 workgroups 1 024 nested blocks take 8 or 6 % longer.
 constexpr int kHxCells = 5;   // 5 x 256 >= 12^3 - 8^3
+constexpr long kHxGroups = 2048;
 
+// in and out: the pool.  No cell that is read here is written here.  Workgroup (array, grid, part) forms
+// components part * per .. of every ghost cell of the grid.
 template <int NG>   // ghost layers, 0: L.ng
-__global__ void __launch_bounds__(256) k_hx_fill(double *pool, const int2 *__restrict__ ent, int b0, int nb,
+__global__ void __launch_bounds__(256) k_hx_fill(const double *__restrict__ in, double *__restrict__ out,
+                                                 const int2 *__restrict__ ent, int b0, int nb,
                                                  const int *__restrict__ su, const int *__restrict__ s1,
-                                                 const int *__restrict__ s2, int mode, sg_blockmem L)
+                                                 const int *__restrict__ s2, int mode, sg_blockmem L, int per, int parts)
 {
     const int ng = NG ? NG : L.ng, W = 8 + 2 * ng, W3 = W * W * W;
     const int nz = 2 * ng * W * W, ny = 8 * 2 * ng * W, nghost = W3 - 512;
     const int w = xcd_block((int)blockIdx.x, (int)gridDim.x);
-    const int tab = w / nb, b = b0 + w % nb;
+    const int part = w % parts, tab = w / parts / nb, b = b0 + w / parts % nb;
+    const int m0 = part * per, m1 = min(L.ncomp, m0 + per);
     const int *slots = tab == 0 ? su : (tab == 1 ? s1 : s2);
     const int *cs = mode == 1 ? s2 : (mode == 2 ? s1 : su);
     __shared__ int2 se[27];
     __shared__ long sbase[27];
+    __shared__ int s_list[kHxCells * 256];   // ghost cells to interpolate: region << 16 | cell
+    __shared__ int s_count;
     if (threadIdx.x < 27) {
         const int2 e = ent[27 * (b - b0) + threadIdx.x];
         se[threadIdx.x] = e;
         sbase[threadIdx.x] = e.x < 0 ? 0 : (long)((e.y & 8) ? cs[e.x] : slots[e.x]) * L.stride;
     }
-    __syncthreads();
     const long own = (long)slots[b] * L.stride;
     // ghost layer a of 2 ng along one axis -> its coordinate
     auto layer = [&](int a) { return a < ng ? a - ng : a - ng + 8; };
-    auto cell = [&](int g, int &i, int &j, int &k) {
-        if (g < nz) {                       // z slabs, the whole extent of x and y
-            i = g % W - ng;
-            j = (g / W) % W - ng;
-            k = layer(g / (W * W));
-        } else if (g < nz + ny) {           // y slabs of the interior planes
-            const int h = g - nz;
-            i = h % W - ng;
-            j = layer((h / W) % (2 * ng));
-            k = h / (W * 2 * ng);
-        } else {                            // x ends of the interior rows
-            const int h = g - nz - ny;
-            i = layer(h % (2 * ng));
-            j = (h / (2 * ng)) & 7;
-            k = h / (16 * ng);
-        }
-    };
-    for (int g0 = threadIdx.x; g0 < nghost; g0 += 256 * kHxCells) {
+    auto side = [](int i) { return i < 0 ? 0 : (i < 8 ? 1 : 2); };
+    for (int g0 = 0; g0 < nghost; g0 += 256 * kHxCells) {
+        if (threadIdx.x == 0) s_count = 0;
+        __syncthreads();
         long so[kHxCells];
         int dst[kHxCells];
-        unsigned copy = 0u, interp = 0u;
+        unsigned copy = 0u;
 #pragma unroll
         for (int q = 0; q < kHxCells; ++q) {
-            const int g = g0 + 256 * q;
-            so[q] = own;
+            const int g = g0 + (int)threadIdx.x + 256 * q;
+            so[q] = own + ((long)ng * W + ng) * W + ng;
             dst[q] = 0;
             if (g >= nghost) continue;
             int i, j, k;
-            cell(g, i, j, k);
-            const int rx = i < 0 ? 0 : (i < 8 ? 1 : 2), ry = j < 0 ? 0 : (j < 8 ? 1 : 2), rz = k < 0 ? 0 : (k < 8 ? 1 : 2);
-            const int r = rx + 3 * ry + 9 * rz, c = ((k + ng) * W + j + ng) * W + i + ng;
+            if (g < nz) {                       // z slabs, the whole extent of x and y
+                i = g % W - ng;
+                j = (g / W) % W - ng;
+                k = layer(g / (W * W));
+            } else if (g < nz + ny) {           // y slabs of the interior planes
+                const int h = g - nz;
+                i = h % W - ng;
+                j = layer((h / W) % (2 * ng));
+                k = h / (W * 2 * ng);
+            } else {                            // x ends of the interior rows
+                const int h = g - nz - ny;
+                i = layer(h % (2 * ng));
+                j = (h / (2 * ng)) & 7;
+                k = h / (16 * ng);
+            }
+            const int rx = side(i), ry = side(j), rz = side(k), r = rx + 3 * ry + 9 * rz;
+            const int c = ((k + ng) * W + j + ng) * W + i + ng;
             const int2 e = se[r];
             dst[q] = c;
             if (e.x < 0) continue;
             if (e.y & 8) {
-                interp |= 1u << q;
+                s_list[atomicAdd(&s_count, 1)] = r << 16 | c;
             } else {
                 copy |= 1u << q;
                 so[q] = sbase[r] + c + ((e.y & 1) ? 8 * (1 - rx) : 0) + ((e.y & 2) ? 8 * W * (1 - ry) : 0) +
                         ((e.y & 4) ? 8 * W * W * (1 - rz) : 0);
             }
         }
-        const int M = L.ncomp;
-        // cells without a copy read the array's first cell and store nothing
-        for (int m = 0; m < M; ++m) {
+        // cells without a copy read an interior cell of their grid and store nothing
+        for (int m = m0; m < m1; ++m) {
             double v[kHxCells];
 #pragma unroll
-            for (int q = 0; q < kHxCells; ++q) v[q] = pool[so[q] + (long)m * W3];
+            for (int q = 0; q < kHxCells; ++q) v[q] = in[so[q] + (long)m * W3];
 #pragma unroll
             for (int q = 0; q < kHxCells; ++q)
-                if ((copy >> q) & 1u) __builtin_nontemporal_store(v[q], pool + own + (long)m * W3 + dst[q]);
+                if ((copy >> q) & 1u) __builtin_nontemporal_store(v[q], out + own + (long)m * W3 + dst[q]);
         }
-        if (interp) {
-#pragma unroll
-            for (int q = 0; q < kHxCells; ++q) {
-                if (!((interp >> q) & 1u)) continue;
-                int i, j, k;
-                cell(g0 + 256 * q, i, j, k);
-                const int rx = i < 0 ? 0 : (i < 8 ? 1 : 2), ry = j < 0 ? 0 : (j < 8 ? 1 : 2), rz = k < 0 ? 0 : (k < 8 ? 1 : 2);
-                const int r = rx + 3 * ry + 9 * rz, fl = se[r].y;
-                const int p[3] = {i + ((fl & 1) ? 8 * (1 - rx) : 0), j + ((fl & 2) ? 8 * (1 - ry) : 0),
-                                  k + ((fl & 4) ? 8 * (1 - rz) : 0)};
-                const double *bu = pool + sbase[r] + hx_coarse(L, p, (fl >> 4) & 3, (fl >> 6) & 1, (fl >> 7) & 7);
-                for (int m = 0; m < M; ++m, bu += W3) {
-                    const double g[6] = {bu[-1], bu[1], bu[-W], bu[W], bu[-W * W], bu[W * W]};
-                    pool[own + (long)m * W3 + dst[q]] = hx_value(bu[0], g, p);
-                }
-            }
+        __syncthreads();
+        // the listed cells, dealt to all threads: few regions of a grid interpolate, and a thread's own
+        // cells would be interpolated one after the other
+        const int n = s_count;
+        for (int t = threadIdx.x; t < n * (m1 - m0); t += 256) {
+            const int m = m0 + t / n, x = s_list[t % n], r = x >> 16, c = x & 0xffff, fl = se[r].y;
+            const int p[3] = {c % W - ng + ((fl & 1) ? 8 * (1 - r % 3) : 0),
+                              c / W % W - ng + ((fl & 2) ? 8 * (1 - r / 3 % 3) : 0),
+                              c / (W * W) - ng + ((fl & 4) ? 8 * (1 - r / 9) : 0)};
+            const double *bu = in + sbase[r] + (long)m * W3 + hx_coarse(L, p, (fl >> 4) & 3, (fl >> 6) & 1, (fl >> 7) & 7);
+            const double g[6] = {bu[-1], bu[1], bu[-W], bu[W], bu[-W * W], bu[W * W]};
+            out[own + (long)m * W3 + c] = hx_value(bu[0], g, p);
         }
+        if (g0 + 256 * kHxCells < nghost) __syncthreads();   // the list has been read
     }
 }
 

@@ -156,6 +156,26 @@ def test_hydro_argument_checks(gpu):
         s.close()
 
 
+def test_hydro_boundary_component_parts(gpu):
+    """Levels of some hundred grids, whose components are shared out over two or three workgroups a grid
+    (of nine components, a last part of fewer): bit for bit the oracle's staged passes."""
+    import torch
+    h = ah.nested(base=8, levels=2, bc=ah.SPHERE)
+    lay = LAY["hd"]
+    pool, su, s1, s2 = problems.blockmem_pool(h, lay, seed=66)
+    s = AmrSolver(h)
+    try:
+        s.set_blockmem(lay, pool.shape[0], su, s1, s2)
+        exp = pool.copy()
+        oracle.bm_grid_boundary(exp, oracle.blockmem(**lay), h, su, s1, s2, 1, 1)
+        dp = torch.from_numpy(pool).to(gpu)
+        s.hydro_boundary(dp, 1, 1)
+        got = dp.cpu().numpy()
+        assert np.array_equal(got, exp), _diff(got, exp)
+    finally:
+        s.close()
+
+
 def test_first_exchange_builds_its_tables_quickly(gpu):
     """The first exchange on a hierarchy, which builds its tables, takes less than two later ones (the
     best of three fresh contexts; 8 192 blocks): a program that regrids every step pays it every step."""
