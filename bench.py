@@ -363,7 +363,7 @@ def bench_uniform(a, dev):
     tiles = {}
     dims = [(32, 16, 16, 1024), (16, 8, 8, 1024), (16, 8, 8, 256), (64, 8, 8, 512), (8, 8, 8, 512)]
     # streaming shapes, two sweeps per launch: (SX, SY, ZC)
-    sdims = [(64, 16, 32), (64, 16, 16), (64, 16, 64), (32, 16, 32), (32, 32, 64), (32, 16, 16), (32, 8, 16),
+    sdims = [(64, 16, 32), (64, 16, 32), (64, 16, 64), (32, 16, 16), (32, 32, 64), (32, 16, 16), (32, 16, 16),
              (32, 32, 32), (16, 16, 16), (64, 16, 128), (32, 16, 64), (16, 8, 8)]
     names = ["x".join(map(str, d[:3])) + f"/{d[3]}" for d in dims] + \
             ["stream " + "x".join(map(str, d[:2])) + f" z{d[2]}" for d in sdims]

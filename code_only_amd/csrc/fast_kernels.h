@@ -319,17 +319,14 @@ k_sweep_tile(const T *__restrict__ uin, T *__restrict__ uout, const T *__restric
 // (one where a single sweep is left): column SX x SY, chunk of ZC planes.  A longer chunk spends less on
 // its halo planes, a shorter one makes more workgroups: 512^3 is fastest with 128 planes, 256^3 with 64.
 // A shape's number is public (sg_uniform_set_tile) and fixes the widths it takes, the multiples of its
-// largest extent: shapes are appended, never renumbered.  Numbers 2 and 4 (Stream2, Stream4) once named
-// columns of 64 x 32 and 128 x 16, whose pairs exceed a workgroup, and take their widths (4 also 64).  Numbers 1, 3
-// and 6 are there for callers that hold them; the autotuners do not time them (their longer or wider
-// neighbours spend less on halos at the same widths).
+// largest extent: shapes are appended, never renumbered.  Numbers 1, 3 and 6 named shapes that are no longer
+// built and run the shape of the same column family that takes the same widths (Stream0, Stream5, Stream5);
+// 2 and 4 named columns of 64 x 32 and 128 x 16, whose pairs exceed a workgroup, and take their widths
+// (4 also 64).
 using Stream0 = StreamShape<64, 16, 32>;
-using Stream1 = StreamShape<64, 16, 16>;
 using Stream2 = StreamShape<64, 16, 64>;
-using Stream3 = StreamShape<32, 16, 32>;
 using Stream4 = StreamShape<32, 32, 64>;
 using Stream5 = StreamShape<32, 16, 16>;
-using Stream6 = StreamShape<32, 8, 16>;
 using Stream7 = StreamShape<32, 32, 32>;
 using Stream8 = StreamShape<16, 16, 16>;
 using Stream9 = StreamShape<64, 16, 128>;
@@ -337,15 +334,15 @@ using Stream10 = StreamShape<32, 16, 64>;
 using Stream11 = StreamShape<16, 8, 8>;
 constexpr int kNumStream = 12;
 static const int kStreamDims[kNumStream][3] = {
-    {64, 16, 32}, {64, 16, 16}, {64, 16, 64}, {32, 16, 32}, {32, 32, 64},  {32, 16, 16},
-    {32, 8, 16},  {32, 32, 32}, {16, 16, 16}, {64, 16, 128}, {32, 16, 64}, {16, 8, 8}};
+    {64, 16, 32}, {64, 16, 32}, {64, 16, 64}, {32, 16, 16},  {32, 32, 64}, {32, 16, 16},
+    {32, 16, 16}, {32, 32, 32}, {16, 16, 16}, {64, 16, 128}, {32, 16, 64}, {16, 8, 8}};
 
 // sweep configurations: 0 .. kNumTiles-1 tiles, kNumTiles .. kNumTiles+kNumStream-1 streams
 constexpr int kNumCfg = kNumTiles + kNumStream;
 constexpr int kNumCand = kNumTiles * kMaxSweepsPerLaunch * 2 + kNumStream;
 static_assert(kNumCand <= 32, "autotuner timing tables hold 32 candidates");
 
-// whether the autotuners time configuration cfg
+// whether the autotuners time configuration cfg (not the second numbers of a shape)
 inline bool cfg_timed(int cfg) { return cfg != kNumTiles + 1 && cfg != kNumTiles + 3 && cfg != kNumTiles + 6; }
 
 inline bool cfg_fits(int cfg, int n)
@@ -365,7 +362,7 @@ template <class TL, int NS, bool FS, typename T> constexpr bool sweep_built()
 }
 template <class SS, typename T> constexpr bool stream_built()
 {
-    return sizeof(T) == sizeof(float) || (SS::SX == 32 && SS::SY == 16 && SS::ZC != 32);
+    return sizeof(T) == sizeof(float) || (SS::SX == 32 && SS::SY == 16);
 }
 template <class SS, typename T> constexpr bool stream_built_fits()
 {
@@ -421,13 +418,13 @@ template <typename T> inline bool cfg_ok(int cfg, int ns, bool fs)
     if (cfg < kNumTiles) return cand_ok<T>(cfg, ns, fs);
     if (ns < 1 || ns > kMaxSweepsPerLaunch || fs) return false;
     switch (cfg - kNumTiles) {
-    case 0: return stream_built<Stream0, T>();
-    case 1: return stream_built<Stream1, T>();
+    case 0:
+    case 1: return stream_built<Stream0, T>();
     case 2: return stream_built<Stream2, T>();
-    case 3: return stream_built<Stream3, T>();
     case 4: return stream_built<Stream4, T>();
-    case 5: return stream_built<Stream5, T>();
-    case 6: return stream_built<Stream6, T>();
+    case 3:
+    case 5:
+    case 6: return stream_built<Stream5, T>();
     case 7: return stream_built<Stream7, T>();
     case 8: return stream_built<Stream8, T>();
     case 9: return stream_built<Stream9, T>();

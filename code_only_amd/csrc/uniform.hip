@@ -349,13 +349,13 @@ static int launch_sweep_cfg(hipStream_t s, int cfg, int ns, bool fs, const T *ui
     SG_REQUIRE(cfg_ok<T>(cfg, ns, fs), "sweep shape %d with %d sweeps (staged %d) does not exist", cfg, ns, (int)fs);
     const T h2 = (T)(h * h), h2i = (T)(1.0 / (h * h));
     switch (cfg) {
-    case kNumTiles + 0: stream_variant<Stream0, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 1: stream_variant<Stream1, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 0:
+    case kNumTiles + 1: stream_variant<Stream0, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case kNumTiles + 2: stream_variant<Stream2, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 3: stream_variant<Stream3, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case kNumTiles + 4: stream_variant<Stream4, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 5: stream_variant<Stream5, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
-    case kNumTiles + 6: stream_variant<Stream6, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
+    case kNumTiles + 3:
+    case kNumTiles + 5:
+    case kNumTiles + 6: stream_variant<Stream5, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case kNumTiles + 7: stream_variant<Stream7, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case kNumTiles + 8: stream_variant<Stream8, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;
     case kNumTiles + 9: stream_variant<Stream9, T>(s, ns, uin, uout, f, n, h2, h2i, zero, prolong, resid, uc, rc, resmax); break;

@@ -140,9 +140,9 @@ int sg_uniform_time_smoother(sg_uniform *ctx, int prec, int reps, double *ms_per
  * cycle (two sweeps ending with the residual restriction, two starting with the prolongated
  * correction) of every candidate (-1 where it does not fit or is not timed): 32 candidates, the LDS
  * tiles first, indexed tile * 4 + (sweeps - 1) * 2 + staged (cfg 0..4), then the twelve streaming
- * shapes at 20 + cfg - 5, timed with two sweeps per launch: column and planes, cfg 5 64x16x32, 6
- * 64x16x16 (not timed), 7 64x16x64, 8 32x16x32 (not timed), 9 32x32x64, 10 32x16x16, 11 32x8x16 (not
- * timed), 12 32x32x32, 13 16x16x16, 14 64x16x128, 15 32x16x64, 16 16x8x8. */
+ * shapes at 20 + cfg - 5, timed with two sweeps per launch: column and planes, cfg 5 and 6 64x16x32, 7
+ * 64x16x64, 9 32x32x64, 8, 10 and 11 32x16x16, 12 32x32x32, 13 16x16x16, 14 64x16x128, 15 32x16x64, 16
+ * 16x8x8 (6, 8 and 11, second numbers of a shape, are not timed). */
 int sg_uniform_tile_info(sg_uniform *ctx, int level, int *cfg, int *ns, int *fs, float *ms, int nms);
 /* Override the autotuner's choice for fused-sweep level `level` (same meaning of cfg / ns / fs; values
  * do not depend on the choice).  A cfg fits the levels whose width is a multiple of its largest extent;
