@@ -81,6 +81,7 @@ struct sg_batch {
     bool recording = false;
     size_t cursor = 0;
     int ecode = CU;  // code of the buffer holding level 0's correction
+    bool exact = false;  // the cycle at hand ends at each problem's lb
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
 };
@@ -136,8 +137,8 @@ int take(sg_batch *c, const Pairs &pl, FB blocks, const Item **d, int *cnt, int 
 }
 
 template <typename T> BL<T> bl(sg_batch *c, const Item *d, int cnt);
-template <> BL<double> bl<double>(sg_batch *c, const Item *d, int cnt) { return {d, cnt, c->d_pl64, c->d_active}; }
-template <> BL<float> bl<float>(sg_batch *c, const Item *d, int cnt) { return {d, cnt, c->d_pl32, c->d_active}; }
+template <> BL<double> bl<double>(sg_batch *c, const Item *d, int cnt) { return {d, cnt, c->d_pl64, c->d_active, c->exact}; }
+template <> BL<float> bl<float>(sg_batch *c, const Item *d, int cnt) { return {d, cnt, c->d_pl32, c->d_active, c->exact}; }
 
 template <typename T> int pl_n(sg_batch *c, int p, int l)
 {
@@ -390,6 +391,7 @@ int op_sweep(sg_batch *c, const Pairs &pl, int v, int ns, int cin, int cout, int
 // levels ends at its level lb, solved exactly (FP32; as the single-grid solver's SG_COARSE_EXACT).
 template <typename T> int fast_mg_lin(sg_batch *c, int ncycle, int npre, int npost, bool exact)
 {
+    c->exact = exact;
     const std::vector<int> &bot = exact ? c->lb : c->lc;  // level of each problem's coarse-grid solve
     const int maxlc = exact ? c->maxlb : c->maxlc;
     auto fine_at = [&](int l, int minlc) {  // problems with bottom level > minlc, at level l
@@ -839,6 +841,7 @@ int create(sg_batch **out, int np, const int *ns, const double *hs, int precisio
             PL<float> &b = c->h_pl32[q * kBLev + l];
             a.n = b.n = m;
             a.lc = b.lc = lc;
+            a.lb = b.lb = lbq;
             a.dn = b.dn = make_div((unsigned)m);
             a.h2 = hl * hl;
             a.h2i = 1.0 / (hl * hl);

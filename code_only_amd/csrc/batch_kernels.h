@@ -48,6 +48,7 @@ template <typename T> struct PL {
     T *a[kCodes];
     int n;        // cells per side
     int lc;       // first level held by the coarse kernel (problem-wide)
+    int lb;       // level of the exact-coarse cycle's bottom (problem-wide)
     FastDiv dn;   // division by n
     T h2, h2i;
 };
@@ -61,6 +62,7 @@ template <typename T> struct BL {
     int nitems;
     const PL<T> *pl;
     const int *active;
+    bool exact;   // the cycle ends at lb, not lc
 };
 
 __device__ __forceinline__ int find_item(const Item *it, int n, int b)
@@ -283,12 +285,12 @@ __global__ void __launch_bounds__(1024) kb_norm_final(const Item *items, const i
 
 // ---- fused inner solve (FP32: mixed, FP64: plain) -----------------------------------------------------------------
 
-// The coarse array of level l + 1 that a level-l kernel reads: the coarse kernel's U when l + 1 is
-// the problem's first coarse level, else the fused sweeps' current buffer `cur`.
-template <typename T> __device__ __forceinline__ const T *coarse_src(const PL<T> &q, int l, int cur)
+// The coarse array of level l + 1 that a level-l kernel reads: U where l + 1 is the level of the problem's
+// coarse-grid solve, else the fused sweeps' current buffer `cur` (that of the problems whose bottom lies below).
+template <typename T> __device__ __forceinline__ const T *coarse_src(const BL<T> &L, const PL<T> &q, int l, int cur)
 {
     const PL<T> &qc = *(&q + 1);
-    return qc.a[(l + 1 == q.lc) ? CU : cur];
+    return qc.a[(l + 1 == (L.exact ? q.lb : q.lc)) ? CU : cur];
 }
 
 // ns fused sweeps of level l of every item (the fused sweep body of the single-grid solver).
@@ -300,7 +302,7 @@ __global__ void __launch_bounds__(TL::NT) kb_sweep(BL<T> L, int total, int cin, 
     const PL<T> &q = *c.q;
     const int l = c.it->l;
     sweep_tile<TL, NS, ZERO, PROLONG, RESID, FS, T>(q.a[cin], q.a[cout], q.a[CRHS], q.n, q.h2, q.h2i,
-                                                 PROLONG ? coarse_src(q, l, cuc) : nullptr,
+                                                 PROLONG ? coarse_src(L, q, l, cuc) : nullptr,
                                                  RESID ? (&q + 1)->a[CRHS] : nullptr, nullptr, c.lb);
 }
 
@@ -314,7 +316,7 @@ kb_stream(BL<T> L, int total, int cin, int cout, int cuc)
     const PL<T> &q = *c.q;
     const int l = c.it->l;
     sweep_stream<SS, NS, ZERO, PROLONG, RESID, T>(q.a[cin], q.a[cout], q.a[CRHS], q.n, q.h2, q.h2i,
-                                           PROLONG ? coarse_src(q, l, cuc) : nullptr,
+                                           PROLONG ? coarse_src(L, q, l, cuc) : nullptr,
                                            RESID ? (&q + 1)->a[CRHS] : nullptr, nullptr, c.lb);
 }
 
@@ -326,7 +328,7 @@ __global__ void __launch_bounds__(NT) kb_interp_cubic_tile(BL<T> L, int total, i
     Cell<T> c;
     if (!locate(L, xcd_block(total), c)) return;
     const PL<T> &q = *c.q;
-    interp_cubic_tile<FX, FY, FZ, NT, T>(q.a[CU], coarse_src(q, c.it->l, cuc), q.n, c.lb);
+    interp_cubic_tile<FX, FY, FZ, NT, T>(q.a[CU], coarse_src(L, q, c.it->l, cuc), q.n, c.lb);
 }
 
 // Levels of <= 16^3 cells of one problem, resident in one workgroup's LDS (coarse_levels.h).

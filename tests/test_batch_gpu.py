@@ -195,3 +195,25 @@ def test_exact_planes_reduce_every_mode(gpu, n):
         rel_linf[coarse] = st["rel_linf"]
     print(n, rel_linf, flush=True)
     assert rel_linf[SG_COARSE_EXACT] < 1.5 * rel_linf[SG_COARSE_VCYCLE] < 0.1
+
+
+@pytest.mark.parametrize("npre,npost,ncycle", [(3, 2, 1), (3, 2, 2), (2, 3, 1)])
+def test_mixed_batch_of_two_bottoms_odd_launches(gpu, npre, npost, ncycle):
+    """Problems whose exactly solved bottom lies on different levels (256^3: level 2, 128^3: level 1), with
+    five sweeps per visit -- an odd count of launches whether one or two sweeps go into each, so that
+    level 1 of the larger problem ends in its other buffer: each equals the single-grid solve, bit for bit."""
+    sizes = [256, 128]
+    srcs = rhs_list(sizes, seed=23)
+    kw = dict(tol=1e-10, maxit=3, precision=SG_PREC_MIXED, npre=npre, npost=npost, ncycle=ncycle, raise_on_fail=False)
+    b = BatchSolver(sizes, precisions=SG_PREC_MIXED)
+    psis, st = b.solve_host(srcs, **kw)
+    b.close()
+    for q, n in enumerate(sizes):
+        one = UniformSolver(n, precisions=SG_PREC_MIXED)
+        f = torch.tensor(srcs[q], device=gpu)
+        psi = torch.zeros_like(f)
+        s1 = one.cycle(psi, f, **kw)
+        one.close()
+        print(n, st[q]["hist"][:4], s1["hist"][:4], flush=True)
+        assert st[q]["rel_linf"] == s1["rel_linf"]
+        assert np.array_equal(psis[q], psi.cpu().numpy()), f"n = {n}"
