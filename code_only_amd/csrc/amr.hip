@@ -70,7 +70,7 @@ struct sg_amr {
     int *d_cf = nullptr, *d_cf_slot = nullptr, *d_ovslot = nullptr, *d_cov = nullptr;
     // fused refresh (mixed solve): covered blocks' face layers read by same-level leaf neighbours
     // (entries b*6+f), the child table, and per FMG level whether the hierarchy admits the fused
-    // form (build_prep_tables); fused_on is set for the duration of a mixed solve that asks for it
+    // form (build_prep_tables); fused_on is set for the duration of a solve that asks for it
     std::vector<int> covf;
     int *d_child = nullptr;
     // k_prep's source tables per fused FMG level (build_prep_tables): covered face-layer cells
@@ -202,6 +202,14 @@ struct sg_amr {
 };
 
 namespace {
+
+// The fused launch structure for the scope of a solve or operation: off again on every way out, errors
+// included (nothing else turns it on).
+struct FusedScope {
+    sg_amr &s;
+    FusedScope(sg_amr &s_, int on) : s(s_) { s.fused_on = on; }
+    ~FusedScope() { s.fused_on = 0; }
+};
 
 template <typename T> inline Arrays<T> &ar(sg_amr &s);
 template <> inline Arrays<double> &ar<double>(sg_amr &s) { return s.d; }
@@ -1336,7 +1344,7 @@ int solve(sg_amr &s, double *psi, const double *src, double *g, const sg_params 
     if (std::fabs(resh2max) <= 2.2250738585072014e-308) nmax = 0;
     double prev = HUGE_VAL;
     int it = 0, status = SG_ERR_NOT_CONVERGED;
-    s.fused_on = s.fp64_fused;   // reset below, before the epilogue reads the stored ghosts
+    FusedScope fused_scope(s, s.fp64_fused);
     auto measure = [&](int slot) -> int {
         SG_TRY(norms(s, C_RHO));
         SG_TRY(read_scalars(s));
@@ -1373,7 +1381,7 @@ int solve(sg_amr &s, double *psi, const double *src, double *g, const sg_params 
     }
     st.iterations = it;
     st.status = status;
-    s.fused_on = 0;
+    s.fused_on = 0;   // the epilogue reads the stored ghosts
     SG_TRY(fmg_copy<double>(s, 0, C_U, C_PSI, 1));
     SG_TRY(c2p<double>(s, 0, C_U, 0));
     SG_TRY(go(s, k_blocks_to_dense, (long)s.nblk * 512, psi, (const double *)s.d.A[0][C_U], s.nblk));
@@ -1507,11 +1515,7 @@ int solve_mixed(sg_amr &s, double *psi, const double *src, double *g, const sg_p
     int nmax = src_finite ? p.maxit : 0;
     if (std::fabs(resh2max) <= 2.2250738585072014e-308) nmax = 0;
     // fused refreshes in the outer residual and the inner fmg_lin (same values as the staged ones)
-    struct FusedScope {
-        sg_amr &s;
-        FusedScope(sg_amr &s_, int on) : s(s_) { s.fused_on = on; }
-        ~FusedScope() { s.fused_on = 0; }
-    } fused_scope(s, p.fused ? 1 : 0);
+    FusedScope fused_scope(s, p.fused ? 1 : 0);
     SG_TRY(outer_resid(s));
     SG_TRY(read_scalars(s));
     double prev = HUGE_VAL;
@@ -2165,11 +2169,7 @@ int op(sg_amr &s, int opc, int L, int a, int b, int c, int flag, double *ret)
     SG_REQUIRE(a >= 0 && a < NCODE && b >= 0 && b < NCODE && c >= 0 && c < NCODE, "sg_amr_op: bad array code");
     double r = 0.0;
     // relax / resid with flag & 4: the fused refresh of the mixed solve (where the hierarchy admits it)
-    struct FusedScope {
-        sg_amr &s;
-        FusedScope(sg_amr &s_, int on) : s(s_) { s.fused_on = on; }
-        ~FusedScope() { s.fused_on = 0; }
-    } fused_scope(s, (opc == SG_AMR_OP_RELAX || opc == SG_AMR_OP_RESID || opc == SG_AMR_OP_FMG_LIN) && (flag & 4) ? 1 : 0);
+    FusedScope fused_scope(s, (opc == SG_AMR_OP_RELAX || opc == SG_AMR_OP_RESID || opc == SG_AMR_OP_FMG_LIN) && (flag & 4) ? 1 : 0);
     if (opc == SG_AMR_OP_RELAX || opc == SG_AMR_OP_RESID) flag &= 1;
     switch (opc) {
     case SG_AMR_OP_C2P: SG_TRY(c2p<double>(s, L, a, flag)); break;

@@ -112,3 +112,15 @@ def test_amr_create_rejects_block_positions_outside_the_level_box():
         rc = lib.sg_amr_create(ctypes.byref(ctx), h.nblk, h.nlev, *[ip(a) for a in arrs], h.h0, x0,
                                _lib.SG_BC_SPHERE)
         assert rc == _lib.SG_ERR_ARG and b"out of [0" in lib.sg_last_error(), (b, bad, lib.sg_last_error())
+
+
+def test_fused_mode_is_only_turned_on_by_its_scope_guard():
+    """Every turn-on of the AMR solver's fused launch structure sits in the guard whose destructor turns it
+    off, so that a solve that fails half way does not leave the context in it (a HIP error cannot be
+    forced from outside without harming the device, so the source is what is checked)."""
+    text = open(os.path.join(ROOT, "code_only_amd", "csrc", "amr.hip")).read()
+    guard = re.search(r"struct FusedScope \{.*?\n\};", text, re.S).group(0)
+    assert "~FusedScope() { s.fused_on = 0; }" in guard
+    rest = text.replace(guard, "")
+    assert re.findall(r"fused_on = (?!0;)", rest) == []
+    assert text.count("struct FusedScope") == 1 and len(re.findall(r"FusedScope fused_scope\(", rest)) == 3
