@@ -46,9 +46,8 @@ constexpr int kNormBlocks = 2048;  // grid of the norm-reducing kernels (fixed: 
 
 template <typename T> struct Levels {
     T *U[kMaxLev] = {};
-    T *RES[kMaxLev] = {};
     T *RHO[kMaxLev] = {};  // RHO[l] also serves as RHS[l]: see mg_lin below
-    T *U1[kMaxLev] = {};   // second U buffer: the fused sweeps ping-pong
+    T *U1[kMaxLev] = {};   // second U buffer: the fused sweeps ping-pong; the residual of the unfused cycle
     void *mem = nullptr;   // the allocation that holds them all
 };
 
@@ -220,7 +219,8 @@ template <typename T> static int launch_interp(hipStream_t s, T *uf, const T *uc
 // separate RHS array at each FMG level (mg.F90:176) and later overwrites RHS of coarser levels
 // with restricted residuals (mg.F90:188).  RHO of a level is never read again after that copy
 // within one mg_lin call (the next call restricts RHO afresh from level 0), so RHS and RHO share
-// storage here; every kernel reads the same values as in the reference.
+// storage here; every kernel reads the same values as in the reference.  The residual of a level goes to
+// U1, which only the fused sweeps and the exact solve of level lb (which forms no residual) write.
 // resmax: receives max|resh2| of the last smoothing call (the one mg_cycle's test reads).
 // exact (FP32 only, and only when the first level of <= 16^3 cells lies below level 0): the levels
 // end at level lb (the first level below level 0 with <= 64^3 cells, or with <= 16^3), solved
@@ -252,8 +252,8 @@ template <typename T> static int mg_lin(sg_uniform *c, int ncycle, int npre, int
             for (int v = ml; v <= lmax - 1; ++v) {
                 for (int p = 0; p < npre; ++p)
                     SG_TRY(launch_relax<T>(s, A.U[v], A.RHO[v], c->nl[v], c->hl[v], nullptr));
-                SG_TRY((launch_resid<T, T>(c, A.RES[v], A.U[v], A.RHO[v], c->nl[v], c->hl[v], nullptr)));
-                SG_TRY(launch_restrict<T>(s, A.RHO[v + 1], A.RES[v], c->nl[v + 1]));
+                SG_TRY((launch_resid<T, T>(c, A.U1[v], A.U[v], A.RHO[v], c->nl[v], c->hl[v], nullptr)));
+                SG_TRY(launch_restrict<T>(s, A.RHO[v + 1], A.U1[v], c->nl[v + 1]));
                 SG_TRY(launch_fill<T>(s, A.U[v + 1], n3(c->nl[v + 1])));
             }
             SG_TRY(bottom());
@@ -900,7 +900,7 @@ template <typename T> static int alloc_levels(sg_uniform *c, Levels<T> &A)
     for (int pass = 0; pass < 2; ++pass) {
         size_t at = 0;
         for (int l = 0; l < c->nlev; ++l)
-            for (T **p : {&A.U[l], &A.RES[l], &A.RHO[l], &A.U1[l]}) {
+            for (T **p : {&A.U[l], &A.RHO[l], &A.U1[l]}) {
                 if (pass) *p = reinterpret_cast<T *>(static_cast<char *>(A.mem) + at);
                 at += (sizeof(T) * (size_t)n3(c->nl[l]) + 255) / 256 * 256;
             }

@@ -429,3 +429,17 @@ def test_small_grid_mixed_equals_unfused(n, gpu):
             assert sa["hist"] == sb["hist"] or sa["status"] == 4
     finally:
         s.close()
+
+
+@pytest.mark.parametrize("prec,word", [(SG_PREC_FP64, 8), (SG_PREC_MIXED, 4)])
+def test_context_memory(prec, word, gpu):
+    """A context holds three arrays per level and a second phi: 3 x 8/7 words and 8 bytes per cell."""
+    n = 256
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    s = UniformSolver(n, precisions=prec)
+    used = free0 - torch.cuda.mem_get_info()[0]
+    s.close()
+    print(used / n ** 3, flush=True)
+    # 0.2 bytes per cell of norm partials, and 16 MiB for the allocator's granularity and small tables
+    assert used <= (3 * 8 / 7 * word + 8 + 0.2) * n ** 3 + (16 << 20)
