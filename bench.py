@@ -334,19 +334,23 @@ def bench_uniform(a, dev):
     log(f"[bench] mixed: {msmx:.3f} ms/solve, {stmx['iterations']} it, rel {stmx['rel_linf']:.3e}")
 
     # dominant kernel: the fine-level smoother of the mixed solve, timed with HIP events on the
-    # library's stream.  Algorithmic bytes of one full sweep = read u + read f + write u = 3 * 4 B
-    # per fine cell (FP32).
+    # library's stream, in launches of as many sweeps as the solve's.  Algorithmic bytes of one launch
+    # = read u + read f + write u = 3 * 4 B per fine cell (FP32).
     import ctypes
-    ms_sweep = ctypes.c_double()
+    cfg, ns, fs, ms_sweep = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_double()
+    _lib.check(solver._lib.sg_uniform_tile_info(solver._ctx, 0, ctypes.byref(cfg), ctypes.byref(ns), ctypes.byref(fs),
+                                                None, 0))
+    per_launch = max(1, ns.value)
     _lib.check(solver._lib.sg_uniform_time_smoother(solver._ctx, SG_PREC_MIXED, a.smoother_reps,
                                                      ctypes.byref(ms_sweep)))
-    sweep_bytes = 3 * 4 * n ** 3
-    achieved = sweep_bytes / (ms_sweep.value * 1e-3) / 1e9
-    log(f"[bench] smoother sweep {ms_sweep.value * 1e3:.1f} us -> {achieved:.0f} GB/s algorithmic")
-    # The same sweep with a cold last-level cache: the 256^3 FP32 working set of one sweep (u, f and
-    # the new u: 192 MiB) fits in MI355X's 256 MiB Infinity Cache, so back-to-back sweeps (and the
-    # solve's own) partly hit it.  Before each timed sweep a 1 GiB fill evicts it; each sweep is
-    # timed alone with HIP events, so the figure includes one launch's start-up.
+    ms_launch = ms_sweep.value * per_launch
+    launch_bytes = 3 * 4 * n ** 3
+    achieved = launch_bytes / (ms_launch * 1e-3) / 1e9
+    log(f"[bench] smoother launch of {per_launch} sweeps {ms_launch * 1e3:.1f} us -> {achieved:.0f} GB/s algorithmic")
+    # The same launch with a cold last-level cache: the 256^3 FP32 working set (u, f and the new u:
+    # 192 MiB) fits in MI355X's 256 MiB Infinity Cache, so back-to-back launches (and the solve's own)
+    # partly hit it.  Before each timed launch a 1 GiB fill evicts it; each is timed alone with HIP
+    # events, so the figure includes one launch's start-up.
     flush = torch.empty(1 << 28, dtype=torch.float32, device=dev)
     cold = []
     ms1 = ctypes.c_double()
@@ -354,11 +358,11 @@ def bench_uniform(a, dev):
         flush.fill_(float(r))
         torch.cuda.synchronize()
         _lib.check(solver._lib.sg_uniform_time_smoother(solver._ctx, SG_PREC_MIXED, 1, ctypes.byref(ms1)))
-        cold.append(ms1.value)
+        cold.append(ms1.value * per_launch)
     del flush
     ms_cold = sorted(cold)[len(cold) // 2]
-    achieved_cold = sweep_bytes / (ms_cold * 1e-3) / 1e9
-    log(f"[bench] smoother sweep, cache cold: {ms_cold * 1e3:.1f} us -> {achieved_cold:.0f} GB/s algorithmic")
+    achieved_cold = launch_bytes / (ms_cold * 1e-3) / 1e9
+    log(f"[bench] smoother launch, cache cold: {ms_cold * 1e3:.1f} us -> {achieved_cold:.0f} GB/s algorithmic")
 
     tiles = {}
     dims = [(32, 16, 16, 1024), (16, 8, 8, 1024), (16, 8, 8, 256), (64, 8, 8, 512), (8, 8, 8, 512)]
@@ -388,17 +392,11 @@ def bench_uniform(a, dev):
     log(f"[bench] autotuned tiles {json.dumps(tiles)}")
 
     # HBM bytes per launch of the roofline kernel (the autotuned shape at this size), from the
-    # committed rocprofv3 counter summary: lines "traffic_bytes_per_launch[<shape>]: <bytes>"
-    traffic = None
-    prof = os.path.join(ROOT, "profiles", "uniform256_hbm_traffic.md")
+    # committed rocprofv3 counter summary: lines "traffic_bytes_per_launch[<shape>/<sweeps>sw]: <bytes>"
     shape = tiles.get(str(n), {}).get("shape")
-    if shape and tiles[str(n)]["source_in_lds"]:
-        shape += "/fLDS"
-    if n == 256 and shape and os.path.exists(prof):
-        key = f"traffic_bytes_per_launch[{shape}]:"
-        for line in open(prof):
-            if line.startswith(key):
-                traffic = int(line[len(key):])
+    if shape:
+        shape += f"/{per_launch}sw" + ("/fLDS" if tiles[str(n)]["source_in_lds"] else "")
+    traffic = _profile_traffic("uniform256_hbm_traffic.md", shape) if n == 256 and shape else None
 
     p64 = psi64 - psi64.mean()
     pmx = psimx - psimx.mean()
@@ -432,12 +430,13 @@ def bench_uniform(a, dev):
         "phi_err_vs_cpu_oracle": err_vs_oracle,
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
-                     "kernel": "fine-level FP32 smoother sweep (both colours), " + (shape or "?"),
-                     "algorithmic_bytes_per_launch": sweep_bytes,
-                     "ms_per_launch": ms_sweep.value,
+                     "kernel": "fine-level FP32 smoother launch, " + (shape or "?"),
+                     "sweeps_per_launch": per_launch,
+                     "algorithmic_bytes_per_launch": launch_bytes,
+                     "ms_per_launch": ms_launch,
                      "cache_cold": {"achieved": round(achieved_cold, 1), "frac": round(achieved_cold / HBM_PEAK_GBS, 4),
                                     "ms_per_launch": ms_cold,
-                                    "note": "Infinity Cache evicted by a 1 GiB fill before each sweep, median"}},
+                                    "note": "Infinity Cache evicted by a 1 GiB fill before each launch, median"}},
         "cpu_oracle": cpu,
         "autotune": tiles,
     }

@@ -1227,14 +1227,15 @@ int sg_uniform_time_smoother(sg_uniform *c, int prec, int reps, double *ms_per_s
     SG_REQUIRE(c && ms_per_sweep && reps > 0 && reps <= 100000, "bad argument");
     SG_REQUIRE(c->precisions & prec, "context lacks precision %d", prec);
     const bool fused = prec == SG_PREC_MIXED && c->n > sg::kCoarseMaxN;
+    const int ns = fused ? c->tile_ns[0] : 1;   // sweeps per repetition
     SG_HIP(hipEventRecord(c->ev0, c->stream));
     for (int r = 0; r < reps; ++r) {
         if (prec == SG_PREC_FP64)
             SG_TRY(sg::launch_relax<double>(c->stream, c->d.U[0], c->d.RHO[0], c->n, c->h, nullptr));
         else if (fused) {
-            // the mixed path's fine-level sweep: U[0] -> U1[0] and back on alternate repetitions
+            // the mixed path's fine-level launch: U[0] -> U1[0] and back on alternate repetitions
             float *a = (r & 1) ? c->f.U1[0] : c->f.U[0], *b = (r & 1) ? c->f.U[0] : c->f.U1[0];
-            SG_TRY(sg::launch_sweep_cfg<float>(c->stream, c->tile_cfg[0], 1, c->tile_fs[0] != 0, a, b, c->f.RHO[0], c->n,
+            SG_TRY(sg::launch_sweep_cfg<float>(c->stream, c->tile_cfg[0], ns, c->tile_fs[0] != 0, a, b, c->f.RHO[0], c->n,
                                         c->h, false, false, false, nullptr, nullptr, nullptr));
         } else
             SG_TRY(sg::launch_relax<float>(c->stream, c->f.U[0], c->f.RHO[0], c->n, c->h, nullptr));
@@ -1243,7 +1244,7 @@ int sg_uniform_time_smoother(sg_uniform *c, int prec, int reps, double *ms_per_s
     SG_HIP(hipEventSynchronize(c->ev1));
     float ms = 0.f;
     SG_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-    *ms_per_sweep = (double)ms / reps;
+    *ms_per_sweep = (double)ms / ((double)reps * ns);
     return SG_OK;
 }
 

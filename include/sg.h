@@ -131,7 +131,9 @@ int sg_uniform_interp_dev(sg_uniform *ctx, int prec, void *uf, const void *uc, i
                                                        /* interpolation.F90:40-247 via mg.F90:608-633 */
 
 /* Measurement helper (no reference counterpart): average device time of one full smoothing sweep
- * (both colours) on the finest level's own arrays, timed with HIP events on the library's stream. */
+ * (both colours) on the finest level's own arrays, timed with HIP events on the library's stream.  One
+ * repetition is one launch of the mixed solve's sweep kernel, of as many sweeps as sg_uniform_tile_info
+ * reports for level 0 (two passes of one colour each in FP64 and for grids of n <= 16). */
 int sg_uniform_time_smoother(sg_uniform *ctx, int prec, int reps, double *ms_per_sweep);
 
 /* Autotuner result (no reference counterpart): tile shape, sweeps per launch and source staging
