@@ -885,8 +885,8 @@ template <bool ZB> int base_lin(sg_amr &s, double *mx, const double **u0)
     while (M.n[lc] > kCoarseMaxN) ++lc;
     const CoarseCoef<double> P = coarse_coef<double>(M.h[lc]);
     auto coarse = [&](int mode) -> int {
-        hipLaunchKernelGGL((k_coarse<double, 16, ZB>), dim3(1), dim3(kCoarseThreads), 0, s.stream,
-                           (const double *)s.bc_rhs[lc], s.bc_u[lc][0], P, mode, 2, 2, 2, (double *)nullptr);
+        hipLaunchKernelGGL((k_coarse<double, ZB>), dim3(1), dim3(kCoarseThreads), 0, s.stream,
+                           (const double *)s.bc_rhs[lc], s.bc_u[lc][0], P, mode, 2, 2, 2);
         SG_CHECK_LAUNCH();
         return SG_OK;
     };

@@ -356,13 +356,13 @@ kb_coarse(BL<T> L, const CoarseDesc<T> *descs, int mode, int ncycle, int npre, i
     const T *f = c.q->a[CRHS];
     T *u = c.q->a[CU];
     switch (D.n) {
-    case 16: coarse_solve<T, 16>(S, D.coef, f, u, mode, ncycle, npre, npost, nullptr); break;
-    case 12: coarse_solve<T, 12>(S, D.coef, f, u, mode, ncycle, npre, npost, nullptr); break;
-    case 8: coarse_solve<T, 8>(S, D.coef, f, u, mode, ncycle, npre, npost, nullptr); break;
-    case 6: coarse_solve<T, 6>(S, D.coef, f, u, mode, ncycle, npre, npost, nullptr); break;
-    case 4: coarse_solve<T, 4>(S, D.coef, f, u, mode, ncycle, npre, npost, nullptr); break;
-    case 3: coarse_solve<T, 3>(S, D.coef, f, u, mode, ncycle, npre, npost, nullptr); break;
-    default: coarse_solve<T, 2>(S, D.coef, f, u, mode, ncycle, npre, npost, nullptr); break;
+    case 16: coarse_solve<T, 16>(S, D.coef, f, u, mode, ncycle, npre, npost); break;
+    case 12: coarse_solve<T, 12>(S, D.coef, f, u, mode, ncycle, npre, npost); break;
+    case 8: coarse_solve<T, 8>(S, D.coef, f, u, mode, ncycle, npre, npost); break;
+    case 6: coarse_solve<T, 6>(S, D.coef, f, u, mode, ncycle, npre, npost); break;
+    case 4: coarse_solve<T, 4>(S, D.coef, f, u, mode, ncycle, npre, npost); break;
+    case 3: coarse_solve<T, 3>(S, D.coef, f, u, mode, ncycle, npre, npost); break;
+    default: coarse_solve<T, 2>(S, D.coef, f, u, mode, ncycle, npre, npost); break;
     }
 }
 

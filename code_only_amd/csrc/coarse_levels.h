@@ -645,12 +645,10 @@ template <typename T, int N, bool ZERO> __device__ __forceinline__ void coarse_t
 
 // mode 0: FMG over all held levels from the right-hand side of the first (mg.F90:142-215 restricted to
 // them); mode 1: one V-cycle from it with zero initial guess (mg.F90:179-210).  rhs_in, u_out: dense
-// N^3 arrays.  resmax receives max|resh2| of the last smoothing of the first level when non-null.
-// Every thread of a kCoarseThreads workgroup calls it.
+// N^3 arrays.  Every thread of a kCoarseThreads workgroup calls it.
 template <typename T, int N, bool ZERO = false>
 __device__ __forceinline__ void coarse_solve(CoarseLds<T> &S, const CoarseCoef<T> &P, const T *__restrict__ rhs_in,
-                                             T *__restrict__ u_out, int mode, int ncycle, int npre, int npost,
-                                             double *resmax)
+                                             T *__restrict__ u_out, int mode, int ncycle, int npre, int npost)
 {
     using L = CoarseLevel<N>;
     for (int c = threadIdx.x; c < L::len; c += kCoarseThreads) {
@@ -662,7 +660,7 @@ __device__ __forceinline__ void coarse_solve(CoarseLds<T> &S, const CoarseCoef<T
     }
     if (mode == 0 && threadIdx.x >= kCoarseThreads - 64) coarse_tables<T, N, ZERO>(S, (int)threadIdx.x - (kCoarseThreads - 64));
     __syncthreads();
-    coarse_run<T, N, ZERO>(S, P, mode == 0, ncycle, npre, npost, resmax);
+    coarse_run<T, N, ZERO>(S, P, mode == 0, ncycle, npre, npost, nullptr);
     for (int c = threadIdx.x; c < L::len; c += kCoarseThreads) {
         int i, j, k;
         L::decode(c, i, j, k);

@@ -541,16 +541,15 @@ __global__ void __launch_bounds__(NT) k_interp_cubic_tile(T *__restrict__ uf, co
 }
 
 // ------------------------------------------------------------------------------------------------
-// Single-workgroup solvers of the first level of <= 16^3 cells: the reference's cycles from there down
-// (coarse_levels.h), or its exact solve.
+// Single-workgroup solvers of the first level of <= 16^3 cells (of a grid of n = 2^a > 16: the 16^3 one):
+// the reference's cycles from there down (coarse_levels.h), or its exact solve.
 // ------------------------------------------------------------------------------------------------
-template <typename T, int N, bool ZERO = false>
+template <typename T, bool ZERO = false>
 __global__ void __launch_bounds__(kCoarseThreads)
-k_coarse(const T *__restrict__ rhs_in, T *__restrict__ u_out, CoarseCoef<T> P, int mode, int ncycle, int npre, int npost,
-         double *resmax)
+k_coarse(const T *__restrict__ rhs_in, T *__restrict__ u_out, CoarseCoef<T> P, int mode, int ncycle, int npre, int npost)
 {
     __shared__ CoarseLds<T> S;
-    coarse_solve<T, N, ZERO>(S, P, rhs_in, u_out, mode, ncycle, npre, npost, resmax);
+    coarse_solve<T, kCoarseMaxN, ZERO>(S, P, rhs_in, u_out, mode, ncycle, npre, npost);
 }
 
 // mg_cycle (mg.F90:42-94) of a grid held by the coarse levels alone (N <= 16) in one launch: FP64

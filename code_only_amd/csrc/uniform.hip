@@ -8,8 +8,8 @@
 //  * SG_PREC_MIXED: the inner mg_lin runs on FP32 level arrays; the outer residual
 //    r = f - L phi and the update phi += e stay FP64.
 // Either runs the fused kernels with its inner solve captured once into a hipGraph and replayed (FP64,
-// 64^3: 1 732 launches of 1.4-2 us each, host-bound at 6.2 ms per solve, became 111 and 0.9 ms; 16^3:
-// 3.1 to 0.43 ms), or with fused = 0 one kernel per reference loop nest.
+// 64^3: 1 732 launches of 1.4-2 us each, host-bound at 6.2 ms per solve, became 111 and 0.9 ms), a grid of
+// n <= 16 as one launch (FP64, 16^3: 3.1 to 0.32 ms), or with fused = 0 one kernel per reference loop nest.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -371,13 +371,6 @@ static int launch_sweep_cfg(hipStream_t s, int cfg, int ns, bool fs, const T *ui
     return SG_OK;
 }
 
-static int level_of(const sg_uniform *c, int n)
-{
-    for (int l = 0; l < c->nlev; ++l)
-        if (c->nl[l] == n) return l;
-    return -1;
-}
-
 // sweeps per launch on level l; one launch of ns sweeps there with its shape (FP32: autotuned)
 template <typename T> static int level_ns(sg_uniform *c, int l)
 {
@@ -504,25 +497,12 @@ static int coarse_levels(sg_uniform *c)
     return SG_OK;
 }
 
-template <typename T, int N>
-static void coarse_n(sg_uniform *c, const T *rhs, T *u, int mode, int ncycle, int npre, int npost, double *resmax)
+// The reference's cycles on level lc, the 16^3 one, and below (a grid of n <= 16 takes small_cycle).
+template <typename T> static int launch_coarse(sg_uniform *c, int mode, int ncycle, int npre, int npost)
 {
-    hipLaunchKernelGGL((k_coarse<T, N>), dim3(1), dim3(kCoarseThreads), 0, c->stream, rhs, u,
-                       coarse_coef<T>(c->hl[c->lc]), mode, ncycle, npre, npost, resmax);
-}
-
-// The reference's cycles on level lc and below.
-template <typename T>
-static int launch_coarse(sg_uniform *c, int mode, int ncycle, int npre, int npost, double *resmax)
-{
-    const T *rhs = levels<T>(c).RHO[c->lc];
-    T *u = levels<T>(c).U[c->lc];
-    switch (c->nl[c->lc]) {
-    case 16: coarse_n<T, 16>(c, rhs, u, mode, ncycle, npre, npost, resmax); break;
-    case 8: coarse_n<T, 8>(c, rhs, u, mode, ncycle, npre, npost, resmax); break;
-    case 4: coarse_n<T, 4>(c, rhs, u, mode, ncycle, npre, npost, resmax); break;
-    default: coarse_n<T, 2>(c, rhs, u, mode, ncycle, npre, npost, resmax); break;
-    }
+    SG_REQUIRE(c->lc > 0 && c->nl[c->lc] == kCoarseMaxN, "coarse levels of a grid of %d", c->n);
+    hipLaunchKernelGGL(k_coarse<T>, dim3(1), dim3(kCoarseThreads), 0, c->stream, (const T *)levels<T>(c).RHO[c->lc],
+                       levels<T>(c).U[c->lc], coarse_coef<T>(c->hl[c->lc]), mode, ncycle, npre, npost);
     SG_CHECK_LAUNCH();
     return SG_OK;
 }
@@ -574,7 +554,7 @@ static int fast_mg_lin(sg_uniform *c, int ncycle, int npre, int npost, double *r
     auto buf = [&](int l, int b) -> T * { return b ? A.U1[l] : A.U[l]; };
     auto bottom = [&](int mode) -> int {
         if (exact) return exact_bottom(c);
-        return launch_coarse<T>(c, mode, ncycle, npre, npost, lc == 0 ? resmax : nullptr);
+        return launch_coarse<T>(c, mode, ncycle, npre, npost);
     };
     for (int l = rhs1_ready ? 2 : 1; l <= lc; ++l) SG_TRY(launch_restrict<T>(s, A.RHO[l], A.RHO[l - 1], c->nl[l]));
     SG_TRY(bottom(0));
@@ -729,12 +709,12 @@ template <typename T> static int inner_solve(sg_uniform *c, const sg_params *p, 
     return mg_lin<T>(c, p->ncycle, p->npre, p->npost, resmax, exact);
 }
 
-// The inner solve replayed as a graph.  Not for a grid held by k_coarse alone (its inner solve is one
-// launch), nor for the FP64 solve without fused kernels (the plain form: every launch eager).
+// The inner solve replayed as a graph, but for the FP64 solve without fused kernels (the plain form: every
+// launch eager).
 template <typename T> static int run_inner_solve(sg_uniform *c, const sg_params *p, const T **u0)
 {
     const bool fp64 = std::is_same<T, double>::value;
-    if (!p->use_graph || (fused_solve(c, p) ? c->lc == 0 : fp64)) return inner_solve<T>(c, p, u0);
+    if (!p->use_graph || (fp64 && !fused_solve(c, p))) return inner_solve<T>(c, p, u0);
     sg_uniform::Graph &g = c->graph[fp64 ? 1 : 0];
     const bool same = g.exec && g.ncycle == p->ncycle && g.npre == p->npre && g.npost == p->npost &&
                       g.fused == p->fused && g.stop == p->stop_mode && g.coarse == p->coarse;
