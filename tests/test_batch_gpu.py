@@ -159,11 +159,45 @@ def test_uneven_48_problem_batch(gpu):
     b.close()
 
 
-@pytest.mark.parametrize("sizes", [[96] * 10 + [48, 24, 128], [192, 192, 24, 48], [128, 96, 24], [24, 48, 64], [3, 6, 12, 24]])
+FP64_SIZES = [[96] * 10 + [48, 24, 128], [192, 192, 24, 48], [128, 96, 24], [24, 48, 64], [3, 6, 12, 24]]
+
+
+def fp64_shapes(sizes):
+    """The sweep shapes (numbers of fp64_sweep_shape) that a batch of these sizes takes on its levels of more
+    than 16^3 cells, by the rule as the source states it: the widest common unit and the cells of the
+    problems whose width there is a multiple of 32, and of the others."""
+    import os
+    import re
+    src = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "code_only_amd", "csrc",
+                            "fast_kernels.h")).read()
+    body = src[src.index("inline int fp64_sweep_shape("):]
+    rule = [(int(u), 256 * eval(c), 5 + int(k)) for u, c, k in
+            re.findall(r"if \(unit >= (\d+) && cells >= kSweepCUs \* ([\d* ]+)\) return kNumTiles \+ (\d+);", body)][:2]
+    u, c, a, b = re.search(r"return unit >= (\d+) && cells >= kSweepCUs \* ([\d* ]+) \? (\d+) : (\d+);", body).groups()
+    rule += [(int(u), 256 * eval(c), int(a)), (0, 0, int(b))]
+    assert len(rule) == 4 and "kSweepCUs = 256;" in src and "kNumTiles = 5;" in src
+    out = set()
+    for lev in range(8):
+        for wide in (True, False):
+            ns = [n >> lev for n in sizes if (n >> lev) << lev == n and n >> lev > 16 and ((n >> lev) % 32 == 0) == wide]
+            if ns:
+                unit = max(x for x in (64, 32, 16, 8) if all(n % x == 0 for n in ns))
+                out.add(next(k for mu, mc, k in rule if unit >= mu and sum(n ** 3 for n in ns) >= mc))
+    return out
+
+
+def test_fp64_sizes_reach_every_shape():
+    """Streams of 32 x 16 columns in chunks of 64 (two 192^3 problems) and 16 planes (ten of 96^3), tiles of
+    16 x 8 x 8 (two of 96^3, the second level of the former) and of 8^3 (whatever has a 24^3 beside it)."""
+    assert [fp64_shapes(s) for s in FP64_SIZES] == [{10, 1, 4}, {15, 1, 4}, {10, 1, 4}, {1, 4}, {4}]
+
+
+@pytest.mark.parametrize("sizes", FP64_SIZES)
 def test_fp64_sweep_shapes_do_not_change_values(gpu, sizes):
-    """The FP64 rule takes another sweep shape (streams of 64 x 16 and 32 x 32, tiles of one and two
-    sweeps) as the cells of a level add up, and the problems of a multiple of 32 apart from the
-    others: every problem equals its batch-of-one solve bit for bit, odd sweep counts included."""
+    """The FP64 rule takes another sweep shape (streams of 32 x 16, tiles of 16 x 8 x 8 and 8^3; the shapes
+    that each list of sizes reaches: test_fp64_sizes_reach_every_shape) as the cells of a level add up, and
+    the problems of a multiple of 32 apart from the others: every problem equals its batch-of-one solve bit
+    for bit, odd sweep counts included."""
     for npre, npost in ((2, 2), (3, 1)):
         srcs = rhs_list(sizes, seed=21)
         b = BatchSolver(sizes, precisions=SG_PREC_FP64)

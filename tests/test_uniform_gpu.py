@@ -381,8 +381,9 @@ def test_fused_other_cycle_shapes_bitwise(gpu, npre, npost, ncycle):
 @pytest.mark.parametrize("cycle", [(2, 2, 2), (1, 3, 1), (2, 1, 2)])
 @pytest.mark.parametrize("n", [2, 4, 8, 16, 32, 64, 128, 256])
 def test_fp64_fused_equals_plain(n, cycle, gpu):
-    """The fused FP64 solve (k_coarse below 16^3, every sweep shape of the rule: tiles of two sweeps at
-    32 and 64, streams of two sweeps at 128 and 256; odd sweep counts) against one kernel per loop nest,
+    """The fused FP64 solve (one launch for n <= 16, k_coarse from the 16^3 level down for the others, of
+    the rule's sweep shapes the 8^3 tile at 32, the 16 x 8 x 8 tile at 64 and the streams of 32 x 16 columns
+    in chunks of 16 planes at 128 and 64 at 256; odd sweep counts) against one kernel per loop nest,
     bit for bit, in both stopping modes, and again with other phi and source arrays (the graph is
     the context's own)."""
     import torch
