@@ -24,7 +24,10 @@
 // and 60 launches of 1.4-2 us); cycles per step of 16^3 / 8^3 / 4^3: down 6.9k / 3.8k / 2.7k, up 7.3k /
 // 3.7k / 2.6k, the 2^3 bottom 3.3k.  Without the row order and the shared neighbours a 16^3 step took
 // 10-13k; 1 024 threads with one cell each the same.  What is left is the latency of dependent LDS
-// reads and FP64 adds, some 450 cycles per colour of a small level.
+// reads and FP64 adds, some 450 cycles per colour of a small level, and, where a kernel holds more than 256
+// registers beside the levels' code, spills to scratch: the compiler reports none for the periodic k_coarse,
+// 129 spilled registers for the FP64 one with zero ghosts, for 16^3 132 and 68 in k_cycle_small (FP64, FP32)
+// and 149 and 274 in k_base_small (periodic, zero ghosts), 9 in kb_coarse<double>.
 // Boundaries: periodic (ZERO false), or zero ghosts (ZERO: mg_boundary_fill0, with mg_boundary_extrap's
 // odd continuation, (-1)^g times the clamped interior cell for g ghost coordinates, before a
 // prolongation; mg.F90:735-771).

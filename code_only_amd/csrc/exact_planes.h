@@ -23,15 +23,17 @@
 // plane between two passes goes through LDS.  Two launch forms of the same tiles, so the same bits:
 // * whole (the batched solver): one workgroup of four wavefronts per plane (row); wavefront w takes the
 //   lines 16 w .. 16 w + 15 to all frequencies, then the outputs 16 w .. of the second pass.  Bound by
-//   the FP32 rate of the matrix cores (2 300 planes: about 15 us of the 20).
+//   latency: the launch's 1 712 planes (32 us) are on the chip at once, each one chain load, product, LDS,
+//   product, store; counters find the wavefronts waiting 45 % of their cycles and the matrix cores busy 25 %
+//   of the launch (8 us).
 // * split (k_exact_*_split; the single-grid solver): n / 16 workgroups per plane (row), each with 16 of
 //   the first transform's frequencies (columns), which it takes through both passes alone.  Bound by the
 //   launch and the chain load, product, LDS, product, store: one level's n planes alone would leave most
 //   of the chip idle.
 // Measured against multiply-add chains over lines and Q staged in LDS: split, 64^3, three launches 24.1
-// -> 14.7 us; whole, the 48-problem batch, per launch xy 27.3 -> 20.3 and z 31.7 -> 20.6 us.  Root mean
-// square error of the solution against 64-bit sums, n = 64: 2.7 .. 4.2e-7 -> 1.5 .. 2.4e-7 (n = 24, 32,
-// 48: 1.7 .. 3.0e-7 -> 0.8 .. 2.0e-7).
+// -> 14.7 us; whole, the 48-problem batch, per launch (average over its plane counts) xy 27.3 -> 20.3 and
+// z 31.7 -> 20.6 us.  Root mean square error of the solution against 64-bit sums, n = 64: 2.7 .. 4.2e-7 ->
+// 1.5 .. 2.4e-7 (n = 24, 32, 48: 1.7 .. 3.0e-7 -> 0.8 .. 2.0e-7).
 #pragma once
 #include <hip/hip_runtime.h>
 

@@ -51,8 +51,9 @@ class UniformSolver:
     def cycle(self, psi, src, tol=1e-10, maxit=50, stop_mode=SG_STOP_TRUE_RESIDUAL, precision=SG_PREC_MIXED,
               ncycle=2, npre=2, npost=2, use_graph=True, fused=True, raise_on_fail=True, coarse=SG_COARSE_EXACT):
         """mg_cycle(ju, jrho) (mg.F90:42-94): psi updated in place; returns stats dict.  coarse
-        (mixed precision only): SG_COARSE_EXACT solves the first level of <= 16^3 cells exactly,
-        SG_COARSE_VCYCLE keeps the reference's levels down to 1^3."""
+        (mixed precision only): SG_COARSE_EXACT ends the cycle at the first level below the finest of
+        <= 64^3 cells (<= 16^3 for a grid of 32^3), solved exactly; SG_COARSE_VCYCLE keeps the
+        reference's levels down to 1^3."""
         n = self.n
         self._check(psi, shape=(n, n, n))
         self._check(src, shape=(n, n, n))

@@ -53,7 +53,9 @@ typedef struct sg_params {
     int precision;    /* SG_PREC_*                                                  */
     int ncycle;       /* V-cycles per FMG level (mg.F90:123, 2)                     */
     int npre, npost;  /* smoothing sweeps (mg.F90:124-125, 2 and 2)                 */
-    int use_graph;    /* replay the inner cycle as a hipGraph (AMR: SG_PREC_MIXED)  */
+    int use_graph;    /* replay the inner cycle as a hipGraph (AMR FP64: fmg_lin, in */
+                      /* stretches between base solves, with the fused refresh on;  */
+                      /* the staged refresh is always launched eagerly)             */
     int fused;        /* fused LDS-tiled kernels (same values); uniform FP64 with 0: */
                       /* one eager launch per reference loop nest                   */
     int coarse;       /* SG_PREC_MIXED only: SG_COARSE_* (default SG_COARSE_EXACT)  */
