@@ -436,6 +436,7 @@ def test_small_grid_mixed_equals_unfused(n, gpu):
 def test_context_memory(prec, word, gpu):
     """A context holds three arrays per level and a second phi: 3 x 8/7 words and 8 bytes per cell."""
     n = 256
+    UniformSolver(n, precisions=prec).close()   # the runtime's own memory (code, queues) is there from here on
     torch.cuda.synchronize()
     free0 = torch.cuda.mem_get_info()[0]
     s = UniformSolver(n, precisions=prec)
