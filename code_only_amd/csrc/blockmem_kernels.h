@@ -303,10 +303,10 @@ __global__ void k_hx_table(int2 *ent, int *staged, int nblk, int nlev, HxBlocks 
 // cells of each 96-byte row, and read ghost cells back; here each ghost cell is written once (88 KB
 // read, 88 KB written).  One workgroup per (grid, array): its stores to the ends of a row meet in L2,
 // and a thread's kHxCells cells keep their offsets over the loop over components.  4 096 grids of 12^3
-// cells and 9 components: 0.67 ms for three arrays (three passes: 1.7 ms), 2.93 GB of HBM traffic, 4.3 TB/s.  Non-temporal stores: nothing
-// reads a ghost cell soon, and the neighbours' lines stay in L2 (4 % on the whole step).  Measured
-// slower: one or three components per workgroup (10 %), cells taken row by row with the interior's
-// lanes idle (7 %).
+// cells and 9 components: 0.67 ms for three arrays (three passes: 1.7 ms), 2.93 GB of HBM traffic, 4.3
+// TB/s.  Non-temporal stores: nothing reads a ghost cell soon, and the neighbours' lines stay in L2 (4 % on
+// the whole step).  Measured slower: one or three components per workgroup (10 %), cells taken row by row
+// with the interior's lanes idle (7 %).
 // Levels of fewer grids are bound by the latency of a workgroup's loop over the components, so they are
 // shared out over workgroups until kHxGroups of them, the eight of 256 threads that each CU holds, and
 // the interpolated cells, which sit in a few regions, are dealt to all threads.  Without either the
